@@ -6,21 +6,26 @@
 // arithmetic; for f64 arrays the difference is taken in double and rounded to
 // float first.
 //
-// One launch reads the array once: each workgroup reduces a strided share
-// with 16-byte loads, writes its (min, max) pair, and the last workgroup to
-// finish (an agent-scope ticket) reduces the pairs and resets the ticket.
+// One launch reads the array once: each workgroup reduces a strided share with
+// 16-byte loads and publishes its (min, max) pair; the last workgroup reduces
+// the pairs (grid_words.hpp) and writes the result to pinned host memory.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <map>
+#include <memory>
 #include <mutex>
 
 #include "../../include/cuSZp.h"
+#include "grid_words.hpp"
 
 namespace cuszp_range {
 
 constexpr int kThreads = 256;
-constexpr unsigned kMaxBlocks = 2048;
+// Bound by the read. Four workgroups per CU with eight 16-byte loads in flight
+// per lane cover the memory latency.
+constexpr unsigned kMaxBlocks = 1024;
+constexpr int kInFlight = 8;
 
 template <class T>
 struct Vec;
@@ -64,33 +69,33 @@ __device__ __forceinline__ void block_reduce(T& mn, T& mx, T* smn, T* smx) {
 }
 
 // x: the array; head: elements before the first 16-byte boundary; nv: whole
-// vectors after it. part: 2 * gridDim.x values; res: {min, max}.
+// vectors after it. gw: 2 values' words per workgroup; res: {min, max}, and in
+// res[kGridResults - 1] whether a workgroup's words never came.
 template <class T>
 __global__ void __launch_bounds__(kThreads) range_kernel(const T* __restrict__ x, uint64_t n, uint64_t head,
-                                                         uint64_t nv, T* __restrict__ part, unsigned* ticket,
-                                                         T* __restrict__ res) {
+                                                         uint64_t nv, const cuszp::GridWords gw, double* res) {
     typedef typename Vec<T>::type V;
+    typedef cuszp::Words<T> W;
     constexpr int N = Vec<T>::N;
     __shared__ T smn[kThreads / 64], smx[kThreads / 64];
-    __shared__ bool last;
+    __shared__ bool lost;
+    if (threadIdx.x == 0) lost = false;
     T mn = INFINITY, mx = -INFINITY;
     const V* __restrict__ xv = (const V*)(x + head);
     const uint64_t stride = (uint64_t)gridDim.x * kThreads;
     uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-    for (; i + 3 * stride < nv; i += 4 * stride) {   // four loads in flight per lane
-        V v[4];
+    for (; i < nv; i += kInFlight * stride) {   // past the end: the last vector again
+        V v[kInFlight];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = __builtin_nontemporal_load(xv + i + k * stride);
+        for (int k = 0; k < kInFlight; ++k) {
+            const uint64_t j = i + k * stride;
+            v[k] = xv[j < nv ? j : nv - 1];
+        }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < kInFlight; ++k) {
 #pragma unroll
             for (int j = 0; j < N; ++j) take((T)v[k][j], mn, mx);
         }
-    }
-    for (; i < nv; i += stride) {
-        const V v = __builtin_nontemporal_load(xv + i);
-#pragma unroll
-        for (int j = 0; j < N; ++j) take((T)v[j], mn, mx);
     }
     if (blockIdx.x == 0) {   // elements before the first vector and after the last
         const uint64_t tail0 = head + nv * N;
@@ -98,43 +103,51 @@ __global__ void __launch_bounds__(kThreads) range_kernel(const T* __restrict__ x
         for (uint64_t t = tail0 + threadIdx.x; t < n; t += kThreads) take(x[t], mn, mx);
     }
     block_reduce(mn, mx, smn, smx);
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = mn;
-        part[2 * blockIdx.x + 1] = mx;
-        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        last = t == gridDim.x - 1;
+    const bool last = blockIdx.x == gridDim.x - 1;
+    if (!last) {
+        if (threadIdx.x == 0) {
+            const W a = W::of(mn), b = W::of(mx);
+#pragma unroll
+            for (int k = 0; k < W::N; ++k) {
+                gw.put((uint64_t)blockIdx.x * 2 * W::N + k, a.u[k]);
+                gw.put((uint64_t)blockIdx.x * 2 * W::N + W::N + k, b.u[k]);
+            }
+        }
+        return;
     }
-    __syncthreads();
-    if (!last) return;
-    __atomic_thread_fence(__ATOMIC_ACQUIRE);
-    mn = INFINITY;
-    mx = -INFINITY;
-    for (unsigned b = threadIdx.x; b < gridDim.x; b += kThreads) {
-        const T a = __hip_atomic_load(part + 2 * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const T c = __hip_atomic_load(part + 2 * b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        mn = a < mn ? a : mn;
-        mx = c > mx ? c : mx;
+    bool ok = true;
+    for (unsigned b = threadIdx.x; b + 1 < gridDim.x; b += kThreads) {
+        uint32_t u[2 * W::N];
+        ok &= gw.get_n(b * 2 * W::N, u);
+        W a, c;
+#pragma unroll
+        for (int k = 0; k < W::N; ++k) {
+            a.u[k] = u[k];
+            c.u[k] = u[W::N + k];
+        }
+        const T va = a.value(), vc = c.value();
+        mn = va < mn ? va : mn;
+        mx = vc > mx ? vc : mx;
     }
     __syncthreads();   // smn/smx are reused
+    if (!ok) lost = true;
     block_reduce(mn, mx, smn, smx);
     if (threadIdx.x == 0) {
         const T x0 = x[0];
         const bool nan0 = x0 != x0;   // the reference's loop starts from element 0
-        res[0] = nan0 ? x0 : mn;
-        res[1] = nan0 ? x0 : mx;
-        *ticket = 0u;   // ready for the next launch on this stream
+        cuszp::host_store(res, (double)(nan0 ? x0 : mn));
+        cuszp::host_store(res + 1, (double)(nan0 ? x0 : mx));
+        cuszp::host_store(res + cuszp::kGridResults - 1, lost ? 1.0 : 0.0);
     }
 }
 
 struct State {
-    void* part = nullptr;      // 2 * kMaxBlocks doubles
-    unsigned* ticket = nullptr;
-    double* res = nullptr;     // device {min, max}
-    double* h_res = nullptr;   // pinned
+    cuszp::GridState g;
     std::mutex mu;
 };
+constexpr uint64_t kWords = (uint64_t)kMaxBlocks * 2 * 2;   // (min, max) of two words each
 std::mutex g_mu;
-std::map<std::pair<int, hipStream_t>, State*> g_state;
+std::map<std::pair<int, hipStream_t>, std::unique_ptr<State>> g_state;
 
 #define RANGE_HIP(call)                                \
     do {                                               \
@@ -142,48 +155,37 @@ std::map<std::pair<int, hipStream_t>, State*> g_state;
         if (e_ != hipSuccess) return CUSZP_ERROR_HIP;  \
     } while (0)
 
-int state_for(int dev, hipStream_t st, State*& out) {
+State& state_for(int dev, hipStream_t st) {
     std::lock_guard<std::mutex> lk(g_mu);
-    State*& s = g_state[{dev, st}];
-    if (!s) {
-        State* n = new State();
-        if (hipMalloc(&n->part, 2 * kMaxBlocks * sizeof(double)) != hipSuccess ||
-            hipMalloc((void**)&n->ticket, 256) != hipSuccess || hipMalloc((void**)&n->res, 2 * sizeof(double)) != hipSuccess ||
-            hipHostMalloc((void**)&n->h_res, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-            hipMemsetAsync(n->ticket, 0, 256, st) != hipSuccess) {
-            delete n;   // (device buffers of a failed set-up are not reclaimed)
-            return CUSZP_ERROR_HIP;
-        }
-        s = n;
-    }
-    out = s;
-    return CUSZP_SUCCESS;
+    auto& s = g_state[{dev, st}];
+    if (!s) s.reset(new State());
+    return *s;
 }
 
 template <class T>
 int run(const T* x, size_t n, double* mn, double* mx, hipStream_t st) {
     int dev = 0;
     RANGE_HIP(hipGetDevice(&dev));
-    State* s = nullptr;
-    int rc = state_for(dev, st, s);
-    if (rc) return rc;
-    std::lock_guard<std::mutex> lk(s->mu);
+    State& s = state_for(dev, st);
+    std::lock_guard<std::mutex> lk(s.mu);
+    RANGE_HIP(cuszp::grid_state_init(s.g, kWords, st));
+    cuszp::GridWords gw;
+    RANGE_HIP(cuszp::grid_next_tag(s.g, kWords, st, gw));
     constexpr int N = Vec<T>::N;
     const uint64_t mis = (uint64_t)((uintptr_t)x % 16) / sizeof(T);
     uint64_t head = mis ? (uint64_t)N - mis : 0;
     if (head > n) head = n;
     const uint64_t nv = (n - head) / N;
-    uint64_t blocks = (nv + 4ull * kThreads - 1) / (4ull * kThreads);
+    uint64_t blocks = (nv + (uint64_t)kInFlight * kThreads - 1) / ((uint64_t)kInFlight * kThreads);
     if (blocks < 1) blocks = 1;
     if (blocks > kMaxBlocks) blocks = kMaxBlocks;
-    hipLaunchKernelGGL(range_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, st, x, (uint64_t)n, head, nv,
-                       (T*)s->part, s->ticket, (T*)s->res);
+    hipLaunchKernelGGL(range_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, st, x, (uint64_t)n, head, nv, gw,
+                       s.g.h_res);
     RANGE_HIP(hipGetLastError());
-    RANGE_HIP(hipMemcpyAsync(s->h_res, s->res, 2 * sizeof(T), hipMemcpyDeviceToHost, st));
     RANGE_HIP(hipStreamSynchronize(st));
-    const T* r = (const T*)s->h_res;
-    *mn = (double)r[0];
-    *mx = (double)r[1];
+    if (s.g.h_res[cuszp::kGridResults - 1] != 0.0) return CUSZP_ERROR_INTERNAL;
+    *mn = s.g.h_res[0];
+    *mx = s.g.h_res[1];
     return CUSZP_SUCCESS;
 }
 
