@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcuszp_amd.so")
 CLI = os.path.join(HERE, "cuszp")
-SOURCES = ["kern_batch_c.hip", "kern_batch_d.hip", "kern_f32.hip", "kern_f64.hip", "kern_range.hip", "kern_quality.hip",
+SOURCES = ["kern_batch_c.hip", "kern_batch_c8.hip", "kern_batch_d.hip", "kern_batch_d8.hip", "kern_f32.hip", "kern_f64.hip", "kern_range.hip", "kern_quality.hip",
            "cuszp_api.cpp",
            "cuszp_batch.cpp", "cuszp_serve.cpp", "cuszp_container.cpp",
            "cuszp_noalloc.hip"]

@@ -7,22 +7,20 @@
 //
 // Work decomposition (wave64-native; see the repository's design notes):
 //   * a "group" is 64 consecutive elements of cuSZp block order: two 32-element
-//     blocks in 1D, one 8x8 (2D) or 4x4x4 (3D) block otherwise. One wave holds
-//     one group, one element per lane;
-//   * a workgroup is WAVES waves and handles one tile: each wave owns kChunks
-//     chunks of G consecutive groups, so a tile is WAVES*kChunks*G groups.
-//     The grid has one workgroup per tile (tile = launch base + blockIdx.x).
-//     No ticket atomics: one hot device-scope atomic serialises at about
-//     12 ns per operation on MI355X;
-//   * lane e holds element e of the group. Each lane packs its sign into bit 31
-//     above the 31-bit magnitude; a 32x32 bit-matrix transpose across each
-//     32-lane half (five ds_swizzle xor stages) then leaves plane p's stream
-//     word in lane p and the sign word in lane 31 -- for every rate at a fixed
-//     cost. The transpose also puts the elements in the bit order of cuSZp's
-//     sign/plane bytes (element e at byte e/8, bit 7-e%8, i.e. bit e^7 of the
-//     word) at no extra cost; decompression runs the inverse transpose;
-//   * per-block bookkeeping (rates, header bytes, sizes, offsets) runs once per
-//     wave with one lane per block;
+//     blocks in 1D, one 8x8 (2D) or 4x4x4 (3D) block otherwise. A "chunk" is 8
+//     groups, 512 elements: a wave holds one, a lane two quads of four
+//     consecutive elements (QuadLane);
+//   * a workgroup is WAVES waves and handles one tile: each wave owns KC
+//     chunks. The grid has one workgroup per tile (tile = launch base +
+//     blockIdx.x). No ticket atomics: one hot device-scope atomic serialises at
+//     about 12 ns per operation on MI355X;
+//   * sign and magnitude bits travel as byte slices of a quad, as many as the
+//     chunk's largest rate needs (one for 7 bits), which a transpose across
+//     eight lanes turns into plane words in the bit order of cuSZp's sign/plane
+//     bytes (to_planes); decompression runs the inverse;
+//   * a block's rate is the bit length of its largest residual; every lane
+//     keeps its own block's books in compression, and in decompression one lane
+//     per block, once per wave;
 //   * the inter-tile exclusive scan of compressed bytes is a single-pass
 //     decoupled lookback: one 64-bit status word per tile packs
 //     {epoch, flag, value}, is read 128 or 256 predecessors at a time by one
@@ -90,7 +88,8 @@ struct Geom {
     uint64_t XY;        // X*Y
     uint32_t X, Y, Z;
     uint32_t Bx, By;    // blocks along x and y (2D/3D)
-    uint32_t aligned;   // 2D/3D: every block lies entirely inside the array (extents multiples of the block)
+    uint32_t runs;      // every chunk's blocks lie inside the array, 2D/3D consecutive along x (extents multiples
+                        // of the block, Bx of a chunk's 8 blocks), and their places fit 32-bit offsets
 };
 
 // Launch-wide scan state.
@@ -137,22 +136,16 @@ __device__ __forceinline__ uint32_t dpp(uint32_t v) {
 }
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
 constexpr int kDppWaveShr1 = 0x138, kDppRowMirror = 0x140, kDppHalfMirror = 0x141;
+constexpr int kDppRowRor8 = 0x128;
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
 constexpr int kDppQuadSwap1 = 0xB1;   // quad_perm [1,0,3,2]
 constexpr int kDppQuadSwap2 = 0x4E;   // quad_perm [2,3,0,1]
 constexpr int kDppQuadShr1 = 0x90;    // quad_perm [0,0,1,2]
 constexpr int kDppQuadShr2 = 0x40;    // quad_perm [0,0,0,1]
-constexpr int kDppQuadBcast0 = 0x00;  // quad_perm [0,0,0,0]
 constexpr int kDppRowNewBcast0 = 0x150;   // lane 0 of each row to the whole row
 
 __device__ __forceinline__ uint32_t rdlane(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
-}
-// old[L] <- v for a compile-time lane L (v wave-uniform)
-template <int L>
-__device__ __forceinline__ uint32_t wrlane(uint32_t v, uint32_t old) {
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(old) : "s"(v), "i"(L));
-    return old;
 }
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 // A value the compiler cannot prove wave-uniform but that is (kept in SGPRs,
@@ -162,103 +155,225 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
            ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32);
 }
 
-// ---------------------------------------------------------------------------
-// 32x32 bit transposes within each 32-lane half, with the element order of
-// cuSZp's sign/plane bytes folded in. In the stream, element e of a 32-element
-// half sits at bit e^7 of its plane word (byte e/8, bit 7-e%8). Lanes hold
-// elements in natural order, so:
-//   compress   (ENC): out lane i bit j = in lane j^7 bit i   (lane e's word -> plane words)
-//   decompress (DEC): out lane i bit j = in lane j bit i^7   (plane words -> lane e's word)
-// Stage J exchanges lane-index bit log2(J) with data bit log2(J). Stages 16 and
-// 8 move whole bytes (v_perm); stages 4, 2, 1 rotate the lane's own word and
-// merge in its partner's (v_alignbit + v_bfi). Exchanging the bit with its
-// complement in those three stages (the order twist e -> e^7) costs nothing:
-// it only changes which half of each pair stays in place, i.e. the per-lane
-// shift and mask constants. The partner value (lane^J) comes from ds_swizzle
-// (xor mode), which runs on the LDS pipe, not the VALU.
-// ---------------------------------------------------------------------------
-struct XposeConsts {
-    uint32_t sh1, mk1, sh2, mk2, sh4, mk4, sel8, sel16;
-    // dec: the decompress transpose (plane words -> elements)
-    __device__ __forceinline__ void init(int lane, bool dec) {
-        const int l = lane & 31;
-        const bool lo1 = !(l & 1) != dec, lo2 = !(l & 2) != dec, lo4 = !(l & 4) != dec;
-        const bool lo8 = !(l & 8), lo16 = !(l & 16);
-        sh1 = lo1 ? 31 : 1;  mk1 = lo1 ? 0xAAAAAAAAu : 0x55555555u;
-        sh2 = lo2 ? 30 : 2;  mk2 = lo2 ? 0xCCCCCCCCu : 0x33333333u;
-        sh4 = lo4 ? 28 : 4;  mk4 = lo4 ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-        sel8 = lo8 ? 0x06020400u : 0x03070105u;     // [x0,y0,x2,y2] | [y1,x1,y3,x3]
-        sel16 = lo16 ? 0x05040100u : 0x03020706u;   // [x0,x1,y0,y1] | [y2,y3,x2,x3]
-    }
-};
 template <int J>
 __device__ __forceinline__ uint32_t swizzle_xor(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x1f | (J << 10));
 }
-__device__ __forceinline__ uint32_t rotr(uint32_t v, uint32_t s) { return __builtin_amdgcn_alignbit(v, v, s); }
 // (m & a) | (~m & b) in one v_bfi_b32 (the compiler otherwise emits and + and_or)
 __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
     uint32_t r;
     asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
     return r;
 }
-__device__ __forceinline__ uint32_t xpose32(uint32_t x, const XposeConsts& c) {
-    x = __builtin_amdgcn_perm(swizzle_xor<16>(x), x, c.sel16);
-    x = __builtin_amdgcn_perm(swizzle_xor<8>(x), x, c.sel8);
-    x = bfi(c.mk4, rotr(x, c.sh4), swizzle_xor<4>(x));
-    x = bfi(c.mk2, rotr(x, c.sh2), swizzle_xor<2>(x));
-    x = bfi(c.mk1, rotr(x, c.sh1), swizzle_xor<1>(x));
-    return x;
+
+// ---------------------------------------------------------------------------
+// Byte slices and plane words.
+//
+// A lane holds four consecutive elements (a quad) of a 32-element half, which
+// eight lanes hold together: lane k = lane & 7 has elements 4k .. 4k+3. Slice t
+// of a quad is a word with byte t of its four elements (element 3 - j in byte
+// j). to_planes turns a slice that the eight lanes hold into the plane words of
+// bits 8t .. 8t+7 of the half, one per lane: lane k gets plane
+// 8t + plane_of_lane(k). In the stream, element e of a half sits at bit e^7 of
+// its plane word (byte e/8, bit 7-e%8); that order comes out by itself.
+//
+// The slice is transposed as 8x8 bits over lane pairs (two exchanges inside the
+// word, one of nibbles with lane ^ 1), then as 4x4 bytes over the four pairs
+// (lane ^ 2, lane ^ 4): 15 VALU operations for 32 elements' eight planes, where
+// one element per lane and a 32x32 transpose took 16 for any number of planes
+// of 64 elements, i.e. 4 times as many for the one slice that most data need.
+// from_planes is the inverse.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t plane_of_lane(uint32_t k) { return 4 * (k & 1) + 2 * ((k >> 2) & 1) + ((k >> 1) & 1); }
+struct PlaneConsts {
+    uint32_t rot, msk, sel2, sel4;
+    // dec: for from_planes
+    __device__ __forceinline__ void init(int lane, bool dec) {
+        const bool odd = lane & 1;
+        rot = odd != dec ? 4 : 28;                             // bits to the right: 28 is 4 to the left
+        msk = odd != dec ? 0x0f0f0f0fu : 0xf0f0f0f0u;
+        sel2 = !(lane & 2) ? 0x06020400u : 0x03070105u;        // [x0,y0,x2,y2] | [y1,x1,y3,x3]
+        sel4 = !(lane & 4) ? 0x05040100u : 0x03020706u;        // [x0,x1,y0,y1] | [y2,y3,x2,x3]
+    }
+};
+// Exchanges inside the word: bit 0 (1) of the byte's number with bit 0 (1) of the bit's number.
+__device__ __forceinline__ uint32_t swap_bits1(uint32_t x) {
+    const uint32_t t = (x ^ (x >> 7)) & 0x00AA00AAu;
+    return x ^ t ^ (t << 7);
 }
-// The same transpose on N independent values, stage by stage, so the N
-// swizzles of a stage are in flight together (one LDS round trip per stage
-// instead of one per value); the lanes' own rotations are computed while the
-// swizzles are in flight.
+__device__ __forceinline__ uint32_t swap_bits2(uint32_t x) {
+    const uint32_t t = (x ^ (x >> 14)) & 0x0000CCCCu;
+    return x ^ t ^ (t << 14);
+}
+// N slices at a time, so that the cross-lane reads of a stage are in flight together.
 template <int N>
-__device__ __forceinline__ void xpose32_n(uint32_t* x, const XposeConsts& c) {
+__device__ __forceinline__ void to_planes(uint32_t (&x)[N], const PlaneConsts& c) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = swap_bits2(swap_bits1(x[i]));
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = bfi(c.msk, __builtin_amdgcn_alignbit(x[i], x[i], c.rot), dpp<kDppQuadSwap1>(x[i]));
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(dpp<kDppQuadSwap2>(x[i]), x[i], c.sel2);
     uint32_t t[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) t[i] = swizzle_xor<16>(x[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(t[i], x[i], c.sel16);
-#pragma unroll
-    for (int i = 0; i < N; ++i) t[i] = swizzle_xor<8>(x[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(t[i], x[i], c.sel8);
 #pragma unroll
     for (int i = 0; i < N; ++i) t[i] = swizzle_xor<4>(x[i]);
 #pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = bfi(c.mk4, rotr(x[i], c.sh4), t[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) t[i] = swizzle_xor<2>(x[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = bfi(c.mk2, rotr(x[i], c.sh2), t[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) t[i] = swizzle_xor<1>(x[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = bfi(c.mk1, rotr(x[i], c.sh1), t[i]);
+    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(t[i], x[i], c.sel4);
 }
-// Bit j of each 32-bit half of m moved to bit j^7 (each byte bit-reversed):
-// a per-element mask in natural order as a sign word in stream order.
-__device__ __forceinline__ uint64_t stream_order64(uint64_t m) {
-    const uint32_t lo = __builtin_bswap32(__builtin_bitreverse32((uint32_t)m));
-    const uint32_t hi = __builtin_bswap32(__builtin_bitreverse32((uint32_t)(m >> 32)));
-    return (uint64_t)lo | ((uint64_t)hi << 32);
+template <int N>
+__device__ __forceinline__ void from_planes(uint32_t (&x)[N], const PlaneConsts& c) {
+    uint32_t t[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) t[i] = swizzle_xor<4>(x[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(t[i], x[i], c.sel4);
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_perm(dpp<kDppQuadSwap2>(x[i]), x[i], c.sel2);
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = bfi(c.msk, __builtin_amdgcn_alignbit(x[i], x[i], c.rot), dpp<kDppQuadSwap1>(x[i]));
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = swap_bits1(swap_bits2(x[i]));
 }
 
-// p[lane - 1] - q[lane] in one DPP subtract (wave_shr:1; lane 0 reads p = 0).
-// Measured on gfx950 with this assembler: v_sub_u32_dpp d, a, b gives
-// a[lane - 1] - b[lane]; v_subrev_u32_dpp d, a, b gives b[lane - 1] - a[lane]
-// (the shift is on its second operand), so neither forms q[lane] - q[lane - 1]
-// in one instruction. The two wait states a DPP read of a VGPR needs after the
-// VALU write of it are in the block, since the compiler cannot see into it.
-__device__ __forceinline__ uint32_t sub_prev_wave_shr1(uint32_t p, uint32_t q) {
-    uint32_t d;
-    asm("s_nop 1\n\tv_sub_u32_dpp %0, %1, %2 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
-        : "=v"(d)
-        : "v"(p), "v"(q));
-    return d;
+// Four elements' residuals as byte slices of sign | magnitude: NS slices hold
+// 8 NS - 1 magnitude bits and, in the top bit of the last slice, the sign.
+template <int NS>
+__device__ __forceinline__ void slices_of(const uint32_t (&d)[4], uint32_t (&w)[NS]) {
+    static_assert(NS == 1 || NS == 2 || NS == 4, "7, 15 or 31 magnitude bits");
+    if constexpr (NS == 4) {
+        uint32_t x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int32_t v = (int32_t)d[i], n = (int32_t)(0u - d[i]);
+            x[i] = bfi(0x80000000u, d[i], (uint32_t)(v > n ? v : n));
+        }
+        const uint32_t a = __builtin_amdgcn_perm(x[2], x[3], 0x05010400u), b = __builtin_amdgcn_perm(x[2], x[3], 0x07030602u);
+        const uint32_t e = __builtin_amdgcn_perm(x[0], x[1], 0x05010400u), f = __builtin_amdgcn_perm(x[0], x[1], 0x07030602u);
+        w[0] = __builtin_amdgcn_perm(e, a, 0x05040100u);
+        w[1] = __builtin_amdgcn_perm(e, a, 0x07060302u);
+        w[2] = __builtin_amdgcn_perm(f, b, 0x05040100u);
+        w[3] = __builtin_amdgcn_perm(f, b, 0x07060302u);
+    } else {
+        const uint32_t p01 = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);    // low halves
+        const uint32_t p23 = __builtin_amdgcn_perm(d[3], d[2], 0x05040100u);
+        if constexpr (NS == 1) {
+            const uint32_t v = __builtin_amdgcn_perm(p01, p23, 0x04060002u);    // low bytes, element 3 first
+            const uint32_t m = __builtin_amdgcn_perm(p01, p23, 0x0a0b0809u);    // their signs: 0xff or 0
+            const uint32_t a = (v ^ m) + (m & 0x01010101u);                     // |d|: no byte carries (|d| <= 127)
+            w[0] = bfi(0x80808080u, m, a);
+        } else {
+            typedef short s2 __attribute__((ext_vector_type(2)));
+            uint32_t x[2] = {p01, p23};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                s2 v, n, a;
+                __builtin_memcpy(&v, &x[i], 4);
+                n = (s2)0 - v;
+                a = __builtin_elementwise_max(v, n);
+                uint32_t u;
+                __builtin_memcpy(&u, &a, 4);
+                x[i] = bfi(0x80008000u, x[i], u);
+            }
+            w[0] = __builtin_amdgcn_perm(x[0], x[1], 0x04060002u);
+            w[1] = __builtin_amdgcn_perm(x[0], x[1], 0x05070103u);
+        }
+    }
 }
+
+// Dot products of four signed bytes (two halves) with a constant, plus an
+// accumulator: sums of neighbouring residuals in one operation.
+__device__ __forceinline__ uint32_t dot4(uint32_t v, uint32_t m, uint32_t acc) {
+    return (uint32_t)__builtin_amdgcn_sdot4((int)v, (int)m, (int)acc, false);
+}
+__device__ __forceinline__ uint32_t dot2(uint32_t v, uint32_t m, uint32_t acc) {
+    typedef short s2 __attribute__((ext_vector_type(2)));
+    s2 a, b;
+    __builtin_memcpy(&a, &v, 4);
+    __builtin_memcpy(&b, &m, 4);
+    return (uint32_t)__builtin_amdgcn_sdot2(a, b, (int)acc, false);
+}
+
+// A quad's residuals as they come back from NS slices: signed bytes (element
+// 3 - j in byte j), signed halves ([0]: elements 1, 0; [1]: elements 3, 2, the
+// later one low) or words (element i in [i]).
+template <int NS>
+struct Residuals {
+    static constexpr int N = NS == 1 ? 1 : (NS == 2 ? 2 : 4);
+    uint32_t v[N];
+    // w: slices of sign | magnitude. A sign without a magnitude (element 0 of
+    // an outlier-selected block) counts as 0. s0: element 0's sign, 0 or ~0.
+    __device__ __forceinline__ void from_slices(const uint32_t (&w)[NS], uint32_t& s0) {
+        if constexpr (NS == 1) {
+            const uint32_t a = w[0] & 0x7f7f7f7fu;
+            const uint32_t s = (a + 0x7f7f7f7fu) & w[0] & 0x80808080u;   // negative and not 0
+            const uint32_t t = s >> 7;
+            v[0] = (a ^ ((s << 1) - t)) + t;
+            s0 = (uint32_t)((int32_t)w[0] >> 31);
+        } else if constexpr (NS == 2) {
+            typedef short s2 __attribute__((ext_vector_type(2)));
+            const uint32_t x[2] = {__builtin_amdgcn_perm(w[1], w[0], 0x07030602u), __builtin_amdgcn_perm(w[1], w[0], 0x05010400u)};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t a = x[i] & 0x7fff7fffu;
+                s2 h, m, y;
+                __builtin_memcpy(&h, &x[i], 4);
+                m = h >> 15;
+                uint32_t mu;
+                __builtin_memcpy(&mu, &m, 4);
+                const uint32_t z = a ^ mu;
+                __builtin_memcpy(&y, &z, 4);
+                y = y - m;
+                __builtin_memcpy(&v[i], &y, 4);
+            }
+            s0 = (uint32_t)((int32_t)x[0] >> 31);
+        } else {
+            const uint32_t e = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u), a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);
+            const uint32_t f = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u), b = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+            const uint32_t x[4] = {__builtin_amdgcn_perm(f, e, 0x07060302u), __builtin_amdgcn_perm(f, e, 0x05040100u),
+                                   __builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(b, a, 0x05040100u)};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t m = (uint32_t)((int32_t)x[i] >> 31);
+                v[i] = ((x[i] & 0x7fffffffu) ^ m) - m;
+            }
+            s0 = (uint32_t)((int32_t)x[0] >> 31);
+        }
+    }
+    // element I by itself
+    template <int I>
+    __device__ __forceinline__ uint32_t at() const {
+        if constexpr (NS == 1) return (uint32_t)(((int32_t)(v[0] << (8 * I))) >> 24);
+        else if constexpr (NS == 2) return (uint32_t)(((int32_t)(v[I / 2] << (16 * (I % 2)))) >> 16);
+        else return v[I];
+    }
+    // acc plus the elements of MASK (bit i: element i)
+    template <int MASK>
+    __device__ __forceinline__ uint32_t sum(uint32_t acc) const {
+        if constexpr (NS == 1) {
+            constexpr uint32_t m = ((MASK & 1) ? 0x01000000u : 0) | ((MASK & 2) ? 0x010000u : 0) | ((MASK & 4) ? 0x0100u : 0) |
+                                   ((MASK & 8) ? 1u : 0);
+            return dot4(v[0], m, acc);
+        } else if constexpr (NS == 2) {
+            constexpr uint32_t m01 = ((MASK & 1) ? 0x10000u : 0) | ((MASK & 2) ? 1u : 0);
+            constexpr uint32_t m23 = ((MASK & 4) ? 0x10000u : 0) | ((MASK & 8) ? 1u : 0);
+            if constexpr (m01 != 0) acc = dot2(v[0], m01, acc);
+            if constexpr (m23 != 0) acc = dot2(v[1], m23, acc);
+            return acc;
+        } else {
+            if constexpr (MASK & 1) acc += v[0];
+            if constexpr (MASK & 2) acc += v[1];
+            if constexpr (MASK & 4) acc += v[2];
+            if constexpr (MASK & 8) acc += v[3];
+            return acc;
+        }
+    }
+    // acc plus element 0 in lanes where `on` is ~0
+    __device__ __forceinline__ uint32_t first(uint32_t on, uint32_t acc) const {
+        if constexpr (NS == 1) return dot4(v[0], on & 0x01000000u, acc);
+        else if constexpr (NS == 2) return dot2(v[0], on & 0x10000u, acc);
+        else return acc + (v[0] & on);
+    }
+};
 
 // Inclusive prefix sums (wrapping u32).
 __device__ __forceinline__ uint32_t scan_row16(uint32_t v) {
@@ -279,7 +394,13 @@ __device__ __forceinline__ uint32_t scan_wave(uint32_t v) {
     return v;
 }
 
-__device__ __forceinline__ uint32_t bitlen(uint32_t v) { return v ? 32u - (uint32_t)__builtin_clz(v) : 0u; }
+__device__ __forceinline__ uint32_t bitlen(uint32_t v) { return 32u - (uint32_t)__builtin_clzg(v, 32); }
+// Hides a lane constant's origin: the compiler otherwise turns its uses into
+// compares and selects of their own.
+__device__ __forceinline__ void opaque(uint32_t& v) { asm("" : "+v"(v)); }
+// The same for a value that is to be computed where it is used, not once
+// before a loop in a register of its own.
+__device__ __forceinline__ void opaque_here(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
 // ---------------------------------------------------------------------------
 // quantisation: t = RN(x*r); s = (t >= -0.5 ? 0 : 1); q = sat_trunc(RN(t+0.5)) - s
@@ -367,27 +488,12 @@ __device__ __forceinline__ BlockView outlier_code(uint32_t fr1, uint32_t fr2, ui
     return v;
 }
 
-// Byte-granular little-endian store of 1..4 bytes (outlier prefixes).
-__device__ __forceinline__ void store_le(uint8_t* p, uint32_t v, uint32_t nb) {
-    typedef uint32_t __attribute__((aligned(1))) u32u;
-    typedef uint16_t __attribute__((aligned(1))) u16u;
-    if (nb == 4) {
-        *(u32u*)p = v;
-    } else {
-        if (nb & 2) { *(u16u*)p = (uint16_t)v; p += 2; v >>= 16; }
-        if (nb & 1) { *p = (uint8_t)v; }
-    }
-}
 // LDS byte pointers and unaligned LDS words (gfx950 accesses LDS unaligned).
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 typedef __attribute__((address_space(3))) uint32_t __attribute__((aligned(1))) lds_u32u;
 __device__ __forceinline__ void store_u32u(uint8_t* p, uint32_t v) {
     typedef uint32_t __attribute__((aligned(1))) u32u;
     *(u32u*)p = v;
-}
-__device__ __forceinline__ uint32_t load_u32u(const uint8_t* p) {
-    typedef uint32_t __attribute__((aligned(1))) u32u;
-    return *(const u32u*)p;
 }
 
 // ---------------------------------------------------------------------------
@@ -584,6 +690,14 @@ __device__ __forceinline__ uint64_t wave_lookback(const ScanCtx& sc, uint64_t ti
     return excl;
 }
 
+// wave_lookback with a window of 128 (2) or 256 (4 words per lane) predecessors.
+template <class AggF>
+__device__ __forceinline__ uint64_t lookback(const ScanCtx& sc, uint64_t tile, uint64_t first, uint64_t agg, int lane,
+                                             int window, AggF&& agg_of) {
+    return window == 2 ? wave_lookback<2>(sc, tile, first, agg, lane, agg_of)
+                       : wave_lookback<4>(sc, tile, first, agg, lane, agg_of);
+}
+
 // ---------------------------------------------------------------------------
 // Block walking for 2D/3D: wave-uniform block coordinates advanced by +1 block.
 // Block order: b = z*By*Bx + by*Bx + bx (src/cuSZp_kernels_2D_f32.cu:69-73).
@@ -683,110 +797,302 @@ __device__ __forceinline__ int pred_lane(int e) {
     }
 }
 
-// Inverse Lorenzo: rebuild q from residuals d in natural element order.
+// ---------------------------------------------------------------------------
+// Quads: a lane's four consecutive elements. A chunk is 512 elements, two sets
+// of 64 quads; a 1D block is 8 lanes (eight blocks per set), a 2D/3D block a
+// DPP row of 16 lanes (four blocks per set; a quad is half a row of an 8x8
+// block or a row of a 4x4x4 one). Extents along x are multiples of 4, so a quad
+// of a 2D/3D array lies inside the array or outside it as a whole.
+// ---------------------------------------------------------------------------
 template <int DIM>
-__device__ __forceinline__ uint32_t inverse_lorenzo(uint32_t d, int e) {
-    if constexpr (DIM == 1) {
-        return scan_seg32(d);
-    } else if constexpr (DIM == 2) {
-        // q(r,c) = sum_{r'<=r} d(r',0) + sum_{1<=c'<=c} d(r,c')
-        const bool c0 = (e & 7) == 0;
-        const uint32_t col = scan_wave(c0 ? d : 0u);
-        uint32_t v = c0 ? 0u : d;
-        uint32_t t = dpp<kDppRowShr1>(v);
-        v += ((e & 7) >= 1) ? t : 0u;
-        t = dpp<kDppRowShr2>(v);
-        v += ((e & 7) >= 2) ? t : 0u;
-        v += dpp<kDppRowShr4, 0xf, 0xa>(v);
-        return col + v;
-    } else {
-        // q(z,y,x) = sum_{z'<=z} d(z',0,0) + sum_{1<=y'<=y} d(z,y',0) + sum_{1<=x'<=x} d(z,y,x')
-        // (lane e = 16z + 4y + x: a DPP row per z, a quad per y)
-        const int x = e & 3, y = (e >> 2) & 3;
-        uint32_t vx = x ? d : 0u;
-        vx += dpp<kDppQuadShr1>(vx);
-        vx += dpp<kDppQuadShr2>(vx);
-        uint32_t vy = (x == 0 && y != 0) ? d : 0u;   // prefix over the quads' first lanes, then across the quad
-        vy += dpp<kDppRowShr4>(vy);
-        vy += dpp<kDppRowShr8>(vy);
-        vy = dpp<kDppQuadBcast0>(vy);
-        // the row's first lane (x = y = 0) across the row, then the prefix over the rows
-        uint32_t vz = dpp<kDppRowNewBcast0>(d);
-        vz += dpp<kDppBcast15, 0xa>(vz);
-        vz += dpp<kDppBcast31, 0xc>(vz);
-        return vz + vy + vx;
+struct QuadLane {
+    static constexpr int BL = (DIM == 1) ? 8 : 16;   // lanes per block
+    static constexpr int SB = 64 / BL;               // blocks per set
+    static constexpr int NB = 2 * SB;                // blocks per chunk
+    static constexpr int BW = (DIM == 2) ? 8 : 4;    // extent of a 2D/3D block along x (and y)
+    uint32_t k;       // lane within its 32-element half
+    uint32_t h;       // 2D/3D: which half
+    uint32_t blk;     // block within the set
+    uint32_t x, y, z; // 2D/3D: the quad's place in its block
+    uint32_t e0;      // ~0 in the lane that holds the block's element 0
+    uint32_t p1, p2;  // masks of the two candidates for element 0's predecessor (prev_code)
+    bool second;      // the lane is in the second half of its block's lanes
+    __device__ __forceinline__ void init(int lane) {
+        const uint32_t m = (uint32_t)lane % BL;
+        k = (uint32_t)lane & 7;
+        h = (DIM == 1) ? 0u : m >> 3;
+        blk = (uint32_t)lane / BL;
+        e0 = m == 0 ? ~0u : 0u;
+        if constexpr (DIM == 1) {
+            x = y = z = 0;
+            p1 = k ? ~0u : 0u;
+            p2 = 0;
+        } else if constexpr (DIM == 2) {
+            x = 4 * (m & 1);
+            y = m >> 1;
+            z = 0;
+            p1 = (m & 1) ? ~0u : 0u;
+            p2 = !(m & 1) && m ? ~0u : 0u;
+        } else {
+            x = 0;
+            y = m & 3;
+            z = m >> 2;
+            p1 = y ? ~0u : 0u;
+            p2 = !y && z ? ~0u : 0u;
+        }
+        second = (lane & (BL / 2)) != 0;
+        opaque(e0);
+        opaque(p1);
+        opaque(p2);
     }
-}
-
-// The same sums for N independent groups, step by step, so each DPP step of
-// one group fills the other groups' hazard slots instead of s_nop.
-template <int DIM, int N>
-__device__ __forceinline__ void inverse_lorenzo_n(uint32_t* d, int e) {
-    if constexpr (DIM == 1) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] += dpp<kDppRowShr1>(d[i]);
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] += dpp<kDppRowShr2>(d[i]);
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] += dpp<kDppRowShr4>(d[i]);
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] += dpp<kDppRowShr8>(d[i]);
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] += dpp<kDppBcast15, 0xa>(d[i]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] = inverse_lorenzo<DIM>(d[i], e);
+    // Code of the predecessor of the quad's element 0 in the block's Lorenzo
+    // chain (0: none): 1D the previous lane's last code; 2D that one, or in
+    // column 0 the first code of the row above; 3D the first code of the row
+    // before, or in the first row of a slice that of the slice before.
+    __device__ __forceinline__ uint32_t prev_code(const uint32_t (&q)[4]) const {
+        if constexpr (DIM == 1) return dpp<kDppRowShr1>(q[3]) & p1;
+        else if constexpr (DIM == 2) return (dpp<kDppRowShr1>(q[3]) & p1) | (dpp<kDppRowShr2>(q[0]) & p2);
+        else return (dpp<kDppRowShr1>(q[0]) & p1) | (dpp<kDppRowShr4>(q[0]) & p2);
     }
-}
-
-// ---------------------------------------------------------------------------
-// per-block metadata handed from the bookkeeping lanes to the stream-word
-// lanes through LDS (one 16-byte entry per block):
-//   a: byte offset of the block's sign word from the wave's first block (past
-//      any outlier prefix)
-//   b: 0 for a block without payload, else R + 1 (R planes; 33 for a 2D/3D
-//      block of 32 planes). Lane l of a 32-lane half carries one of the
-//      block's words iff key(l) < b, with key(31) = 0 (the sign word, or plane
-//      31 of a 32-plane block) and key(l) = l + 1 (plane l): one compare.
-//   c: the plane words' mask of an outlier-selected block (element 0 travels
-//      in the prefix: bit 7, element 0's stream bit, cleared), else all ones
-// ---------------------------------------------------------------------------
-struct Meta {
-    uint32_t a, b, c, pad;
-    __device__ __forceinline__ uint32_t off() const { return a; }
-    __device__ __forceinline__ bool sel() const { return c != ~0u; }
-    __device__ __forceinline__ bool nz() const { return b != 0; }
-    __device__ __forceinline__ bool has(uint32_t key) const { return key < b; }
+    // Both sets' bookkeeping at once: the first half of a block's lanes does it
+    // for their block of set 0, the second half for that of set 1. The halves
+    // meet in one DPP move (kMeet), which a bank mask confines to either.
+    static constexpr int kMeet = (DIM == 1) ? kDppHalfMirror : kDppRowRor8;
+    static constexpr int kFirst = (DIM == 1) ? 0x5 : 0x3, kSecond = (DIM == 1) ? 0xa : 0xc;
+    // Maxima over the block's lanes of N values per set (0 where absent), in
+    // the half that keeps the set's books.
+    template <int N>
+    __device__ __forceinline__ void block_max(const uint32_t (&v0)[N], const uint32_t (&v1)[N], uint32_t (&r)[N]) const {
+        auto mx = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = second ? v1[i] : v0[i];
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = mx(r[i], dpp<kMeet, 0xf, kFirst>(v0[i]));
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = mx(r[i], dpp<kMeet, 0xf, kSecond>(v1[i]));
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = mx(r[i], dpp<kDppQuadSwap1>(r[i]));
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = mx(r[i], dpp<kDppQuadSwap2>(r[i]));
+        if constexpr (DIM != 1) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) r[i] = mx(r[i], dpp<kDppHalfMirror>(r[i]));
+        }
+    }
+    // A value of the books of set 0 (1) in all lanes of the block.
+    __device__ __forceinline__ static uint32_t of_set(uint32_t v, int s) {
+        return s == 0 ? (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kMeet, 0xf, kSecond, false)
+                      : (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kMeet, 0xf, kFirst, false);
+    }
+    // Inclusive sums over the set's blocks of a value that is the same in all lanes of a block.
+    __device__ __forceinline__ static uint32_t scan_blocks(uint32_t v) {
+        if constexpr (DIM == 1) v += dpp<kDppRowShr8>(v);
+        v += dpp<kDppBcast15, 0xa>(v);
+        v += dpp<kDppBcast31, 0xc>(v);
+        return v;
+    }
+    // Byte offset of plane p's word of this lane's half in a block's payload
+    // after any prefix (the sign word is where plane -1 would be); 2D/3D blocks
+    // interleave the halves' words (src/cuSZp_kernels_2D_f32.cu:896-903).
+    __device__ __forceinline__ uint32_t plane_offset(uint32_t p) const { return DIM == 1 ? 4 + 4 * p : 8 + 8 * p + 4 * h; }
+    // Codes from residuals; r0 is added to element 0 of the block (its
+    // magnitude where it travels in the prefix), only in lane e0.
+    template <int NS>
+    __device__ __forceinline__ void codes(const Residuals<NS>& r, uint32_t r0, uint32_t (&q)[4]) const {
+        if constexpr (DIM == 1) {
+            const uint32_t t = r.template sum<15>(r0);
+            uint32_t s = scan_row16(t);   // two blocks per DPP row: the second starts over
+            s -= dpp_newbcast7_hi(s);
+            q[0] = r.template sum<1>(s - t + r0);
+        } else if constexpr (DIM == 2) {
+            // element 0 of a row adds up over the rows, the rest along its row
+            const uint32_t col = scan_row16(r.first(~p1, r0));
+            q[0] = r.first(p1, col + (dpp<kDppRowShr1>(r.template sum<14>(0u)) & p1));
+        } else {
+            // element 0 of a slice adds up over the slices, of a row over the slice's rows
+            const uint32_t sl = scan_row16(r.first(~p1, r0));
+            uint32_t row = r.first(p1, 0u);   // 0 in the slice's first row
+            row += dpp<kDppQuadShr1>(row);
+            row += dpp<kDppQuadShr2>(row);
+            q[0] = sl + row;
+        }
+        q[1] = r.template sum<2>(q[0]);
+        q[2] = r.template sum<4>(q[1]);
+        q[3] = r.template sum<8>(q[2]);
+    }
+    // Lane 7's value of each DPP row in lanes 8..15, 0 in lanes 0..7.
+    __device__ __forceinline__ static uint32_t dpp_newbcast7_hi(uint32_t v) { return dpp<kDppRowNewBcast0 + 7, 0xf, 0xc>(v); }
 };
-template <int MODE>
-__device__ __forceinline__ Meta make_meta(uint32_t off, const BlockView& v, bool nz) {
-    Meta m;
-    m.a = off + v.head;
-    m.b = nz ? v.R + 1u : 0u;
-    m.c = (MODE == kOutlier && v.sel) ? ~0x80u : ~0u;
-    m.pad = 0;
-    return m;
-}
 
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
+// Four consecutive elements, from any element-aligned address.
+template <bool NT, class T>
+__device__ __forceinline__ void load_quad(const T* p, T (&x)[4]) {
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef T VT __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+#pragma unroll
+    for (int i = 0; i < 4 / V; ++i) {
+        const VT v = NT ? __builtin_nontemporal_load((const VT*)p + i) : ((const VT*)p)[i];
+#pragma unroll
+        for (int j = 0; j < V; ++j) x[V * i + j] = v[j];
+    }
+}
+template <bool NT, class T>
+__device__ __forceinline__ void store_quad(T* p, const T (&x)[4]) {
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef T VT __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+#pragma unroll
+    for (int i = 0; i < 4 / V; ++i) {
+        VT v;
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[j] = x[V * i + j];
+        if constexpr (NT) __builtin_nontemporal_store(v, (VT*)p + i);
+        else ((VT*)p)[i] = v;
     }
 }
 
-// Byte offset of lane (l, h)'s word inside a block payload (after the outlier
-// prefix): lane 31 carries the sign word, lane l < 31 plane l; 2D/3D blocks
-// interleave the two 32-element halves h word by word (src/cuSZp_kernels_2D_f32.cu:896-903).
+// Raw buffer resources (gfx9): word 3 of the descriptor, and an offset that is
+// always past a resource's range (the range of one wave's payload is < 2^31).
+constexpr int kBufferWord3 = 0x00020000;
+constexpr uint32_t kAbsent = 0x80000000u;
+// How a fast wave's values are loaded and stored: in pieces of 16 bytes per
+// lane, such that an instruction covers whole 128-byte lines (loads that do not
+// fetch the rest later, nontemporal stores that do not reach 2.3 TB/s instead of
+// 6.1). Quads of 1D f32 (1 KiB in a row) and 2D f32 (rows of 128 bytes) are such
+// pieces. Four blocks of 3D f32 give rows of 64 bytes only, and a quad of f64 is
+// two pieces: there the lanes whose bit 3 is set trade pieces with those whose
+// bit 3 is clear (trade_codes on the codes, 32 bits in either type), so that
+// one instruction holds the first ones' rows or lines and the other the rest.
+// A lane's piece is at a wave-uniform address plus lane_off bytes (Geom::runs
+// bounds it): set s's at p + s * kSetOff, its second half (f64) hi_off further;
+// of 3D f32 the second piece hi_off further than the first.
+template <int DIM, class T>
+struct Pieces {
+    static constexpr bool kTrade = sizeof(T) == 8 || DIM == 3;
+    static constexpr uint64_t kSetOff = (DIM == 1) ? 256 : QuadLane<DIM>::SB * QuadLane<DIM>::BW;
+    uint32_t lane_off;   // bytes
+    uint64_t hi_off;     // elements
+    __device__ __forceinline__ void init(const QuadLane<DIM>& ql, const Geom& g, int lane) {
+        const uint32_t b3 = ((uint32_t)lane >> 3) & 1;
+        constexpr uint32_t half = sizeof(T) == 8 ? 2 : (uint32_t)kSetOff;
+        if constexpr (DIM == 1) {
+            lane_off = kTrade ? 4 * (uint32_t)(lane & ~8) + half * b3 : 4 * (uint32_t)lane;
+            hi_off = 32;
+        } else if constexpr (DIM == 2) {
+            lane_off = (kTrade ? ql.y & 3 : ql.y) * g.X + ql.x + ql.blk * 8 + (kTrade ? half * b3 : 0u);
+            hi_off = 4 * (uint64_t)g.X;
+        } else {
+            lane_off = (ql.z & 1) * (uint32_t)g.XY + ql.y * g.X + ql.blk * 4 + half * b3;
+            hi_off = 2 * g.XY;
+        }
+        lane_off *= (uint32_t)sizeof(T);
+        opaque(lane_off);
+    }
+    // Set s's share of a chunk at the wave-uniform p; no memory access and
+    // zeros unless `there` (wave-uniform).
+    template <bool NT>
+    __device__ __forceinline__ void load(const T* p, bool there, int s, T (&x)[4]) const {
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+        constexpr int kAux = NT ? 2 : 0;   // nt
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void*)uniform64((uint64_t)p), 0, there ? 0x7fffffff : 0, kBufferWord3);
+        if constexpr (sizeof(T) == 8) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, (uint32_t)((s * kSetOff + j * hi_off) * 8), kAux);
+                __builtin_memcpy(&x[2 * j], &v, 16);
+            }
+        } else {
+            const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, (uint32_t)(s * (kTrade ? hi_off : kSetOff) * 4), kAux);
+            __builtin_memcpy(&x[0], &v, 16);
+        }
+    }
+    __device__ __forceinline__ void store(T* p, int s, const T (&x)[4]) const {   // nontemporal
+        typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+        if constexpr (sizeof(T) == 8) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const V2 v = {x[2 * j], x[2 * j + 1]};
+                __builtin_nontemporal_store(v, (V2*)((char*)(p + s * kSetOff + j * hi_off) + lane_off));
+            }
+        } else {
+            store_quad<true>((T*)((char*)(p + s * (kTrade ? hi_off : kSetOff)) + lane_off), x);
+        }
+    }
+};
+// Codes of pieces to codes of quads, and back.
+template <int DIM, class T>
+__device__ __forceinline__ void trade_codes(uint32_t (&q)[2][4]) {
+    auto trade = [](uint32_t& a, uint32_t& b) {   // lanes 8..15 of a row: a from b; lanes 0..7: b from a
+        const uint32_t na = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, kDppRowRor8, 0xf, 0xc, false);
+        const uint32_t nb = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, kDppRowRor8, 0xf, 0x3, false);
+        a = na;
+        b = nb;
+    };
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) trade(q[s][i], q[s][2 + i]);
+    } else if constexpr (DIM == 3) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) trade(q[0][i], q[1][i]);
+    }
+}
+
+// Where the quads of a 2D/3D chunk lie. The chunk's 8 blocks follow each other
+// along x; past the end of the row they go on in the next one. With Bx >= 8
+// that happens at most once, and both rows' origins are wave-uniform.
 template <int DIM>
-__device__ __forceinline__ uint32_t word_offset(uint32_t l, uint32_t h, bool sign_in_lane31) {
-    if constexpr (DIM == 1) {
-        return (l == 31) ? 0u : 4u + 4u * l;
-    } else {
-        return (sign_in_lane31 && l == 31) ? 4u * h : 8u + 8u * l + 4u * h;
+struct ChunkQuads {
+    uint64_t off[2];   // element offset of set s's quad (0 where outside)
+    bool ok[2];        // it lies inside the array
+    // The quads of the chunk at wk, which moves on to the next chunk.
+    __device__ __forceinline__ void locate(const Geom& g, const QuadLane<DIM>& ql, Walker& wk) {
+        constexpr uint32_t BW = QuadLane<DIM>::BW, SB = QuadLane<DIM>::SB;
+        uint32_t blk = ql.blk, x = ql.x, y = ql.y, z = ql.z;
+        opaque_here(blk);   // nothing of this in registers across the chunk's work
+        if (g.Bx >= 8) {
+            const uint32_t left = g.Bx - wk.bx;   // blocks of the chunk in its first row
+            Walker w1 = wk;
+            w1.step(g, left);
+            const uint64_t o0 = block_origin<DIM>(g, wk), o1 = block_origin<DIM>(g, w1) - (uint64_t)left * BW;
+            const uint32_t y0 = g.Y - wk.by * BW, y1 = g.Y - w1.by * BW;
+            const uint32_t z0 = g.Z - wk.bz * 4, z1 = g.Z - w1.bz * 4;   // 3D
+            const uint64_t nb = wk.b < g.nblocks ? g.nblocks - wk.b : 0;
+            const uint32_t blocks = nb < 8 ? (uint32_t)nb : 8u;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const uint32_t i = blk + s * SB;
+                const bool in0 = i < left;
+                bool v = (i < blocks) & (y < (in0 ? y0 : y1));
+                if constexpr (DIM == 2) v &= (in0 ? wk.bx + i : i - left) * BW + x < g.X;
+                else v &= z < (in0 ? z0 : z1);
+                ok[s] = v;
+                off[s] = (in0 ? o0 : o1) + (uint64_t)i * BW;
+            }
+            wk.step(g, 8);
+        } else {   // block by block
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                ok[s] = false;
+                off[s] = 0;
+#pragma unroll 1
+                for (uint32_t i = 0; i < SB; ++i) {
+                    bool v = (wk.b < g.nblocks) & (wk.by * BW + y < g.Y);
+                    if constexpr (DIM == 2) v &= wk.bx * BW + x < g.X;
+                    else v &= wk.bz * 4 + z < g.Z;
+                    const uint64_t o = block_origin<DIM>(g, wk);
+                    ok[s] = blk == i ? v : ok[s];
+                    off[s] = blk == i ? o : off[s];
+                    wk.next(g);
+                }
+            }
+        }
+        const uint64_t lane_off = (uint64_t)z * g.XY + (uint64_t)y * g.X + x;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) off[s] = ok[s] ? off[s] + lane_off : 0;
     }
-}
+};
 
 // The arrays of a batched launch: descriptors in device memory, ordered by
 // tile0; a tile belongs to the last array whose tile0 is not above it.
@@ -1023,59 +1329,44 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
 // one tile per workgroup pass
 // ---------------------------------------------------------------------------
 
-// Tile shape. A wave works through kChunks chunks of ShapeC<T>::G groups (one
-// element per lane per group); a tile is WAVES * kChunks * G groups (16384 f32
-// or 8192 f64 elements at 4 waves), for compress and decompress alike.
-template <class T> struct ShapeC;
-template <> struct ShapeC<float> { static constexpr int G = 8; };
-template <> struct ShapeC<double> { static constexpr int G = 4; };
-constexpr int kChunks = 8;
-__host__ __device__ constexpr uint64_t tile_groups(bool f64, int waves) {
-    return (uint64_t)waves * kChunks * (f64 ? 4 : 8);
+// Tile shape. A wave works through KC chunks of 512 elements (kChunksOf<T> of
+// them: 16 KiB of values); a tile is WAVES * KC chunks, for compress and
+// decompress alike.
+constexpr int kChunkElems = 512;
+template <class T> constexpr int kChunksOf = sizeof(T) == 4 ? 8 : 4;
+__host__ __device__ constexpr uint64_t tile_groups(bool f64, int waves) {   // groups of 64 elements
+    return (uint64_t)waves * (f64 ? 4 : 8) * (kChunkElems / 64);
 }
 
-// Compressed bytes a compress wave stages in LDS; a wave whose payload is
-// larger (compression ratio below about 2.7 on its share of the tile)
-// recomputes its groups once the tile's offset is known and stores them
-// directly.
+// Compressed bytes a compress wave stages in LDS. A wave's chunks past that
+// (compression ratio below about 2.7 on its share of the tile) run twice.
 constexpr uint32_t kStageBytes = 6144;
-// Waves per SIMD the compress kernels are built for (the register budget):
-// six 4-wave workgroups of about 26 KB of LDS fit one CU's 160 KB.
+// Payload bytes of a chunk, at most: 16 blocks of 32 planes in 1D, 8 in 2D/3D.
+constexpr uint32_t kMaxChunkBytes = 16 * (4 + 32 * 4 + 4);
+static_assert(kMaxChunkBytes >= 8 * (8 + 32 * 8 + 4) && kMaxChunkBytes <= kStageBytes, "a chunk fits the staging area");
+// Waves per SIMD the compress kernels are built for (the register budget): three
+// 8-wave workgroups of about 49 KB of LDS fit one CU's 160 KB. 8 waves per SIMD
+// with 4,960-byte staging areas: 1D the same, 2D/3D 12-30 % slower (64 VGPRs spill).
 constexpr int kCompressWavesPerSimd = 6;
 // Waves per SIMD the decompress kernels are built for: 8 needs at most 64
 // VGPRs and few enough SGPRs for eight waves' scalar files.
 constexpr int kDecompressWavesPerSimd = 8;
-// Raw buffer resources (gfx9): word 3 of the descriptor, and an offset that is
-// always past a resource's range (the range of one wave's payload is < 2^31).
-constexpr int kBufferWord3 = 0x00020000;
-constexpr uint32_t kAbsent = 0x80000000u;
-// Groups whose bit transposes run side by side (a divisor of the groups per chunk).
-constexpr int kXposeBatch = 4;
-// 2D/3D decompress: a chunk's G blocks along x are rows of 128 (3D) or 256 (2D)
-// bytes; they pass through LDS, each row padded by 16 bytes (fewer bank
-// conflicts), so the global stores write whole rows 16 bytes per lane.
-constexpr int kOutPad = 16;
-constexpr int kOutStage = 16 * (128 + kOutPad);   // the larger of 16 x 128 B and 8 x 256 B, padded
 // Largest chunk payload (from its 4-byte-aligned start) read with dense loads
-// into the LDS buffer of a decompress wave; kOutStage bytes hold it.
+// into the LDS buffer of a decompress wave.
 constexpr int kDenseBytes = 2048;
-static_assert(kDenseBytes <= kOutStage, "dense chunk buffer");
-// The LDS buffer of a decompress wave: a 1D wave's whole payload, read in one
+// The LDS buffer of a decompress wave: the wave's whole payload, read in one
 // burst of up to four 16-byte-per-lane loads where it fits; otherwise one
-// chunk's payload at a time (kDenseBytes), or 2D/3D decoded rows (kOutStage).
-// 4032 bytes keep four 8-wave workgroups within a CU's 160 KiB of LDS.
+// chunk's payload at a time (kDenseBytes). 4032 bytes keep four 8-wave
+// workgroups within a CU's 160 KiB of LDS.
 constexpr int kWaveBuf = 4032;
-static_assert(kWaveBuf >= kOutStage && kWaveBuf % 16 == 0, "wave buffer");
+static_assert(kWaveBuf >= kDenseBytes && kWaveBuf % 16 == 0, "wave buffer");
 
 // Shared memory of a compress workgroup.
 template <int WAVES>
 struct SmemC {
     uint64_t wtot[WAVES];                      // per-wave byte counts
     uint64_t excl;                             // the tile's exclusive prefix (wave 0's lookback)
-    uint32_t over[WAVES];                      // the wave's payload did not fit its staging area
-    Meta meta[WAVES][16];                      // per-block metadata of the chunk in work
-    uint32_t aux[WAVES][16];                   // sign words of the chunk's 32-plane 2D/3D groups
-    uint8_t hdr[WAVES][128];                   // header bytes of the wave's blocks, stored after its chunks
+    uint32_t hdr[WAVES][32];                   // header bytes of the wave's blocks, stored after its chunks
     uint4 stage[WAVES][kStageBytes / 16 + 1];  // the wave's payload, as it will appear in the stream (+ a spare word)
 };
 
@@ -1084,484 +1375,401 @@ struct SmemC {
 // of the wave, written once by the wave's bookkeeping):
 //   a:  byte offset of the block's sign word within the wave's payload (past any
 //       outlier prefix)
-//   nb: [31:24] 0 for a block without payload (or of a truncated stream), else
-//       R + 1 (33 for 32 planes); [8] outlier-selected; [9] 32 planes (2D/3D
-//       only: the sign words move in front of the planes)
-// Lane l of a 32-lane half carries one of the block's words iff key(l) < R + 1,
-// with key(31) = 0 (the sign word, or plane 31 of a 32-plane block) and
-// key(l) = l + 1 (plane l). A lane holds its key as (key << 24) | 0xffffff, so
-// the test is one unsigned compare with nb whatever its low flag bits.
+//   nb: [31:24] 0 for a block without payload (or past the array), else R + 1
+//       (33 for 32 planes); [8] outlier-selected; [13:9] bits of the prefix - 1
+// A lane carries the word of plane p iff p + 1 < R + 1, the sign word iff
+// 0 < R + 1: its key, as lane_key, is below nb whatever nb's low flag bits.
 struct DMeta {
     uint32_t a, nb;
     __device__ __forceinline__ uint32_t off() const { return a; }
-    __device__ __forceinline__ bool wide() const { return (nb >> 9) & 1; }
     __device__ __forceinline__ bool sel() const { return (nb >> 8) & 1; }
-    __device__ __forceinline__ bool nz() const { return nb >= (1u << 24); }
-    __device__ __forceinline__ bool has(uint32_t keyx) const { return keyx < nb; }
-    // Buffer offset of the lane's word, wo bytes into the block (a block
-    // without 32 planes), or an offset past every buffer range (reads 0).
+    __device__ __forceinline__ uint32_t prefix_bits() const { return ((nb >> 9) & 31) + 1; }   // 8, 16, 24 or 32
+    // Payload offset of the lane's word, wo bytes into the block, or kAbsent.
     __device__ __forceinline__ uint32_t word_at(uint32_t keyx, uint32_t wo) const {
-        return has(keyx) ? a + wo : kAbsent;
+        return keyx < nb ? a + wo : kAbsent;
     }
 };
-template <int DIM>
+template <int MODE>
 __device__ __forceinline__ DMeta make_dmeta(uint32_t off, const BlockView& v, bool nz) {
     DMeta m;
-    const bool wide = DIM != 1 && v.R >= 32;
     m.a = off + v.head;
-    m.nb = (nz ? (v.R + 1u) << 24 : 0u) | (v.sel << 8) | ((uint32_t)wide << 9);
+    m.nb = nz ? (v.R + 1u) << 24 : 0u;
+    if constexpr (MODE == kOutlier) m.nb |= nz ? (v.sel << 8) | ((8 * v.nb - 1) << 9) : 0u;
     return m;
 }
-__device__ __forceinline__ uint32_t lane_keyx(uint32_t l) { return (((l == 31) ? 0u : l + 1u) << 24) | 0xffffffu; }
+__device__ __forceinline__ uint32_t lane_key(uint32_t key) { return (key << 24) | 0xffffffu; }
 
-// Blocks of metadata per decompress wave (its kChunks * blocks-per-chunk).
+// Blocks of metadata per decompress wave (its KC * blocks-per-chunk).
 constexpr int kMetaPerWave = 128;
 template <int WAVES>
 struct SmemD {
     uint64_t wtot[WAVES];             // per-wave byte counts
     uint64_t excl;                    // the tile's exclusive prefix (wave 0's lookback)
     DMeta meta[WAVES][kMetaPerWave];  // per-block metadata of the wave's blocks
-    // the wave's stream words, loaded densely (then read per lane): its whole
-    // payload (1D, where it fits) or one chunk's; 2D/3D: after that the
-    // chunk's decoded rows, padded
-    uint4 ostage[WAVES][kWaveBuf / 16];
+    uint4 payload[WAVES][kWaveBuf / 16];  // stream words, loaded densely and read per lane: the wave's or one chunk's
     uint32_t zero[WAVES][2];          // two zero words per wave (read by lanes without a word)
 };
 
-// Load of one element per lane. 1D loads cover whole cache lines and stream
-// (nontemporal); a 2D/3D group reads 16 or 32 bytes of each of its rows' lines,
-// whose other bytes belong to the chunk's next groups, so those loads keep
-// the lines cached.
-template <int DIM, class T>
-__device__ __forceinline__ T load_elem(const T* p) {
-    if constexpr (DIM == 1) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-
-// The wave-uniform part of the loads of a wave's G groups.
-template <int DIM, class T, int G>
-struct GroupLoads {
-    // Loads x[g] for the wave's groups grp0 .. grp0+G-1. FULL: every element
-    // lies inside the array (no per-element checks); otherwise out-of-range
-    // lanes read 0 and vmask records the valid (group, lane) pairs per group.
-    template <bool FULL>
-    __device__ __forceinline__ static void run(const T* __restrict__ in, const Geom& geo, const LaneGeo<DIM>& lg,
-                                               uint64_t grp0, int lane, T (&x)[G], uint64_t& vmask) {
-        if constexpr (FULL) {
-            vmask = (G == 64) ? ~0ull : (1ull << G) - 1;
-            if constexpr (DIM == 1) {
-                const T* p = in + grp0 * 64 + (uint64_t)lane;
-#pragma unroll
-                for (int g = 0; g < G; ++g) x[g] = load_elem<DIM>(p + 64 * g);
-            } else {
-                Walker wk;
-                wk.init(grp0, geo);
-                if (wk.bx + G <= geo.Bx) {
-                    // the G blocks are consecutive along x: origins 8 (2D) or 4 (3D) elements apart
-                    const T* p = in + block_origin<DIM>(geo, wk) + lg.off;
-#pragma unroll
-                    for (int g = 0; g < G; ++g) x[g] = load_elem<DIM>(p + (DIM == 2 ? 8 : 4) * g);
-                } else {
-#pragma unroll
-                    for (int g = 0; g < G; ++g) {
-                        x[g] = load_elem<DIM>(in + block_origin<DIM>(geo, wk) + lg.off);
-                        wk.next(geo);
-                    }
-                }
-            }
-        } else {
-            vmask = 0;
-            Walker wk;
-            if constexpr (DIM != 1) wk.init(grp0, geo);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                uint64_t idx;
-                const bool valid = elem_of<DIM>(geo, lg, wk, grp0 + g, lane, idx);
-                x[g] = valid ? load_elem<DIM>(in + idx) : T(0);
-                vmask |= (uint64_t)valid << g;
-                if constexpr (DIM != 1) wk.next(geo);
-            }
-        }
-    }
-};
-
-// Whether every element of groups grp0 .. grp0+G-1 lies inside the array.
-template <int DIM, int G>
-__device__ __forceinline__ bool groups_full(const Geom& geo, uint64_t grp0) {
-    if constexpr (DIM == 1) return (grp0 + G) * 64 <= geo.n;
-    else return geo.aligned && grp0 + G <= geo.nblocks;
+// Chunks of a wave at group wgrp0 that end within `end` groups (round: the
+// groups by which the last one may go past it).
+template <int KC>
+__device__ __forceinline__ int chunks_of(uint64_t wgrp0, uint64_t end, uint64_t round) {
+    if (wgrp0 >= end) return 0;
+    const uint64_t n = (end - wgrp0 + round) / (kChunkElems / 64);
+    return n < KC ? (int)n : KC;
 }
 
 // Compresses tile `tile` of array `cur` (every wave of the workgroup calls it).
-// Each wave runs its kChunks chunks of G groups in turn:
-//   1. loads (one element per lane per group; a chunk's G loads are issued
-//      before the previous chunk is processed);
-//   2. pass 1, per group: quantise, Lorenzo residual, sign|magnitude, bit
-//      transpose; nonzero-plane masks go to the block's bookkeeping lane;
-//   3. bookkeeping, lane j <-> block j of the chunk: header byte (to LDS, stored
-//      after the chunks), size, offset; metadata through LDS;
-//   4. the chunk's stream words are written into the wave's LDS staging area
-//      exactly as they will appear in the stream.
+// Each wave runs its KC chunks of 512 elements in turn, a quad per lane and set:
+//   1. loads (16 bytes per lane and instruction for f32; the next chunk's are
+//      issued as this chunk's values are quantised);
+//   2. quantise, Lorenzo residuals: inside the quad, and one DPP read for its
+//      first element. The block's rate is the bit length of its largest
+//      residual: minimum and maximum over the quad, then over the block's lanes;
+//   3. bookkeeping in every lane for its own block of either set: size, and the
+//      offset from one scan of both sets' sizes packed into 16 bits each;
+//   4. byte slices (as many as the chunk's largest rate needs), their transpose
+//      to plane words, and the words into the wave's LDS staging area exactly
+//      as they will appear in the stream.
 // The wave totals then combine in LDS, wave 0 runs the lookback (publishing
 // the tile's byte count first, then its inclusive prefix), and every wave
-// copies its staged payload to the stream with 16-byte stores. A wave whose
-// payload did not fit its staging area runs its chunks again and stores the
-// words directly.
-template <int DIM, int MODE, class T, int WAVES, int LB = kLookbackWords>
+// copies its staged payload to the stream with 16-byte stores. Chunks that did
+// not fit the wave's staging area any more are only counted at first; once the
+// offset is known the wave runs them again, staging and copying by turns.
+//
+// RUNS: 1D, or 2D/3D with every chunk a run of whole blocks along x
+// (Geom::runs), whose place is wave-uniform. Otherwise every quad is located
+// by itself.
+template <int DIM, int MODE, class T, int WAVES, bool RUNS, int KC = kChunksOf<T>>
 __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t tile, const ScanCtx& sc,
-                                              SmemC<WAVES>& sm) {
-    constexpr int G = ShapeC<T>::G;              // groups per chunk
+                                              SmemC<WAVES>& sm, const int window) {
+    typedef QuadLane<DIM> QL;
+    static_assert(DIM != 1 || RUNS, "1D chunks are runs");
+    constexpr int G = kChunkElems / 64;          // groups per chunk
     constexpr int S = (DIM == 1) ? 4 : 8;        // bytes per plane
-    constexpr int BPG = (DIM == 1) ? 2 : 1;      // blocks per group
-    constexpr int NB = BPG * G;                  // blocks per chunk
-    static_assert(NB <= 16 && 2 * G <= 16, "shared metadata sized for 16 blocks per chunk");
+    constexpr int SB = QL::SB, NB = QL::NB;      // blocks per set, per chunk
+    constexpr bool NT = DIM == 1;                // 1D loads stream; 2D/3D quads share lines with the other set
 
     const int lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t l = (uint32_t)lane & 31, h = (uint32_t)lane >> 5;
     const Geom& geo = cur.geo;
     const T r = (T)cur.param;
     const uint64_t lt = tile - cur.tile0;
     uint8_t* __restrict__ const dst = (uint8_t*)cur.dst;
     const T* __restrict__ const in = (const T*)cur.src;
-    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (kChunks * G);   // this wave's first group
+    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (KC * G);   // this wave's first group
 
-    LaneGeo<DIM> lg;
-    lg.init(lane, geo);
-    const int pl = pred_lane<DIM>(lane);
-    const int pl_src = pl < 0 ? lane : pl;
-    XposeConsts xc;
-    xc.init(lane, false);
-    // after the transpose, element 0 of a block is bit 7 of its plane words: in
-    // both halves for 1D (two blocks), only in the low half for 2D/3D
-    const uint32_t not_e0 = (DIM == 1 || h == 0) ? ~0x80u : ~0u;
-    // bit 7 of this lane's word is not element 0 of a plane (the sign word, or
-    // the high half of a 2D/3D block): kept in selected blocks too
-    const uint32_t keep_e0 = (l == 31 || (DIM != 1 && h != 0)) ? 0x80u : 0u;
-    const uint32_t key = (l == 31) ? 0u : l + 1u;             // see Meta::b
-    const uint32_t wo = word_offset<DIM>(l, h, true);        // this lane's word in a block's payload
-    const uint32_t wo_wide = word_offset<DIM>(l, h, false);  // same, 32-plane 2D/3D layout
-    // LDS addresses of this lane's word in the staging area (offset 0) and of
-    // the spare word past it, where lanes without a word write
+    QL ql;
+    ql.init(lane);
+    PlaneConsts pc;
+    pc.init(lane, false);
+    const uint32_t pl = plane_of_lane(ql.k);
+    // LDS addresses of the wave's staging area and of the spare word past it,
+    // where lanes without a word write
     lds_u8* const sbase = (lds_u8*)sm.stage[wave];
-    const uint32_t s0 = (uint32_t)(size_t)sbase;
-    const uint32_t so = s0 + wo, so_wide = s0 + wo_wide, spare = s0 + kStageBytes;
+    const uint32_t s0 = (uint32_t)(size_t)sbase, spare = s0 + kStageBytes;
+    // this lane's plane word of slice 0 in a block, and its header byte
+    const uint32_t po = ql.plane_offset(pl);
+    lds_u8* const hbase = (lds_u8*)sm.hdr[wave] + (ql.blk + (ql.second ? SB : 0));
 
     uint64_t excl = 0, wexcl = 0, ttot = 0;
-    uint32_t wave_tot = 0;
-    bool over = false;
-    bool lossy = false;   // a 2D/3D outlier block got rate byte 32 (see kWarnLossy)
+    uint32_t wave_tot = 0;   // the wave's payload so far, of which `copied` bytes have left the staging area
+    uint32_t copied = 0, staged = 0;
+    int c_over = KC;         // first chunk that did not fit; `staged` bytes come before it
+    bool lossy = false;      // a 2D/3D outlier block got rate byte 32 (see kWarnLossy)
 
-    // Processes chunk c from xv (vmask: valid elements per group); roll(g) runs
-    // right after group g's value is consumed (the fast path loads the next
-    // chunk's group g into xv[g] there). DIRECT: store the words at gbase
-    // instead of staging them (and write no header bytes).
-    auto process = [&](auto directc, uint8_t* const gbase, int c, T (&xv)[G], const uint64_t vmask, auto&& roll) {
-        constexpr bool DIRECT = decltype(directc)::value;
-        const uint64_t grp0 = wgrp0 + (uint64_t)c * G;
-
-        // ---- pass 1 ---------------------------------------------------------
-        // WIDE = false: the branch-free form, which assumes no 2D/3D block
-        // holds a magnitude of 2^31 and reports the groups where one does;
-        // the chunk is then rerun from memory with WIDE = true.
-        uint32_t W[G];
-        uint32_t bk1, bk2, bko;   // lane j: block j's nonzero-plane mask (all / e >= 1), |d| of element 0
-        uint32_t big;             // bit g: group g's block has a magnitude 2^31 (2D/3D)
-        auto residual = [&](const uint32_t q) -> uint32_t {
-            if constexpr (MODE == kFixed) {
-                return q;
-            } else if constexpr (DIM == 1) {
-                // q - q[lane - 1], negated from one DPP subtract (the negation is
-                // the subtraction |d| needs anyway); element 0 of each block has no
-                // predecessor: lane 31's code is not passed on, lane 0 reads 0
-                const uint32_t p = ((lane & 31) == 31) ? 0u : q;
-                return 0u - sub_prev_wave_shr1(p, q);
-            } else {
-                uint32_t qp = (uint32_t)__builtin_amdgcn_ds_bpermute(pl_src << 2, (int)q);
-                qp = (pl >= 0) ? qp : 0u;
-                return q - qp;
-            }
-        };
-        auto pass1 = [&](auto widec, auto&& xval, const uint64_t vm, auto&& roll_fn) -> uint64_t {
-            constexpr bool WIDE = decltype(widec)::value;
-            bk1 = bk2 = bko = big = 0;
-            uint64_t anywide = 0;
-            if constexpr (!WIDE) {
-                // the words of all groups first, then their transposes side by
-                // side (one LDS round trip per stage for kXposeBatch groups),
-                // then the plane masks
-                uint32_t aor = 0;   // OR of the magnitudes: bit 31 set iff some block needs 32 planes
-                auto code = [&](auto gc, uint32_t d) {   // d: group g's residual
-                    constexpr int g = decltype(gc)::value;
-                    d = ((vm >> g) & 1) ? d : 0u;   // codes and residuals of padding are 0
-                    const uint32_t a = ((int32_t)d < 0) ? 0u - d : d;
-                    if constexpr (DIM != 1) aor |= a;
-                    // sign bit over the low 31 magnitude bits; 1D ranks |-2^31| as 0
-                    // (signed running maximum, src/cuSZp_kernels_1D_f32.cu:552), so bit 31 is free
-                    W[g] = bfi(0x80000000u, d, a);
-                    if constexpr (MODE == kOutlier) {   // |d| of each block's element 0
-                        if constexpr (DIM == 1) {
-                            bko = wrlane<2 * g>(rdlane(a, 0), bko);
-                            bko = wrlane<2 * g + 1>(rdlane(a, 32), bko);
-                        } else {
-                            bko = wrlane<g>(rdlane(a, 0), bko);
-                        }
-                    }
-                };
-                if constexpr (DIM == 1 || MODE == kFixed) {
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        const uint32_t q = quantize<T>(xval(g), r);   // x = 0 outside the array (q = -1 if r = inf: masked below)
-                        roll_fn(g);
-                        code(gc, residual(q));
-                    });
-                } else {
-                    // 2D/3D Lorenzo: every group's codes first (W holds them), then
-                    // the predecessors' codes of all groups in flight together (one
-                    // LDS permute each), then the residuals
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        W[g] = quantize<T>(xval(g), r);
-                        roll_fn(g);
-                    });
-                    uint32_t QP[G];
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        QP[g] = (uint32_t)__builtin_amdgcn_ds_bpermute(pl_src << 2, (int)W[g]);
-                    });
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        code(gc, W[g] - ((pl >= 0) ? QP[g] : 0u));
-                    });
-                }
-                if constexpr (DIM != 1) anywide = ballot((int32_t)aor < 0);
-                constexpr int XB = kXposeBatch < G ? kXposeBatch : G;
+    // Processes chunk c from xv; roll(s) runs right after set s's values are
+    // consumed (the next chunk's loads into xv[s] go there). PIECES: xv holds
+    // pieces (see Pieces), all inside the array; else quads, with vm's bits
+    // 4s + i for the elements inside.
+    auto process = [&](auto piecesc, int c, T (&xv)[2][4], const uint32_t vm, auto&& roll) {
+        constexpr bool PIECES = decltype(piecesc)::value;
+        uint32_t q[2][4], d[2][4];
 #pragma unroll
-                for (int g = 0; g < G; g += XB) xpose32_n<XB>(W + g, xc);
-                static_for<0, G>([&](auto gc) {
-                    constexpr int g = decltype(gc)::value;
-                    const uint64_t m1 = ballot(W[g] != 0) & 0x7fffffff7fffffffull;
-                    uint64_t m2 = 0;
-                    if constexpr (MODE == kOutlier) {
-                        // planes nonzero without element 0 (bit 7 of the words of
-                        // planes 0..30; 2D/3D: low half only): W not in {0, 0x80}
-                        constexpr uint64_t e0lanes = (DIM == 1) ? 0x7fffffff7fffffffull : 0x7fffffffull;
-                        m2 = m1 & ~(ballot(W[g] == 0x80u) & e0lanes);
-                    }
-                    if constexpr (DIM == 1) {
-                        bk1 = wrlane<2 * g>((uint32_t)m1, bk1);
-                        bk1 = wrlane<2 * g + 1>((uint32_t)(m1 >> 32), bk1);
-                        if constexpr (MODE == kOutlier) {
-                            bk2 = wrlane<2 * g>((uint32_t)m2, bk2);
-                            bk2 = wrlane<2 * g + 1>((uint32_t)(m2 >> 32), bk2);
-                        }
-                    } else {
-                        bk1 = wrlane<g>((uint32_t)m1 | (uint32_t)(m1 >> 32), bk1);
-                        if constexpr (MODE == kOutlier) bk2 = wrlane<g>((uint32_t)m2 | (uint32_t)(m2 >> 32), bk2);
-                    }
-                });
-                return anywide;
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q[s][i] = quantize<T>(xv[s][i], r);   // x = 0 outside the array (q = -1 if r = inf: masked below)
+            roll(s);
+        }
+        if constexpr (PIECES) trade_codes<DIM, T>(q);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if constexpr (MODE == kFixed) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[s][i] = q[s][i];
+            } else {
+                d[s][0] = q[s][0] - ql.prev_code(q[s]);
+#pragma unroll
+                for (int i = 1; i < 4; ++i) d[s][i] = q[s][i] - q[s][i - 1];
             }
-            static_for<0, G>([&](auto gc) {
-                constexpr int g = decltype(gc)::value;
-                const uint32_t q = quantize<T>(xval(g), r);   // x = 0 outside the array (q = -1 if r = inf: masked below)
-                roll_fn(g);
-                uint32_t d = residual(q);
-                d = ((vm >> g) & 1) ? d : 0u;   // codes and residuals of padding are 0
-                const uint32_t a = ((int32_t)d < 0) ? 0u - d : d;
-                uint64_t m1, m2 = 0;
-                const bool wide = ballot((int32_t)a < 0) != 0;
-                if (!wide) {
-                    W[g] = xpose32(bfi(0x80000000u, d, a), xc);
-                    m1 = ballot(W[g] != 0) & 0x7fffffff7fffffffull;
-                    if constexpr (MODE == kOutlier) m2 = ballot((W[g] & not_e0) != 0) & 0x7fffffff7fffffffull;
-                } else {
-                    W[g] = xpose32(a, xc);
-                    m1 = ballot(W[g] != 0);
-                    if constexpr (MODE == kOutlier) m2 = ballot((W[g] & not_e0) != 0);
-                    const uint64_t sg = stream_order64(ballot((int32_t)d < 0));   // the sign words
-                    if (lane == 0) {
-                        sm.aux[wave][2 * g] = (uint32_t)sg;
-                        sm.aux[wave][2 * g + 1] = (uint32_t)(sg >> 32);
-                    }
-                    big |= 1u << g;
-                }
-                bk1 = wrlane<g>((uint32_t)m1 | (uint32_t)(m1 >> 32), bk1);
-                if constexpr (MODE == kOutlier) {
-                    bk2 = wrlane<g>((uint32_t)m2 | (uint32_t)(m2 >> 32), bk2);
-                    bko = wrlane<g>(rdlane(a, 0), bko);
-                }
-            });
-            return anywide;
-        };
-        const uint64_t anywide = pass1(std::false_type{}, [&](int g) -> T { return xv[g]; }, vmask, roll);
-        if constexpr (DIM != 1) {
-            if (anywide) {   // rare: rerun the chunk with 32-plane blocks
-                T xr[G];
-                uint64_t vr;
-                GroupLoads<DIM, T, G>::template run<false>(in, geo, lg, grp0, lane, xr, vr);
-                pass1(std::true_type{}, [&](int g) -> T { return xr[g]; }, vr, [](int) {});
+            if constexpr (!PIECES) {   // codes and residuals of padding are 0
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[s][i] = ((vm >> (4 * s + i)) & 1) ? d[s][i] : 0u;
             }
         }
 
-        // ---- bookkeeping: lane j <-> block j of this chunk ---------------------
-        const bool blk = lane < NB;
-        uint32_t byte;
-        BlockView v;
+        // ---- rates ----------------------------------------------------------
+        // [0]: the block's largest magnitude (outlier: of elements e >= 1),
+        // [1] (outlier): element 0's
+        constexpr int NV = (MODE == kOutlier) ? 2 : 1;
+        uint32_t v0[NV], v1[NV], bm[NV];
+        auto mx = [](int32_t a, int32_t b) { return a > b ? a : b; };
+        auto mn = [](int32_t a, int32_t b) { return a < b ? a : b; };
+        auto extremes = [&](const uint32_t (&e)[4], uint32_t (&v)[NV]) {
+            const int32_t f0 = (int32_t)(MODE == kOutlier ? e[0] & ~ql.e0 : e[0]);
+            const int32_t f1 = (int32_t)e[1], f2 = (int32_t)e[2], f3 = (int32_t)e[3];
+            const uint32_t hi = (uint32_t)mx(mx(mx(f0, f1), f2), mx(f3, 0));
+            const uint32_t lo = 0u - (uint32_t)mn(mn(mn(f0, f1), f2), mn(f3, 0));
+            v[0] = hi > lo ? hi : lo;
+            if constexpr (MODE == kOutlier) {
+                const uint32_t z = e[0] & ql.e0;
+                v[NV - 1] = (uint32_t)mx((int32_t)z, (int32_t)(0u - z));   // 2^31 stays 2^31
+            }
+        };
+        extremes(d[0], v0);
+        extremes(d[1], v1);
+        ql.template block_max<NV>(v0, v1, bm);
+        const uint32_t all = (MODE == kOutlier) ? bm[0] | bm[NV - 1] : bm[0];
+        const bool rare = ballot((int32_t)all < 0) != 0;   // a residual of magnitude 2^31 (only from saturated or wrapped codes)
+        if (DIM == 1 && rare) {   // 1D ranks |-2^31| as 0 (signed running maximum, src/cuSZp_kernels_1D_f32.cu:552)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t o = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t v = (MODE == kOutlier && i == 0) ? d[s][0] & ~ql.e0 : d[s][i];
+                    const uint32_t a = ((int32_t)v < 0 ? 0u - v : v) & 0x7fffffffu;
+                    o = o > a ? o : a;
+                }
+                (s ? v1 : v0)[0] = o;
+            }
+            ql.template block_max<NV>(v0, v1, bm);
+        }
+
+        // ---- the books: planes + 1 (0: no payload), bytes, header byte, prefix bytes
+        uint32_t b, sz, hb, nb = 0;
         if constexpr (MODE == kOutlier) {
-            if (DIM == 1 || !anywide) {
-                v = outlier_code<S>(bitlen(bk1), bitlen(bk2), bitlen(bko), byte);
-            } else {
-                byte = rate_byte<MODE, S>(bitlen(bk1), bitlen(bk2), bitlen(bko));
-                v = view_of<MODE, S>(byte);
-                // R1 = 32 (a residual of magnitude 2^31, only from saturated or
-                // wrapped codes) is kept as the plain byte 32, which every
-                // outlier decoder reads as rate 0 (written by
+            const uint32_t a0 = (DIM == 1) ? bm[1] & 0x7fffffffu : bm[1];
+            const uint32_t m1 = bm[0] > a0 ? bm[0] : a0;
+            BlockView v;
+            if (DIM != 1 && rare) {
+                hb = rate_byte<MODE, S>(bitlen(m1), bitlen(bm[0]), bitlen(bm[1]));
+                v = view_of<MODE, S>(hb);
+                // R1 = 32 is kept as the plain byte 32, which every outlier
+                // decoder reads as rate 0 (written by
                 // src/cuSZp_kernels_2D_f32.cu:1494-1505, masked with 0x1f by the
                 // decoder at :2320): the block decodes to zeros, so the call
                 // reports it
-                lossy |= ballot(blk && byte == 32u) != 0;
+                lossy |= ballot(hb == 32u) != 0;
+            } else {
+                v = outlier_code<S>(bitlen(m1), bitlen(bm[0]), bitlen(bm[1]), hb);
             }
+            nb = v.head;
+            sz = v.size;
+            b = (v.sel || v.R) ? v.R + 1 : 0u;
         } else {
-            byte = bitlen(bk1);
-            v = view_of<MODE, S>(byte);
+            hb = bitlen(bm[0]);
+            b = hb + (hb < 1u ? hb : 1u);
+            sz = S * b;
         }
-        const uint32_t sz = blk ? v.size : 0u;
-        const uint32_t incl = scan_row16(sz);   // the chunk's NB <= 16 blocks sit in lanes 0..NB-1
-        const uint32_t ctot = rdlane(incl, NB - 1);
-        const uint32_t off = wave_tot + incl - sz;   // block offset within the wave's payload
-        const Meta* const mrow = &sm.meta[wave][DIM == 1 ? h : 0];
-        if constexpr (!DIRECT) {
-            // header bytes (lane j: block j) go to the stream after the wave's
-            // chunks: no global store inside the chunk loop, whose waits for
-            // the rolling loads would otherwise also wait for those stores
-            if (blk) sm.hdr[wave][c * NB + lane] = (uint8_t)byte;
-            const bool put = !over && wave_tot + ctot <= kStageBytes;
-            over |= !put;
-            if (put) {
-                if (blk) sm.meta[wave][lane] = make_meta<MODE>(off, v, sz != 0);
-                if constexpr (MODE == kOutlier) {
-                    // |d| of element 0 (4 bytes: the sign word written next
-                    // covers the bytes past the prefix)
-                    if (blk && v.sel) *(lds_u32u*)(sbase + off) = bko;
-                }
-                // staging: every lane writes every group (lanes without a word
-                // of the block write the spare word past the area), so the
-                // metadata reads need no branches
-                if (DIM == 1 || big == 0) {
-                    Meta mnext = mrow[0];
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        const Meta m = mnext;
-                        if constexpr (g + 1 < G) mnext = mrow[BPG * (g + 1)];   // one group ahead
-                        uint32_t w = W[g];
-                        if constexpr (MODE == kOutlier) w &= m.c | keep_e0;   // element 0 travels in the prefix
-                        const uint32_t o = m.has(key) ? m.off() + so : spare;
-                        *(lds_u32u*)(size_t)o = w;
-                    });
-                } else {   // a 2D/3D group of 32 planes in the chunk
-                    static_for<0, G>([&](auto gc) {
-                        constexpr int g = decltype(gc)::value;
-                        const Meta m = mrow[g];
-                        const bool wideg = (big >> g) & 1;
-                        uint32_t w = W[g];
-                        if constexpr (MODE == kOutlier) w &= m.c | keep_e0;
-                        const uint32_t o = m.has(key) ? m.off() + (wideg ? so_wide : so) : spare;
-                        *(lds_u32u*)(size_t)o = w;
-                        if (wideg && m.nz() && lane < 2) *(lds_u32u*)(sbase + m.off() + 4 * lane) = sm.aux[wave][2 * g + lane];
-                    });
-                }
-            }
-        } else {
-            if (blk) sm.meta[wave][lane] = make_meta<MODE>(off, v, sz != 0);
-            if constexpr (MODE == kOutlier) {
-                if (blk && v.sel) store_le(gbase + off, bko, v.nb);   // |d| of element 0, little-endian
-            }
-            static_for<0, G>([&](auto gc) {
-                constexpr int g = decltype(gc)::value;
-                const Meta m = mrow[BPG * g];
-                const bool wideg = (DIM != 1) && ((big >> g) & 1);
-                uint32_t w = W[g];
-                if constexpr (MODE == kOutlier) w &= m.c | keep_e0;
-                if (m.has(key)) store_u32u(gbase + (m.off() + (wideg ? wo_wide : wo)), w);
-                if constexpr (DIM != 1) {
-                    if (wideg && m.nz() && lane < 2) store_u32u(gbase + (m.off() + 4 * lane), sm.aux[wave][2 * g + lane]);
-                }
-            });
+        // header bytes go to the stream after the wave's chunks: no global
+        // store inside the chunk loop, whose waits for the rolling loads would
+        // otherwise also wait for those stores
+        hbase[c * NB] = (uint8_t)hb;   // the same from all lanes that keep the block's books
+        const uint64_t over7 = ballot(b > 8), over15 = ballot(b > 16);
+        const uint32_t info = sz | (b << 16) | (nb << 24);
+        const uint32_t inf0 = QL::of_set(info, 0), inf1 = QL::of_set(info, 1);
+        // both sets' sizes in one scan (a set's are below 2^16 in all)
+        const uint32_t both = __builtin_amdgcn_perm(inf1, inf0, 0x05040100u);
+        const uint32_t incl = QL::scan_blocks(both);
+        const uint32_t tot = rdlane(incl, kWaveSize - 1);
+        const uint32_t ctot = (tot & 0xffffu) + (tot >> 16);
+        const uint32_t ex = incl - both;
+        const uint32_t at0 = wave_tot - copied;
+        uint32_t off[2] = {at0 + (ex & 0xffffu), at0 + (tot & 0xffffu) + (ex >> 16)};   // in the staging area
+        if (c < c_over && at0 + ctot > kStageBytes) {
+            c_over = c;
+            staged = wave_tot;
         }
         wave_tot += ctot;
-    };
-    // The chunks one by one with bounds-checked loads: tiles with elements
-    // past the array, and the direct pass. A chunk past the array's groups is
-    // all zero: rate bytes 0 in every mode and no payload, so it only writes
-    // its header bytes (1D header padding, 2D/3D pad bytes below H).
-    auto checked_chunks = [&](auto directc, uint8_t* const gbase) {
-        constexpr bool DIRECT = decltype(directc)::value;
-        const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;
-        for (int c = 0; c < kChunks; ++c) {
-            const uint64_t grp0 = wgrp0 + (uint64_t)c * G;
-            if (grp0 >= gvalid) {
-                if (!DIRECT && lane < NB) sm.hdr[wave][c * NB + lane] = 0;
-                continue;
+        if (c >= c_over) return;
+
+        // ---- the words ------------------------------------------------------
+        const uint32_t bs[2] = {(inf0 >> 16) & 0xffu, (inf1 >> 16) & 0xffu};
+        uint32_t sign0[2] = {0, 0};   // in bit 31, of an element 0 that travels in the prefix
+        if constexpr (MODE == kOutlier) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const uint32_t pre = (s ? inf1 : inf0) >> 24;
+                const bool drop = (pre & ql.e0) != 0;
+                if (drop) {
+                    // |d| of element 0, little-endian: 4 bytes, of which the
+                    // sign word written next covers what is past the prefix
+                    *(lds_u32u*)(sbase + off[s]) = (s ? v1 : v0)[NV - 1];
+                }
+                off[s] += pre;
+                sign0[s] = drop ? d[s][0] : 0u;
+                d[s][0] = drop ? 0u : d[s][0];
             }
-            T xv[G];
-            uint64_t vmask;
-            GroupLoads<DIM, T, G>::template run<false>(in, geo, lg, grp0, lane, xv, vmask);
-            process(directc, gbase, c, xv, vmask, [](int) {});
+        }
+        // a word of either half's payload; lanes without one write the spare word
+        auto word = [&](int s, bool has, uint32_t o, uint32_t w) {
+            const uint32_t at = has ? off[s] + (s0 + o) : spare;
+            *(lds_u32u*)(size_t)at = w;
+        };
+        // the words of N sets from s on
+        auto emit = [&](auto nsc, auto nc, int s) {
+            constexpr int NS = decltype(nsc)::value, N = decltype(nc)::value;
+            uint32_t w[N * NS];
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                uint32_t t[NS];
+                slices_of<NS>(d[s + j], t);
+                if constexpr (MODE == kOutlier) t[NS - 1] |= sign0[s + j] & 0x80000000u;
+#pragma unroll
+                for (int i = 0; i < NS; ++i) w[j * NS + i] = t[i];
+            }
+            to_planes<N * NS>(w, pc);
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                // plane p is there if p + 1 < b, the sign word if 0 < b
+                uint32_t k = pl, p = po;
+                opaque_here(k);
+                opaque_here(p);
+                const bool sign = i == NS - 1 && k == 7;
+                uint32_t key = sign ? 0u : 8 * i + 1 + k, o = sign ? p - 8 * S : p + 8 * S * i;   // the sign word is 8 planes in front of plane 7
+                opaque_here(key);
+                opaque_here(o);
+#pragma unroll
+                for (int j = 0; j < N; ++j) word(s + j, key < bs[s + j], o, w[j * NS + i]);
+            }
+        };
+        typedef std::integral_constant<int, 1> one;
+        typedef std::integral_constant<int, 2> two;
+        if (!over7 && !rare) {
+            emit(one{}, two{}, 0);
+        } else if (!over15 && !rare) {
+            emit(two{}, two{}, 0);
+        } else if (DIM == 1 || !rare) {
+            emit(std::integral_constant<int, 4>{}, one{}, 0);   // one set at a time: fewer registers
+            emit(std::integral_constant<int, 4>{}, one{}, 1);
+        } else {
+            // blocks of 32 planes: all 32 bits are planes and the sign words go separately
+            uint32_t k = ql.k, p = pl, o = po;
+            opaque_here(k);
+            opaque_here(p);
+            opaque_here(o);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t w[4], a[4], sg = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t neg = d[s][i] >> 31;
+                    a[i] = neg ? 0u - d[s][i] : d[s][i];
+                    sg |= (i == 0 ? neg | (sign0[s] >> 31) : neg) << (7 - 4 * (k & 1) - i);   // element e at bit e^7
+                }
+                sg <<= 8 * (k >> 1);
+                sg |= dpp<kDppQuadSwap1>(sg);
+                sg |= dpp<kDppQuadSwap2>(sg);
+                sg |= dpp<kDppHalfMirror>(sg);
+                word(s, bs[s] != 0, o - 8 * p - 8, sg);   // the same from the half's eight lanes
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    w[t] = ((a[3] >> (8 * t)) & 0xff) | (((a[2] >> (8 * t)) & 0xff) << 8) |
+                           (((a[1] >> (8 * t)) & 0xff) << 16) | (((a[0] >> (8 * t)) & 0xff) << 24);
+                to_planes<4>(w, pc);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) word(s, 8 * i + p + 1 < bs[s], o + 8 * S * i, w[i]);
+            }
         }
     };
 
-    // ---- pass 0: header bytes and staging ------------------------------------
-    // first element of chunk c's first group for this lane; with a fast tile,
-    // group g of the chunk starts `step` * g elements later
-    constexpr uint64_t step = (DIM == 1) ? 64 : (DIM == 2 ? 8 : 4);
-    // fast tile: every element inside the array and (2D/3D) each chunk's
-    // blocks consecutive along x
-    const bool fast = groups_full<DIM, kChunks * G>(geo, wgrp0) && (DIM == 1 || geo.Bx % G == 0);
-    if (fast) {
-        // wkn: the chunk whose loads are issued next (2D/3D; a run of G blocks
-        // along x, so the walker advances by G)
-        Walker wkn;
-        if constexpr (DIM != 1) wkn.init(wgrp0, geo);
-        auto chunk_ptr = [&](int c) -> const T* {
-            if constexpr (DIM == 1) return in + (wgrp0 + (uint64_t)c * G) * 64 + (uint64_t)lane;
-            else return in + block_origin<DIM>(geo, wkn) + lg.off;
-        };
-        T xv[G];
-        const T* p = chunk_ptr(0);
+    // Runs the wave's chunks from c0 on; before(c) runs first for each. A chunk
+    // past the array's groups is all zero: rate bytes 0 in every mode and no
+    // payload.
+    const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;   // groups holding elements
+    const int nch = chunks_of<KC>(wgrp0, gvalid, G - 1);                    // chunks with elements
+    auto run = [&](int c0, auto&& before) {
+        if constexpr (RUNS) {
+            const int nfull = (DIM == 1) ? chunks_of<KC>(wgrp0, geo.n / 64, 0) : nch;   // whole chunks
+            if (c0 < nfull) {
+                Walker wkn;   // 2D/3D: the chunk whose loads are issued next
+                if constexpr (DIM != 1) wkn.init(wgrp0 + (uint64_t)c0 * G, geo);
+                Pieces<DIM, T> pcs;
+                pcs.init(ql, geo, lane);
+                // chunk c's loads of set s; c only goes up (2D/3D: all sets of a chunk first)
+                auto load = [&](int c, int s, T (&x)[4]) {
+                    const T* p;
+                    if constexpr (DIM == 1) p = in + (wgrp0 + (uint64_t)c * G) * 64;
+                    else p = in + block_origin<DIM>(geo, wkn);
+                    pcs.template load<NT>(p, c < nfull, s, x);
+                    if (DIM != 1 && s == 1) wkn.step(geo, G);
+                };
+                T xv[2][4];
 #pragma unroll
-        for (int g = 0; g < G; ++g) xv[g] = load_elem<DIM>(p + step * g);
-        for (int c = 0; c + 1 < kChunks; ++c) {
-            // group g of the next chunk loads as soon as group g of this one is coded
-            if constexpr (DIM != 1) wkn.step(geo, G);
-            const T* const pn = chunk_ptr(c + 1);
-            process(std::false_type{}, nullptr, c, xv, ~0ull, [&](int g) { xv[g] = load_elem<DIM>(pn + step * g); });
+                for (int s = 0; s < 2; ++s) load(c0, s, xv[s]);
+#pragma unroll 1
+                for (int c = c0; c < nfull; ++c) {
+                    // a set's next loads follow as soon as its values are coded
+                    before(c);
+                    process(std::true_type{}, c, xv, 0u, [&](int s) { load(c + 1, s, xv[s]); });
+                }
+            }
+            if (DIM == 1 && nfull < nch) {   // the array's last elements
+                before(nfull);
+                T xv[2][4];
+                uint32_t vm = 0;
+                const uint64_t e = (wgrp0 + (uint64_t)nfull * G) * 64 + 4 * (uint64_t)lane;
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint64_t at = e + 256 * s + i;
+                        const bool v = at < geo.n;
+                        xv[s][i] = v ? in[at] : T(0);
+                        vm |= (uint32_t)v << (4 * s + i);
+                    }
+                process(std::false_type{}, nfull, xv, vm, [](int) {});
+            }
+        } else if (c0 < nch) {
+            Walker wk;
+            wk.init(wgrp0 + (uint64_t)c0 * G, geo);
+            ChunkQuads<DIM> cq;
+            cq.locate(geo, ql, wk);
+            T xv[2][4];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) load_quad<NT>(in + cq.off[s], xv[s]);
+#pragma unroll 1
+            for (int c = c0; c < nch; ++c) {
+                before(c);
+                const uint32_t vm = (cq.ok[0] ? 0xfu : 0u) | (cq.ok[1] ? 0xf0u : 0u);
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) xv[s][i] = cq.ok[s] ? xv[s][i] : T(0);
+                cq.locate(geo, ql, wk);   // quads outside the array read its first one
+                process(std::false_type{}, c, xv, vm, [&](int s) { load_quad<NT>(in + cq.off[s], xv[s]); });
+            }
         }
-        process(std::false_type{}, nullptr, kChunks - 1, xv, ~0ull, [](int) {});   // the last chunk loads nothing more
-    } else {
-        checked_chunks(std::false_type{}, nullptr);
-    }
+    };
+    run(0, [](int) {});
+    for (int c = nch; c < KC; ++c)   // 1D header padding, 2D/3D pad bytes below H
+        if (lane < NB / 4) sm.hdr[wave][c * (NB / 4) + lane] = 0;
 
     // ---- the wave's header bytes (their positions do not depend on the
-    // offset); 2D/3D pad bytes [nblocks, H) are 0 -------------------------------
+    // offset); 2D/3D pad bytes [nblocks, H) are 0. Both H and the wave's first
+    // block are multiples of 4 -------------------------------------------------
     {
-        constexpr int NBW = kChunks * NB;
-        constexpr int BPL = (NBW + kWaveSize - 1) / kWaveSize;
-        static_assert(NBW <= 128, "header bytes of a wave");
+        constexpr int NW = KC * NB / 4;
+        static_assert(KC * NB % 4 == 0 && NW <= 32, "header words of a wave");
         __builtin_amdgcn_wave_barrier();
-        const uint64_t wb0 = (DIM == 1) ? 2 * wgrp0 : wgrp0;
-#pragma unroll
-        for (int k = 0; k < BPL; ++k) {
-            const int j = BPL * lane + k;
-            const uint64_t b = wb0 + (uint64_t)j;
-            if (j < NBW && (DIM == 1 || b < geo.H)) dst[b] = sm.hdr[wave][j];
-        }
+        const uint64_t b = ((DIM == 1) ? 2 * wgrp0 : wgrp0) + 4 * (uint64_t)lane;
+        if (lane < NW && b < geo.H) store_u32u(dst + b, sm.hdr[wave][lane]);
     }
 
     // ---- the tile's offset (wave 0) ---------------------------------------------
     if (lane == 0) {
         sm.wtot[wave] = wave_tot;
-        sm.over[wave] = over;
         if (lossy) atomicOr(cur.err, kWarnLossy);
     }
     __syncthreads();
@@ -1572,9 +1780,8 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
         ttot += t;
     }
     if (wave == 0) {
-        const uint64_t e = wave_lookback<LB>(sc, tile, cur.tile0, ttot, lane, [&](uint64_t p) {
-            return compress_tile_bytes<DIM, MODE, T, kChunks * G, WAVES>((const T*)cur.src, geo, r,
-                                                                        p - cur.tile0, lane);
+        const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
+            return compress_tile_bytes<DIM, MODE, T, KC * G, WAVES>((const T*)cur.src, geo, r, p - cur.tile0, lane);
         });
         if (lane == 0) {
             sm.excl = e;
@@ -1587,68 +1794,99 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
         if (wave == 0 && lane == 0) atomicOr(cur.err, kErrOverflow);
         return;
     }
-    if (over) {   // pass 1: run the chunks again, storing directly
-        wave_tot = 0;
-        checked_chunks(std::true_type{}, dst + uniform64(geo.H + excl + wexcl));
-        return;
-    }
-
     // ---- copy the staged payload: 16 bytes per lane, then the tail bytes ---------
     uint8_t* const obase = dst + uniform64(geo.H + excl + wexcl);
-    typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
-    typedef uint32_t v4ul __attribute__((ext_vector_type(4)));
-    const uint32_t n16 = wave_tot & ~15u;
-    if (cur.flags & kItemStreamNt) {
-        for (uint32_t i = 16u * (uint32_t)lane; i < n16; i += 16u * kWaveSize)
-            __builtin_nontemporal_store(*(const v4ul*)&sm.stage[wave][i / 16], (v4uu*)(obase + i));
-    } else {
-        for (uint32_t i = 16u * (uint32_t)lane; i < n16; i += 16u * kWaveSize)
-            *(v4uu*)(obase + i) = *(const v4ul*)&sm.stage[wave][i / 16];
+    auto copy_out = [&](uint32_t upto) {   // staged bytes [copied, upto) of the wave's payload
+        typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
+        typedef uint32_t v4ul __attribute__((ext_vector_type(4)));
+        uint8_t* const o = obase + copied;
+        const uint32_t n = upto - copied;
+        if (cur.flags & kItemStreamNt) {
+            // Nontemporal stores at 16-byte-aligned addresses (the staged bytes
+            // are then read at any offset), single bytes at the ends: a
+            // compute-free kernel that reads 4 GiB and writes 3,564 bytes per 16
+            // KiB took 0.887 ms with stores from each wave's own start, 0.852 ms
+            // this way.
+            uint32_t head = (0u - (uint32_t)(uintptr_t)o) & 15u;
+            head = head < n ? head : n;
+            const uint32_t body = (n - head) & ~15u, tail = n - head - body;
+            for (uint32_t i = 16u * (uint32_t)lane; i < body; i += 16u * kWaveSize) {
+                const lds_u8* const q = sbase + head + i;
+                const v4ul v = {*(const lds_u32u*)q, *(const lds_u32u*)(q + 4), *(const lds_u32u*)(q + 8), *(const lds_u32u*)(q + 12)};
+                __builtin_nontemporal_store(v, (v4ul*)(o + head + i));
+            }
+            if ((uint32_t)lane < head) o[lane] = sbase[lane];
+            if ((uint32_t)lane < tail) o[head + body + lane] = sbase[head + body + lane];
+        } else {
+            const uint32_t n16 = n & ~15u;
+            for (uint32_t i = 16u * (uint32_t)lane; i < n16; i += 16u * kWaveSize)
+                *(v4uu*)(o + i) = *(const v4ul*)&sm.stage[wave][i / 16];
+            if ((uint32_t)lane < (n & 15u)) o[n16 + lane] = sbase[n16 + lane];
+        }
+        copied = upto;
+    };
+    if (c_over == KC) {
+        copy_out(wave_tot);
+        return;
     }
-    if ((uint32_t)lane < (wave_tot & 15u)) obase[n16 + lane] = ((const uint8_t*)sm.stage[wave])[n16 + lane];
+    // the rest of the chunks: staged as before, copied whenever the next one may not fit
+    wave_tot = staged;
+    const int c0 = c_over;
+    c_over = KC;
+    run(c0, [&](int) {
+        if (wave_tot - copied + kMaxChunkBytes > kStageBytes) {
+            __builtin_amdgcn_wave_barrier();
+            copy_out(wave_tot);
+            __builtin_amdgcn_wave_barrier();
+        }
+    });
+    __builtin_amdgcn_wave_barrier();
+    copy_out(wave_tot);
 }
 
 // Decompresses tile `tile` of array `cur` (every wave of the workgroup calls
-// it); the tile has the compress tile's shape (kChunks chunks of G groups per
+// it); the tile has the compress tile's shape (KC chunks of 512 elements per
 // wave):
 //   1. each wave reads the header bytes of its blocks (one or two per lane),
 //      scans their sizes once and writes every block's metadata (offset within
-//      the wave's payload, lane mask) to LDS;
+//      the wave's payload, planes) to LDS;
 //   2. the wave's payload offset: from the offset table (OFFS), else the wave
 //      totals combine in LDS and wave 0 runs the lookback;
-//   3. each wave works through its chunks: every lane loads its stream words
-//      (the next chunk's loads are issued while this chunk decodes), transposes
-//      them back, rebuilds q along the Lorenzo chains and stores (T)q * eb * 2.
+//   3. each wave works through its chunks: every lane reads the plane words of
+//      its lane number from the payload (one per set and byte slice; as many
+//      slices as the chunk's largest rate needs), transposes them back to its
+//      quad's residuals, sums those along the Lorenzo chains (dot products inside
+//      the quad, one scan of DPP adds across the block's lanes) and stores
+//      (T)q * eb * 2.
 //
 // OFFS (single-array launches): the wave's payload offset comes from the
 // offset table `offs` written by unit_offsets_kernel: no lookback and no
 // workgroup barrier, every wave runs on its own.
-template <int DIM, int MODE, class T, int WAVES, int LB = kLookbackWords, bool OFFS = false>
+template <int DIM, int MODE, class T, int WAVES, bool RUNS, bool OFFS = false, int KC = kChunksOf<T>>
 __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t tile, const ScanCtx& sc,
-                                                SmemD<WAVES>& sm,
+                                                SmemD<WAVES>& sm, const int window,
                                                 const unsigned long long* __restrict__ offs = nullptr) {
-    constexpr int G = ShapeC<T>::G;
+    typedef QuadLane<DIM> QL;
+    constexpr int G = kChunkElems / 64;
     constexpr int S = (DIM == 1) ? 4 : 8;
-    constexpr int BPG = (DIM == 1) ? 2 : 1;
-    constexpr int NB = BPG * G;                         // blocks per chunk
-    constexpr int NBW = kChunks * NB;                   // blocks per wave: 128, 64 or 32
+    constexpr int SB = QL::SB, NB = QL::NB;             // blocks per set, per chunk
+    constexpr int NBW = KC * NB;                        // blocks per wave
     constexpr int BPL = (NBW + kWaveSize - 1) / kWaveSize;   // blocks per bookkeeping lane
     static_assert(NBW <= 2 * kWaveSize && NBW <= kMetaPerWave, "a wave's blocks: at most two per lane");
 
     const int lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t l = (uint32_t)lane & 31, h = (uint32_t)lane >> 5;
     const Geom& geo = cur.geo;
     const uint8_t* __restrict__ cmp = (const uint8_t*)cur.src;
     const uint64_t lt = tile - cur.tile0;
-    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (kChunks * G);   // this wave's first group
-    const uint64_t wb0 = (DIM == 1) ? 2 * wgrp0 : wgrp0;                     // and first block
+    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (KC * G);   // this wave's first group
+    const uint64_t wb0 = (DIM == 1) ? 2 * wgrp0 : wgrp0;               // and first block
 
     // ---- bookkeeping: lane j holds blocks BPL*j .. BPL*j + BPL-1 of the wave ------
     BlockView v[BPL];
     uint32_t sz[BPL];
     bool okb[BPL];
-    uint32_t lsum = 0, r32 = 0;
+    uint32_t lsum = 0, rmax = 0;
 #pragma unroll
     for (int k = 0; k < BPL; ++k) {
         const int j = BPL * lane + k;
@@ -1658,7 +1896,7 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
         v[k] = view_of<MODE, S>(byte);
         sz[k] = okb[k] ? v[k].size : 0u;
         lsum += sz[k];
-        r32 |= (uint32_t)(byte >= 32);
+        rmax = rmax > v[k].R ? rmax : v[k].R;
     }
     const uint32_t incl = scan_wave(lsum);                 // < 2^32; a cross-lane scan: all lanes
     const uint32_t wtot = rdlane(incl, kWaveSize - 1);
@@ -1668,18 +1906,20 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
 #pragma unroll
         for (int k = 0; k < BPL; ++k) {
             const int j = BPL * lane + k;
-            // every entry is written: blocks past the array get an empty lane mask
-            if (j < NBW) sm.meta[wave][j] = make_dmeta<DIM>(off, v[k], okb[k] && sz[k] != 0);
+            // every entry is written: blocks past the array carry no words
+            if (j < NBW) sm.meta[wave][j] = make_dmeta<MODE>(off, v[k], okb[k] && sz[k] != 0);
             off += sz[k];
         }
     }
-    // 2D/3D blocks of 32 planes (not in outlier streams) take the general loop
-    bool wide_blocks = false;
-    if constexpr (DIM != 1 && MODE != kOutlier) wide_blocks = ballot(r32 != 0) != 0;
+    // lanes whose blocks need more than one byte slice, or more than two, or
+    // hold 32 planes (2D/3D: the sign words move in front of all planes)
+    const uint64_t over7 = ballot(rmax > 7), over15 = ballot(rmax > 15);
+    const uint64_t over31 = (MODE == kOutlier) ? 0ull : ballot(rmax > 31);
 
     uint64_t wave_base;
     if constexpr (OFFS) {
         (void)sc;
+        (void)window;
         wave_base = uniform64(offs[lt * WAVES + (uint64_t)wave]);
         __builtin_amdgcn_wave_barrier();   // the metadata in LDS is this wave's own
     } else {
@@ -1696,8 +1936,8 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
         wexcl = uniform64(wexcl);
         ttot = uniform64(ttot);
         if (wave == 0) {
-            const uint64_t e = wave_lookback<LB>(sc, tile, cur.tile0, ttot, lane, [&](uint64_t p) {
-                return header_tile_bytes<DIM, MODE, kChunks * G, WAVES>(cmp, geo, p - cur.tile0, lane);
+            const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
+                return header_tile_bytes<DIM, MODE, KC * G, WAVES>(cmp, geo, p - cur.tile0, lane);
             });
             if (lane == 0) sm.excl = e;
         }
@@ -1715,331 +1955,252 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     const int nrec = __builtin_amdgcn_readfirstlane(intact ? (int)(span < 0x7fffffffull ? span : 0x7fffffffull) : 0);
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)wbase, 0, nrec, kBufferWord3);
 
-    // outlier streams: |d0| prefix word of each selected block of this lane
-    // (masked with PK at the use, so nothing waits for the load here); a
-    // selected block starts with nb <= 4 prefix bytes and then a 4-byte sign
-    // word, so one u32 read at the block start stays inside the block
-    uint32_t PR[BPL], PK[BPL], PV[BPL];   // PV = PR & PK, formed once the first chunk's loads are issued
-#pragma unroll
-    for (int k = 0; k < BPL; ++k) PR[k] = PK[k] = PV[k] = 0;
-    auto prefixes_ready = [&]() {
-#pragma unroll
-        for (int k = 0; k < BPL; ++k) PV[k] = PR[k] & PK[k];
-    };
-    if constexpr (MODE == kOutlier) {
-        uint32_t off = incl - lsum;
-#pragma unroll
-        for (int k = 0; k < BPL; ++k) {
-            const bool pre = okb[k] && v[k].sel;
-            PR[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, pre ? off : kAbsent, 0, 0);
-            PK[k] = v[k].nb < 4 ? (1u << (8 * v[k].nb)) - 1 : ~0u;
-            off += sz[k];
-        }
-    }
-
-    XposeConsts xc;
-    xc.init(lane, true);
-    LaneGeo<DIM> lg;
-    lg.init(lane, geo);
+    QL ql;
+    ql.init(lane);
+    PlaneConsts pc;
+    pc.init(lane, true);
+    const uint32_t pl = plane_of_lane(ql.k), po = ql.plane_offset(pl);   // this lane's plane of slice 0, its word in a block
     T* __restrict__ out = (T*)cur.dst;
     const T eb = (T)cur.param;
-    const uint32_t wo = word_offset<DIM>(l, h, true);
-    const uint32_t wo_wide = word_offset<DIM>(l, h, false);
-    const uint32_t keyx = lane_keyx(l);   // see DMeta
-    constexpr uint64_t step = (DIM == 1) ? 64 : (DIM == 2 ? 8 : 4);
-    // fast tile: every element inside the array and (2D/3D) each chunk's blocks
-    // consecutive along x
-    const bool fast = groups_full<DIM, kChunks * G>(geo, wgrp0) && (DIM == 1 || geo.Bx % G == 0);
+    const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;   // groups holding elements
+    // chunks with elements of the array, and (1D) whole ones
+    const int nch = chunks_of<KC>(wgrp0, gvalid, G - 1);
+    const int nfull = (DIM == 1) ? chunks_of<KC>(wgrp0, geo.n / 64, 0) : nch;
+    Walker wkc;   // 2D/3D: the chunk being stored
+    if constexpr (DIM != 1) wkc.init(wgrp0, geo);
 
-    // metadata of this lane's block in group g of chunk c
-    auto meta = [&](int c, int g) -> DMeta { return sm.meta[wave][c * NB + BPG * g + (DIM == 1 ? (int)h : 0)]; };
-    // stream word of this lane in group g of chunk c (0 for a lane without a
-    // word and for every lane of a truncated stream); no 32-plane blocks
-    auto word = [&](int c, int g) -> uint32_t {
-        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, meta(c, g).word_at(keyx, wo), 0, 0);
-    };
-    // the same where 2D/3D blocks of 32 planes may occur
-    auto word_any = [&](int c, int g) -> uint32_t {
-        const DMeta m = meta(c, g);
-        const bool wideg = (DIM != 1) && (MODE != kOutlier) && m.wide();
-        const uint32_t o = m.off() + (wideg ? wo_wide : wo);
-        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, m.has(keyx) ? o : kAbsent, 0, 0);
-    };
-    // residuals of group g of chunk c from its word after the transpose (lane
-    // e: element e)
-    auto residual_x = [&](int c, int g, uint32_t x, auto widec) -> uint32_t {
-        constexpr bool WIDE = decltype(widec)::value;   // 2D/3D 32-plane blocks possible
-        const DMeta m = meta(c, g);
-        uint32_t a = x & 0x7fffffffu, neg = x >> 31;   // lane l: sign in bit 31 over the magnitude bits
-        if constexpr (WIDE) {
-            if (m.wide()) {   // 32 planes: the sign words sit in their own two words
-                const uint32_t sw = (intact && m.nz()) ? load_u32u(wbase + (m.off() + 4 * h)) : 0u;
-                neg = (sw >> (l ^ 7)) & 1;   // element l's sign: stream bit l^7
-                a = x;
-            }
-        }
-        if constexpr (MODE == kOutlier) {   // element 0 of a selected block (0 when not intact)
-            // block c*NB + BPG*g (+ h in 1D) is held by bookkeeping lane
-            // (block / BPL), slot (block % BPL)
-            uint32_t e0;
-            if constexpr (BPL == 2) {
-                static_assert(DIM == 1 && NB == 2 * G, "two blocks per lane: 1D f32");
-                const int ln = c * G + g;
-                e0 = h ? rdlane(PV[BPL - 1], ln) : rdlane(PV[0], ln);
-            } else if constexpr (DIM == 1) {
-                e0 = h ? rdlane(PV[0], c * NB + 2 * g + 1) : rdlane(PV[0], c * NB + 2 * g);
-            } else {
-                e0 = rdlane(PV[0], c * NB + g);
-            }
-            a = (m.sel() && l == 0 && (DIM == 1 || h == 0)) ? e0 : a;
-        }
-        return neg ? 0u - a : a;
-    };
-    // the value of code q (a block without payload, or of a truncated stream,
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) v4u lds_v4u;
+    lds_u8* const buf = (lds_u8*)sm.payload[wave];
+    const lds_u8* const zw = (const lds_u8*)&sm.zero[wave][0];
+    if (lane < 2) sm.zero[wave][lane] = 0;
+
+    // values of codes (a block without payload, or of a truncated stream,
     // decoded all-zero words: q = 0)
     auto value_of = [&](uint32_t q) -> T { return (T)(int32_t)q * eb * T(2); };   // src/cuSZp_kernels_1D_f32.cu:490
-    auto decode_x = [&](int c, int g, uint32_t x, auto widec) -> T {
-        const uint32_t d = residual_x(c, g, x, widec);
-        if constexpr (MODE == kFixed) return value_of(d);
-        else return value_of(inverse_lorenzo<DIM>(d, lane));
-    };
-    // decodes group g of chunk c from its loaded word w
-    auto decode = [&](int c, int g, uint32_t w, auto widec) -> T { return decode_x(c, g, xpose32(w, xc), widec); };
 
-    if (fast && !wide_blocks) {
-        // ---- every element inside the array, chunks along x: no branches ----------
-        // Chunks go in pairs through two word buffers: a chunk's loads are
-        // issued before the stores of the chunk decoded meanwhile (loads and
-        // stores retire in order on this GPU, so a load issued after a store
-        // would also wait for that store). The values are stored nontemporally:
-        // the output is written once, and dirty lines of it left in L2 and the
-        // last-level cache would cost the next kernel their write-back.
-        Walker wkc;   // 2D/3D: the chunk being decoded
-        if constexpr (DIM != 1) wkc.init(wgrp0, geo);
-        // 2D/3D output staging: block width BW, rows of RL values, row stride RS
-        // (values) in LDS; lane e of group g goes to row ROW, column g * BW + COL.
-        // Read back, lane j (and j + 64) takes 16 bytes: row j / VPR, vector j % VPR.
-        constexpr int BW = (DIM == 3) ? 4 : 8;
-        constexpr int RL = G * BW;
-        constexpr int RS = RL + kOutPad / (int)sizeof(T);
-        constexpr int VPR = RL * (int)sizeof(T) / 16;          // 16-byte vectors per row
-        constexpr int NR = 64 / BW;                            // rows: 16 (3D) or 8 (2D)
-        static_assert(NR * RS * (int)sizeof(T) <= kOutStage, "output staging too small");
-        static_assert(2 * 64 * 16 == NR * RL * (int)sizeof(T), "two 16-byte vectors per lane");
-        uint32_t st_w = 0, st_r = 0;   // LDS byte offsets: this lane's value / first vector
-        uint64_t roff = 0, rdelta = 0;  // global element offsets of the rows read back
-        if constexpr (DIM != 1) {
-            uint32_t rw, cw;
-            if constexpr (DIM == 3) {
-                rw = lg.zz * 4 + lg.yy;
-                cw = lg.xx;
-            } else {
-                rw = lg.r;
-                cw = lg.c;
-            }
-            st_w = (rw * RS + cw) * (uint32_t)sizeof(T);
-            const uint32_t rr = (uint32_t)lane / VPR, cv = (uint32_t)lane % VPR;
-            st_r = rr * RS * (uint32_t)sizeof(T) + cv * 16;
-            // the second vector is 64 / VPR rows further down
-            if constexpr (DIM == 3) {
-                roff = (uint64_t)(rr >> 2) * geo.XY + (uint64_t)(rr & 3) * geo.X + cv * (16 / sizeof(T));
-                rdelta = (uint64_t)(64 / VPR / 4) * geo.XY;
-            } else {
-                roff = (uint64_t)rr * geo.X + cv * (16 / sizeof(T));
-                rdelta = (uint64_t)(64 / VPR) * geo.X;
-            }
-        }
-        auto decode_chunk = [&](int c, const uint32_t (&W)[G]) {
-            uint32_t X[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) X[g] = W[g];
-            constexpr int XB = kXposeBatch < G ? kXposeBatch : G;
-#pragma unroll
-            for (int g = 0; g < G; g += XB) xpose32_n<XB>(X + g, xc);
-            // X[g]: residuals, then (batch by batch) codes
-#pragma unroll
-            for (int g = 0; g < G; ++g) X[g] = residual_x(c, g, X[g], std::false_type{});
-            if constexpr (MODE != kFixed) {
-#pragma unroll
-                for (int g = 0; g < G; g += XB) inverse_lorenzo_n<DIM, XB>(X + g, lane);
-            }
+    Pieces<DIM, T> pcs;
+    if constexpr (RUNS) pcs.init(ql, geo, lane);
+    // Stores a chunk's codes as values. Where chunks are runs of blocks, the
+    // output is written once and nontemporally (in pieces that fill lines): dirty
+    // lines of it left in L2 and the last-level cache would cost the next kernel
+    // their write-back.
+    auto store_chunk = [&](int c, uint32_t (&q)[2][4]) {
+        if (RUNS && (DIM != 1 || c < nfull)) {
+            T* o;
             if constexpr (DIM == 1) {
-                T* const orun = out + (wgrp0 + (uint64_t)c * G) * 64 + (uint64_t)lane;
-#pragma unroll
-                for (int g = 0; g < G; ++g) __builtin_nontemporal_store(value_of(X[g]), orun + step * g);
+                o = out + (wgrp0 + (uint64_t)c * G) * 64;
             } else {
-                lds_u8* const stg = (lds_u8*)sm.ostage[wave];
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    *(__attribute__((address_space(3))) T*)(stg + st_w + g * BW * sizeof(T)) = value_of(X[g]);
-                __builtin_amdgcn_wave_barrier();
-                typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-                typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
-                const v4u v0 = *(__attribute__((address_space(3))) v4u*)(stg + st_r);
-                const v4u v1 = *(__attribute__((address_space(3))) v4u*)(stg + st_r + (64 / VPR) * RS * sizeof(T));
-                __builtin_amdgcn_wave_barrier();
-                T* const ob = out + block_origin<DIM>(geo, wkc);
-                __builtin_nontemporal_store(v0, (v4uu*)(ob + roff));
-                __builtin_nontemporal_store(v1, (v4uu*)(ob + roff + rdelta));
+                o = out + block_origin<DIM>(geo, wkc);
                 wkc.step(geo, G);
             }
-        };
-        // Stream words. A chunk's payload is contiguous: where every chunk of the
-        // wave spans at most kDenseBytes from its 4-byte-aligned start, it is read
-        // with one or two dense 16-byte-per-lane loads into the wave's LDS buffer
-        // and each lane reads its words from there (lanes without a word read a
-        // zero word). Loads with some lanes past the buffer range or 14-of-64
-        // active lanes cost far more memory-pipeline time than dense ones.
-        // Otherwise each lane loads its own word from global memory.
-        uint32_t cs[kChunks + 1];   // chunk starts within the wave's payload (wave-uniform)
+            trade_codes<DIM, T>(q);
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) cs[c] = rdlane(excl0, c * NB / BPL);
-        cs[kChunks] = wtot;
-        // Buffer loads check their range per dword, so the dwords holding the
-        // payload's last bytes must lie inside it: an outlier stream whose length
-        // is not a multiple of 4 ends inside a dword, and its last wave keeps the
-        // per-lane loads (a truncated stream has an empty range: the same).
-        const bool whole = ((wtot + 3u) & ~3u) <= (uint32_t)nrec;   // every payload dword inside the range
-        bool dense = whole;
+            for (int s = 0; s < 2; ++s) {
+                T x[4];
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) dense &= cs[c + 1] - (cs[c] & ~3u) <= (uint32_t)kDenseBytes;
-        // 1D: the wave's whole payload in one burst of loads before its first
-        // chunk, where it fits the wave's buffer. A compute-free kernel with the
-        // 1D decode's traffic (2^30 f32 written, 0.94 GB read) ran 2.5-4 % faster
-        // with each wave's reads in one burst than with a read per chunk.
-        const bool burst = DIM == 1 && whole && wtot <= (uint32_t)kWaveBuf;
-        if (burst) {
-            typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-            constexpr int NL = (kWaveBuf + 1023) / 1024;
-            lds_u8* const buf = (lds_u8*)sm.ostage[wave];
-            if (lane < 2) sm.zero[wave][lane] = 0;
-            const lds_u8* const zw = (const lds_u8*)&sm.zero[wave][0];
-            v4u P[NL];
-#pragma unroll
-            for (int k = 0; k < NL; ++k) {
-                // 1 KiB per load; none past the payload; lanes past the buffer read nothing
-                const uint32_t o = 1024u * (uint32_t)k + 16u * (uint32_t)lane;
-                P[k] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rsrc, (1024u * (uint32_t)k < wtot && o < (uint32_t)kWaveBuf) ? o : kAbsent, 0, 0);
+                for (int i = 0; i < 4; ++i) x[i] = value_of(q[s][i]);
+                pcs.store(o, s, x);
             }
-            prefixes_ready();
+        } else if constexpr (DIM == 1) {   // the array's last elements
+            const uint64_t e = (wgrp0 + (uint64_t)c * G) * 64 + 4 * (uint64_t)lane;
 #pragma unroll
-            for (int k = 0; k < NL; ++k)
-                if (1024 * k + 16 * lane < kWaveBuf) ((__attribute__((address_space(3))) v4u*)buf)[64 * k + lane] = P[k];
-            __builtin_amdgcn_wave_barrier();
-            // this lane's word of group g of chunk c (block offsets are payload offsets)
-            auto word_buf = [&](int c, int g) -> uint32_t {
-                const DMeta m = meta(c, g);
-                typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
-                if constexpr (MODE != kOutlier) {
-                    return *(lds_cu32*)(m.has(keyx) ? buf + (m.a + wo) : zw);
-                } else {
-                    // (v_alignbyte uses the low two bits of its shift operand)
-                    const uint32_t o = m.a + wo;
-                    lds_cu32* const q = (lds_cu32*)(m.has(keyx) ? buf + (o & ~3u) : zw);
-                    return __builtin_amdgcn_alignbyte(q[1], q[0], o);
-                }
-            };
-            static_for<0, kChunks>([&](auto cc) {
-                constexpr int c = decltype(cc)::value;
-                uint32_t W[G];
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int g = 0; g < G; ++g) W[g] = word_buf(c, g);
-                decode_chunk(c, W);
-            });
-        } else if (dense) {
-            typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-            lds_u8* const buf = (lds_u8*)sm.ostage[wave];
-            if (lane < 2) sm.zero[wave][lane] = 0;
-            const lds_u8* const zw = (const lds_u8*)&sm.zero[wave][0];
-            // the chunk's payload from its aligned start; the second KiB only when
-            // needed (else an offset past every range: no memory access)
-            auto load_chunk = [&](int c, v4u (&P)[2]) {
-                const uint32_t a0 = cs[c] & ~3u;
-                P[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, a0 + 16u * (uint32_t)lane, 0, 0);
-                P[1] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rsrc, cs[c + 1] - a0 > 1024u ? a0 + 1024u + 16u * (uint32_t)lane : kAbsent, 0, 0);
-            };
-            auto stage_chunk = [&](const v4u (&P)[2]) {
-                __builtin_amdgcn_wave_barrier();   // the previous chunk's reads of the buffer come first
-                ((__attribute__((address_space(3))) v4u*)buf)[lane] = P[0];
-                ((__attribute__((address_space(3))) v4u*)buf)[64 + lane] = P[1];
-                __builtin_amdgcn_wave_barrier();
-            };
-            auto word_lds = [&](int c, int g) -> uint32_t {
-                const DMeta m = meta(c, g);
-                typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
-                if constexpr (MODE != kOutlier) {
-                    // fixed/plain blocks are whole 4-byte words: an aligned read
-                    const uint32_t o = m.a + wo - (cs[c] & ~3u);
-                    return *(lds_cu32*)(m.has(keyx) ? buf + o : zw);
-                } else {
-                    // outlier prefixes shift later blocks by 1-3 bytes: the two
-                    // aligned words around the word, then a byte funnel shift
-                    // (v_alignbyte uses the low two bits of its shift operand)
-                    const uint32_t o = m.a + wo - (cs[c] & ~3u);
-                    lds_cu32* const q = (lds_cu32*)(m.has(keyx) ? buf + (o & ~3u) : zw);
-                    return __builtin_amdgcn_alignbyte(q[1], q[0], o);
-                }
-            };
-            v4u PA[2], PB[2];
-            load_chunk(0, PA);
-            load_chunk(1, PB);
-            prefixes_ready();
-            static_for<0, kChunks>([&](auto cc) {
-                constexpr int c = decltype(cc)::value;
-                v4u (&P)[2] = (c % 2 == 0) ? PA : PB;
-                stage_chunk(P);
-                if constexpr (c + 2 < kChunks) load_chunk(c + 2, P);
-                uint32_t W[G];
-#pragma unroll
-                for (int g = 0; g < G; ++g) W[g] = word_lds(c, g);
-                decode_chunk(c, W);
-            });
+                for (int i = 0; i < 4; ++i)
+                    if (e + 256 * s + i < geo.n) out[e + 256 * s + i] = value_of(q[s][i]);
         } else {
-            static_assert(kChunks % 2 == 0, "chunks go in pairs");
-            // Fully unrolled: in a loop, the wait for a chunk's words at the loop
-            // head would be merged with the path from before the loop (where no
-            // stores follow the loads) and so count the previous chunk's stores as
-            // well, putting their completion on the critical path.
-            uint32_t WA[G], WB[G];
+            // every quad by its own place; plain stores, which meet in L2
+            ChunkQuads<DIM> cq;
+            cq.locate(geo, ql, wkc);
 #pragma unroll
-            for (int g = 0; g < G; ++g) WA[g] = word(0, g);
-            prefixes_ready();
+            for (int s = 0; s < 2; ++s) {
+                T x[4];
 #pragma unroll
-            for (int c = 0; c + 2 < kChunks; c += 2) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) WB[g] = word(c + 1, g);
-                decode_chunk(c, WA);
-#pragma unroll
-                for (int g = 0; g < G; ++g) WA[g] = word(c + 2, g);
-                decode_chunk(c + 1, WB);
+                for (int i = 0; i < 4; ++i) x[i] = value_of(q[s][i]);
+                if (cq.ok[s]) store_quad<false>(out + cq.off[s], x);
             }
-            // the last pair: nothing more to load after it
+        }
+    };
+
+    // Decodes chunk c; fetch(o) reads the payload word at byte offset o of the
+    // wave's payload, or 0 for o = kAbsent.
+    constexpr int LPC = NB / BPL;   // bookkeeping lanes per chunk
+    static_assert(LPC * BPL == NB, "whole lanes per chunk");
+    auto decode_chunk = [&](int c, auto&& fetch, uint32_t (&q)[2][4]) {
+        DMeta mt[2];
 #pragma unroll
-            for (int g = 0; g < G; ++g) WB[g] = word(kChunks - 1, g);
-            decode_chunk(kChunks - 2, WA);
-            decode_chunk(kChunks - 1, WB);
+        for (int s = 0; s < 2; ++s) mt[s] = sm.meta[wave][c * NB + s * SB + ql.blk];
+        const uint64_t cl = ((1ull << LPC) - 1) << (c * LPC);
+        // |d| of element 0 of a selected block: up to 4 bytes in front of its sign word
+        uint32_t e0[2] = {0, 0};
+        if constexpr (MODE == kOutlier) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const uint32_t nbits = mt[s].prefix_bits();
+                const uint32_t w = fetch(mt[s].sel() && ql.e0 ? mt[s].off() - (nbits >> 3) : kAbsent);
+                e0[s] = (w << (32 - nbits)) >> (32 - nbits);
+            }
+        }
+        auto decode = [&](auto nsc) {
+            constexpr int NS = decltype(nsc)::value;
+            uint32_t w[2 * NS];
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                uint32_t k = pl, p = po;
+                opaque_here(k);
+                opaque_here(p);
+                const bool sign = i == NS - 1 && k == 7;
+                uint32_t key = lane_key(sign ? 0u : 8 * i + 1 + k), o = sign ? p - 8 * S : p + 8 * S * i;   // the sign word is 8 planes in front of plane 7
+                opaque_here(key);
+                opaque_here(o);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) w[s * NS + i] = fetch(mt[s].word_at(key, o));
+            }
+            from_planes<2 * NS>(w, pc);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t t[NS], s0;
+#pragma unroll
+                for (int i = 0; i < NS; ++i) t[i] = w[s * NS + i];
+                Residuals<NS> rs;
+                rs.from_slices(t, s0);
+                const uint32_t r0 = (MODE == kOutlier) ? (e0[s] ^ s0) - s0 : 0u;   // 0 except in lane e0 of a selected block
+                if constexpr (MODE == kFixed) {
+                    q[s][0] = rs.template at<0>();
+                    q[s][1] = rs.template at<1>();
+                    q[s][2] = rs.template at<2>();
+                    q[s][3] = rs.template at<3>();
+                } else {
+                    ql.codes(rs, r0, q[s]);
+                }
+            }
+        };
+        if (!(over7 & cl)) {
+            decode(std::integral_constant<int, 1>{});
+        } else if (!(over15 & cl)) {
+            decode(std::integral_constant<int, 2>{});
+        } else if (DIM == 1 || MODE == kOutlier || !(over31 & cl)) {
+            decode(std::integral_constant<int, 4>{});
+        } else {
+            // 2D/3D blocks of 32 planes among the chunk's: all 32 bits are
+            // magnitude, the signs come from the sign words by themselves
+            uint32_t w[8], sg[2], k = ql.k, p = pl, o = po;
+            opaque_here(k);
+            opaque_here(p);
+            opaque_here(o);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                sg[s] = fetch(mt[s].word_at(lane_key(0), o - 8 * p - 8));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[4 * s + i] = fetch(mt[s].word_at(lane_key(8 * i + p + 1), o + 8 * S * i));
+            }
+            from_planes<8>(w, pc);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                Residuals<4> rs;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int b = 8 * (3 - i);   // element i in byte 3 - i of the slices
+                    const uint32_t a = ((w[4 * s] >> b) & 0xff) | (((w[4 * s + 1] >> b) & 0xff) << 8) |
+                                       (((w[4 * s + 2] >> b) & 0xff) << 16) | (((w[4 * s + 3] >> b) & 0xff) << 24);
+                    const uint32_t neg = (sg[s] >> (8 * (k >> 1) + 7 - 4 * (k & 1) - i)) & 1;   // element e at bit e^7
+                    rs.v[i] = neg ? 0u - a : a;
+                }
+                if constexpr (MODE == kFixed) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) q[s][i] = rs.v[i];
+                } else {
+                    ql.codes(rs, 0u, q[s]);
+                }
+            }
+        }
+    };
+
+    // Where the words come from. A chunk's payload is contiguous: where every
+    // chunk of the wave spans at most kDenseBytes from its 4-byte-aligned start,
+    // it is read with one or two dense 16-byte-per-lane loads into the wave's
+    // LDS buffer and each lane reads its words from there (lanes without a word
+    // read a zero word). Loads with some lanes past the buffer range cost far
+    // more memory-pipeline time than dense ones. Otherwise each lane loads its
+    // own words from global memory.
+    uint32_t cs[KC + 1];   // chunk starts within the wave's payload (wave-uniform)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) cs[c] = rdlane(excl0, c * LPC);
+    cs[KC] = wtot;
+    // Buffer loads check their range per dword, so the dwords holding the
+    // payload's last bytes must lie inside it: an outlier stream whose length
+    // is not a multiple of 4 ends inside a dword, and its last wave keeps the
+    // per-lane loads (a truncated stream has an empty range: the same).
+    const bool whole = ((wtot + 3u) & ~3u) <= (uint32_t)nrec;   // every payload dword inside the range
+    bool dense = whole;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) dense &= cs[c + 1] - (cs[c] & ~3u) <= (uint32_t)kDenseBytes;
+    // The wave's whole payload in one burst of loads before its first chunk,
+    // where it fits the wave's buffer. A compute-free kernel with the 1D
+    // decode's traffic (2^30 f32 written, 0.94 GB read) ran 2.5-4 % faster with
+    // each wave's reads in one burst than with a read per chunk.
+    const bool burst = whole && wtot <= (uint32_t)kWaveBuf;
+    auto fetch_lds = [&](uint32_t origin) {
+        return [=](uint32_t o) -> uint32_t {
+            const lds_u8* const p = (int32_t)o < 0 ? zw : buf + (o - origin);
+            if constexpr (MODE != kOutlier) return *(const __attribute__((address_space(3))) uint32_t*)p;   // whole 4-byte words
+            else return *(const lds_u32u*)p;   // prefixes shift later blocks by 1-3 bytes
+        };
+    };
+    if (burst) {
+        constexpr int NL = (kWaveBuf + 1023) / 1024;
+        v4u P[NL];
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            // 1 KiB per load; none past the payload; lanes past the buffer read nothing
+            const uint32_t o = 1024u * (uint32_t)k + 16u * (uint32_t)lane;
+            P[k] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc, (1024u * (uint32_t)k < wtot && o < (uint32_t)kWaveBuf) ? o : kAbsent, 0, 0);
+        }
+#pragma unroll
+        for (int k = 0; k < NL; ++k)
+            if (1024 * k + 16 * lane < kWaveBuf) ((lds_v4u*)buf)[64 * k + lane] = P[k];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int c = 0; c < nch; ++c) {
+            uint32_t q[2][4];
+            decode_chunk(c, fetch_lds(0), q);
+            store_chunk(c, q);
+        }
+    } else if (dense) {
+        // Chunk by chunk, one chunk ahead: a chunk's loads are issued after the
+        // stores of the one before the last, so that waiting for them (loads
+        // and stores retire in order on this GPU) waits for no later store.
+        auto load_chunk = [&](int c, v4u (&P)[2]) {
+            // from the chunk's aligned start; the second KiB only when needed
+            // (else an offset past every range: no memory access)
+            const uint32_t a0 = rdlane(excl0, (uint32_t)(c * LPC)) & ~3u;
+            const uint32_t a1 = c + 1 < KC ? rdlane(excl0, (uint32_t)((c + 1) * LPC)) : wtot;
+            P[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c < nch ? a0 + 16u * (uint32_t)lane : kAbsent, 0, 0);
+            P[1] = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc, c < nch && a1 - a0 > 1024u ? a0 + 1024u + 16u * (uint32_t)lane : kAbsent, 0, 0);
+        };
+        v4u P[2];
+        uint32_t q[2][4];
+        load_chunk(0, P);
+#pragma unroll 1
+        for (int c = 0; c <= nch; ++c) {
+            if (c) store_chunk(c - 1, q);
+            if (c == nch) break;
+            __builtin_amdgcn_wave_barrier();   // the previous chunk's reads of the buffer come first
+            ((lds_v4u*)buf)[lane] = P[0];
+            ((lds_v4u*)buf)[64 + lane] = P[1];
+            __builtin_amdgcn_wave_barrier();
+            load_chunk(c + 1, P);
+            decode_chunk(c, fetch_lds(rdlane(excl0, (uint32_t)(c * LPC)) & ~3u), q);
         }
     } else {
-        // ---- general: per-element checks, 32-plane blocks -------------------------
-        Walker wk;
-        if constexpr (DIM != 1) wk.init(wgrp0, geo);
-        const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;   // groups holding elements
-        prefixes_ready();
-        for (int c = 0; c < kChunks; ++c) {
-            if (wgrp0 + (uint64_t)c * G >= gvalid) break;   // the rest of the wave writes nothing
-            uint32_t W[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) W[g] = word_any(c, g);
-            const uint64_t grp0 = wgrp0 + (uint64_t)c * G;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const T val = decode(c, g, W[g], std::true_type{});
-                uint64_t idx;
-                if (elem_of<DIM>(geo, lg, wk, grp0 + g, lane, idx)) out[idx] = val;
-                if constexpr (DIM != 1) wk.next(geo);
-            }
+#pragma unroll 1
+        for (int c = 0; c < nch; ++c) {
+            uint32_t q[2][4];
+            decode_chunk(c, [&](uint32_t o) -> uint32_t { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, o, 0, 0); }, q);
+            store_chunk(c, q);
         }
     }
 }
@@ -2049,23 +2210,23 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
 // are numbered in launch order; arrays of more than one grid's tiles take
 // several launches)
 // ---------------------------------------------------------------------------
-template <int DIM, int MODE, class T, int WAVES>
+template <int DIM, int MODE, class T, int WAVES, bool RUNS>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kCompressWavesPerSimd)
 compress_kernel(const Item item, const ScanCtx sc, const uint64_t base) {
     __shared__ SmemC<WAVES> sm;
     // a compress tile's predecessors have mostly published by the time its
     // payload is staged: the 128-tile window (2 words per lane) is enough
-    compress_tile<DIM, MODE, T, WAVES, 2>(item, base + blockIdx.x, sc, sm);
+    compress_tile<DIM, MODE, T, WAVES, RUNS>(item, base + blockIdx.x, sc, sm, 2);
 }
 
 // Waves take their payload offsets from `offs` (unit_offsets_kernel, launched
 // before on the same stream); sc is unused.
-template <int DIM, int MODE, class T, int WAVES>
+template <int DIM, int MODE, class T, int WAVES, bool RUNS>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kDecompressWavesPerSimd)
 decompress_kernel(const Item item, const ScanCtx sc, const unsigned long long* __restrict__ offs,
                   const uint64_t base) {
     __shared__ SmemD<WAVES> sm;
-    decompress_tile<DIM, MODE, T, WAVES, kLookbackWords, true>(item, base + blockIdx.x, sc, sm, offs);
+    decompress_tile<DIM, MODE, T, WAVES, RUNS, true>(item, base + blockIdx.x, sc, sm, kLookbackWords, offs);
 }
 
 // ---------------------------------------------------------------------------
@@ -2096,30 +2257,34 @@ decompress_kernel(const Item item, const ScanCtx sc, const unsigned long long* _
     case 17: RUN(3, kOutlier, double); break;                                         \
     default: break;
 
-template <int WAVES, int LB>
+template <int WAVES>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kCompressWavesPerSimd)
 compress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx sc,
-                      const unsigned long long* __restrict__ epoch, const uint64_t base) {
+                      const unsigned long long* __restrict__ epoch, const int window, const uint64_t base) {
     __shared__ SmemC<WAVES> sm;
     sc.tag = (epoch[0] & kEpochMask) << kEpochShift;
     const ItemTable src{items, nitems};
     const uint64_t tile = base + blockIdx.x;
     const Item cur = src.get(src.locate(tile, 0));
-#define CUSZP_RUN_C(D, M, T) compress_tile<D, M, T, WAVES, LB>(cur, tile, sc, sm)
+#define CUSZP_RUN_C(D, M, T)                                                          \
+    if (D == 1 || cur.geo.runs) compress_tile<D, M, T, WAVES, true>(cur, tile, sc, sm, window); \
+    else compress_tile<D, M, T, WAVES, D == 1>(cur, tile, sc, sm, window)
     switch (cur.variant) { CUSZP_BATCH_CASES(CUSZP_RUN_C) }
 #undef CUSZP_RUN_C
 }
 
-template <int WAVES, int LB>
+template <int WAVES>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kDecompressWavesPerSimd)
 decompress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx sc,
-                        const unsigned long long* __restrict__ epoch, const uint64_t base) {
+                        const unsigned long long* __restrict__ epoch, const int window, const uint64_t base) {
     __shared__ SmemD<WAVES> sm;
     sc.tag = (epoch[0] & kEpochMask) << kEpochShift;
     const ItemTable src{items, nitems};
     const uint64_t tile = base + blockIdx.x;
     const Item cur = src.get(src.locate(tile, 0));
-#define CUSZP_RUN_D(D, M, T) decompress_tile<D, M, T, WAVES, LB>(cur, tile, sc, sm)
+#define CUSZP_RUN_D(D, M, T)                                                            \
+    if (D == 1 || cur.geo.runs) decompress_tile<D, M, T, WAVES, true>(cur, tile, sc, sm, window); \
+    else decompress_tile<D, M, T, WAVES, D == 1>(cur, tile, sc, sm, window)
     switch (cur.variant) { CUSZP_BATCH_CASES(CUSZP_RUN_D) }
 #undef CUSZP_RUN_D
 }

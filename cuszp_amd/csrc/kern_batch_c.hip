@@ -1,5 +1,6 @@
-// Batched compress kernel instantiations (4 or 8 waves per workgroup, lookback
-// windows of 2 or 4 words per lane) and launchers.
+// Batched compress: launcher and the kernel of 4-wave workgroups (that of 8
+// waves is a translation unit of its own, kern_batch_c8.hip: each holds every
+// variant and takes the longest of all to compile).
 #include "launch.hpp"
 
 namespace cuszp {
@@ -13,15 +14,9 @@ __global__ void bump_epoch_kernel(unsigned long long* epoch) {
 hipError_t launch_compress_batch(int waves, int window, const Item* items, uint32_t nitems, uint64_t ntiles,
                                  const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st) {
     if (!ntiles) return hipSuccess;
-#define CUSZP_LAUNCH_C(W, K)                                                                            \
-    if (waves == W && window == K)                                                                    \
-        return launch_tiles(compress_batch_kernel<W, K>, W * kWaveSize, ntiles, st, items, nitems, sc, epoch);
-    CUSZP_LAUNCH_C(4, 2)
-    CUSZP_LAUNCH_C(4, 4)
-    CUSZP_LAUNCH_C(8, 2)
-    CUSZP_LAUNCH_C(8, 4)
-#undef CUSZP_LAUNCH_C
-    return hipErrorInvalidValue;
+    if ((waves != 4 && waves != 8) || (window != 2 && window != 4)) return hipErrorInvalidValue;
+    if (waves == 8) return launch_compress_batch8(window, items, nitems, ntiles, sc, epoch, st);
+    return launch_tiles(compress_batch_kernel<4>, 4 * kWaveSize, ntiles, st, items, nitems, sc, epoch, window);
 }
 
 hipError_t launch_bump_epoch(unsigned long long* epoch, hipStream_t st) {

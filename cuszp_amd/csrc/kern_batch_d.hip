@@ -1,5 +1,5 @@
-// Batched decompress kernel instantiations (4 or 8 waves per workgroup, lookback
-// windows of 2 or 4 words per lane) and launchers.
+// Batched decompress: launcher and the kernel of 4-wave workgroups (that of 8
+// waves: kern_batch_d8.hip).
 #include "launch.hpp"
 
 namespace cuszp {
@@ -7,15 +7,9 @@ namespace cuszp {
 hipError_t launch_decompress_batch(int waves, int window, const Item* items, uint32_t nitems, uint64_t ntiles,
                                    const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st) {
     if (!ntiles) return hipSuccess;
-#define CUSZP_LAUNCH_D(W, K)                                                                            \
-    if (waves == W && window == K)                                                                    \
-        return launch_tiles(decompress_batch_kernel<W, K>, W * kWaveSize, ntiles, st, items, nitems, sc, epoch);
-    CUSZP_LAUNCH_D(4, 2)
-    CUSZP_LAUNCH_D(4, 4)
-    CUSZP_LAUNCH_D(8, 2)
-    CUSZP_LAUNCH_D(8, 4)
-#undef CUSZP_LAUNCH_D
-    return hipErrorInvalidValue;
+    if ((waves != 4 && waves != 8) || (window != 2 && window != 4)) return hipErrorInvalidValue;
+    if (waves == 8) return launch_decompress_batch8(window, items, nitems, ntiles, sc, epoch, st);
+    return launch_tiles(decompress_batch_kernel<4>, 4 * kWaveSize, ntiles, st, items, nitems, sc, epoch, window);
 }
 
 }  // namespace cuszp

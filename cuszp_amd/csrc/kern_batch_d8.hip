@@ -1,0 +1,11 @@
+// Batched decompress kernel of 8-wave workgroups (see kern_batch_d.hip).
+#include "launch.hpp"
+
+namespace cuszp {
+
+hipError_t launch_decompress_batch8(int window, const Item* items, uint32_t nitems, uint64_t ntiles, const ScanCtx& sc,
+                                    const unsigned long long* epoch, hipStream_t st) {
+    return launch_tiles(decompress_batch_kernel<8>, 8 * kWaveSize, ntiles, st, items, nitems, sc, epoch, window);
+}
+
+}  // namespace cuszp

@@ -5,12 +5,15 @@ namespace cuszp {
 
 template <int D, int M, int W>
 static hipError_t launch_c(const Item& item, const ScanCtx& sc, hipStream_t st) {
-    return launch_tiles(compress_kernel<D, M, float, W>, W * kWaveSize, item.geo.ntiles, st,
-                             item, sc);
+    if (D == 1 || item.geo.runs)
+        return launch_tiles(compress_kernel<D, M, float, W, true>, W * kWaveSize, item.geo.ntiles, st, item, sc);
+    return launch_tiles(compress_kernel<D, M, float, W, D == 1>, W * kWaveSize, item.geo.ntiles, st, item, sc);
 }
 template <int D, int M, int W>
 static hipError_t launch_d(const Item& item, const ScanCtx& sc, const unsigned long long* offs, hipStream_t st) {
-    return launch_tiles(decompress_kernel<D, M, float, W>, W * kWaveSize, item.geo.ntiles, st, item, sc, offs);
+    if (D == 1 || item.geo.runs)
+        return launch_tiles(decompress_kernel<D, M, float, W, true>, W * kWaveSize, item.geo.ntiles, st, item, sc, offs);
+    return launch_tiles(decompress_kernel<D, M, float, W, D == 1>, W * kWaveSize, item.geo.ntiles, st, item, sc, offs);
 }
 
 // offset pass: S bytes per plane (1D 4, 2D/3D 8), UB blocks per decode wave
@@ -36,7 +39,7 @@ hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item,
 
 hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
                                    const ScanCtx& sc, hipStream_t st) {
-    static_assert(128 == kChunks * ShapeC<float>::G * 2 && 64 == kChunks * ShapeC<float>::G, "decode wave units");
+    static_assert(kChunksOf<float> * kChunkElems == 128 * 32 && kChunksOf<float> * kChunkElems == 64 * 64, "decode wave units");
     switch ((dim == 1 ? 0 : 3) + mode) {
         case 0: return launch_o<kFixed, 4, 128>(item, nunits, offs, sc, st);
         case 1: return launch_o<kPlain, 4, 128>(item, nunits, offs, sc, st);

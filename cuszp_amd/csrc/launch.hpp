@@ -35,8 +35,8 @@ hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t
                                    const ScanCtx& sc, hipStream_t st);
 hipError_t launch_unit_offsets_f64(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
                                    const ScanCtx& sc, hipStream_t st);
-// Blocks one decode wave handles (kChunks chunks of G groups).
-inline uint64_t unit_blocks(int dim, bool f64) { return (uint64_t)kChunks * (f64 ? 4 : 8) * (dim == 1 ? 2 : 1); }
+// Blocks one decode wave handles.
+inline uint64_t unit_blocks(int dim, bool f64) { return tile_groups(f64, 1) * (dim == 1 ? 2 : 1); }
 // Segments of the offset pass over `nunits` units.
 inline uint64_t unit_segments(int dim, bool f64, uint64_t nunits) {
     return (nunits * unit_blocks(dim, f64) + kPrefixSegBytes - 1) / kPrefixSegBytes;
@@ -50,6 +50,10 @@ hipError_t launch_compress_batch(int waves, int window, const Item* items, uint3
                                  const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
 hipError_t launch_decompress_batch(int waves, int window, const Item* items, uint32_t nitems, uint64_t ntiles,
                                    const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
+hipError_t launch_compress_batch8(int window, const Item* items, uint32_t nitems, uint64_t ntiles, const ScanCtx& sc,
+                                  const unsigned long long* epoch, hipStream_t st);
+hipError_t launch_decompress_batch8(int window, const Item* items, uint32_t nitems, uint64_t ntiles, const ScanCtx& sc,
+                                    const unsigned long long* epoch, hipStream_t st);
 // Increments *epoch (one thread); runs before each batched launch.
 hipError_t launch_bump_epoch(unsigned long long* epoch, hipStream_t st);
 // Largest grid of a tile launch; arrays with more tiles take several launches.

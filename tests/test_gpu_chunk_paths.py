@@ -1,0 +1,59 @@
+"""Compress and decompress where their chunk paths change, against the oracle
+(byte-identical streams, bit-identical values): rates on both sides of a byte
+slice (7 | 8, 15 | 16) and mixed within a chunk, extents whose chunks are runs
+of whole blocks and extents that wrap, are cut or have rows shorter than a
+chunk, and payloads that outgrow a wave's staging area early, late or in part."""
+import numpy as np
+import pytest
+
+from tests.helpers import gpu_compress, gpu_decompress
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, (0, 0, 0), 511), (1, (0, 0, 0), 512), (1, (0, 0, 0), 16384 + 2048 + 3), (1, (0, 0, 0), 70001)]
+SHAPES += [(2, d, 0) for d in [(4, 3, 2), (60, 9, 5), (64, 8, 3), (64, 12, 2), (68, 17, 2), (128, 16, 9), (516, 20, 3), (576, 24, 2)]]
+SHAPES += [(3, d, 0) for d in [(4, 5, 3), (28, 5, 7), (32, 4, 8), (32, 6, 4), (36, 9, 5), (64, 32, 12), (100, 36, 17)]]
+
+
+def _values(n, dtype, seed, bits):
+    """Steps of up to 2^bits[k] codes in runs of 48 values: with a bound of 0.5 the codes are the values."""
+    r = np.random.default_rng(seed)
+    top = np.repeat(r.choice(np.asarray(bits), -(-n // 48)), 48)[:n]
+    step = np.floor(r.random(n) * 2.0 ** top) * r.choice([-1, 1], n)
+    x = np.cumsum(step)
+    return (x - np.round(x / 2.0**30) * 2.0**30).astype(dtype)   # codes stay below 2^31
+
+
+def _check(oracle, x, eb, mode, dim, dims):
+    want = oracle.compress(x, eb, mode, dim, dims)
+    got = gpu_compress(x, eb, mode, dim, dims)
+    assert got == want
+    y = gpu_decompress(want, x.size, x.dtype, eb, mode, dim, dims)
+    ref = oracle.decompress(want, x.size, x.dtype, eb, mode, dim, dims)
+    iv = np.uint64 if x.dtype == np.float64 else np.uint32
+    assert np.array_equal(y.view(iv), ref.view(iv))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}D-{s[2] or 'x'.join(map(str, s[1]))}")
+def test_rates_and_extents(device, oracle, shape, dtype):
+    dim, dims, n = shape
+    n = n or dims[0] * dims[1] * dims[2]
+    for k, bits in enumerate(([0, 3, 6], [6, 7], [7, 8], [0, 7, 14], [14, 15], [3, 16, 24], [0, 30])):
+        x = _values(n, dtype, 100 * k + n, bits)
+        for mode in (0, 1, 2):
+            _check(oracle, x, 0.5, mode, dim, dims)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("dim", [1, 2, 3])
+def test_staging_area_overflows(device, oracle, dim, dtype):
+    dims = {1: (0, 0, 0), 2: (192, 72, 3), 3: (96, 24, 18)}[dim]
+    n = 41472
+    for k, (low, high) in enumerate([(22, 22), (2, 26), (26, 2), (12, 12)]):
+        bits = [low] * 20 + [high] * 20      # the first and the second half of a wave's chunks
+        r = np.random.default_rng(k)
+        top = np.repeat(np.resize(bits, -(-n // 128)), 128)[:n]
+        x = (np.floor(r.random(n) * 2.0 ** top) * r.choice([-1, 1], n)).astype(dtype)
+        for mode in (0, 1, 2):
+            _check(oracle, x, 0.5, mode, dim, dims)
