@@ -2032,13 +2032,17 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
 #pragma unroll
         for (int s = 0; s < 2; ++s) mt[s] = sm.meta[wave][c * NB + s * SB + ql.blk];
         const uint64_t cl = ((1ull << LPC) - 1) << (c * LPC);
-        // |d| of element 0 of a selected block: up to 4 bytes in front of its sign word
-        uint32_t e0[2] = {0, 0};
+        // |d| of element 0 of a selected block: up to 4 bytes in front of its sign
+        // word; the planes' bits of that element (bits 0-30 of byte 3 of the
+        // lane's slices) are ignored (src/cuSZp_kernels_1D_f32.cu:1887)
+        uint32_t e0[2] = {0, 0}, keep[2] = {~0u, ~0u};
         if constexpr (MODE == kOutlier) {
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 const uint32_t nbits = mt[s].prefix_bits();
-                const uint32_t w = fetch(mt[s].sel() && ql.e0 ? mt[s].off() - (nbits >> 3) : kAbsent);
+                const bool own = mt[s].sel() && ql.e0;
+                const uint32_t w = fetch(own ? mt[s].off() - (nbits >> 3) : kAbsent);
+                keep[s] = own ? 0x00ffffffu : ~0u;
                 e0[s] = (w << (32 - nbits)) >> (32 - nbits);
             }
         }
@@ -2062,7 +2066,10 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
             for (int s = 0; s < 2; ++s) {
                 uint32_t t[NS], s0;
 #pragma unroll
-                for (int i = 0; i < NS; ++i) t[i] = w[s * NS + i];
+                for (int i = 0; i < NS; ++i) {
+                    t[i] = w[s * NS + i];
+                    if constexpr (MODE == kOutlier) t[i] &= i == NS - 1 ? keep[s] | 0x80000000u : keep[s];
+                }
                 Residuals<NS> rs;
                 rs.from_slices(t, s0);
                 const uint32_t r0 = (MODE == kOutlier) ? (e0[s] ^ s0) - s0 : 0u;   // 0 except in lane e0 of a selected block

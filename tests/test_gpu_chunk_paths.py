@@ -57,3 +57,24 @@ def test_staging_area_overflows(device, oracle, dim, dtype):
         x = (np.floor(r.random(n) * 2.0 ** top) * r.choice([-1, 1], n)).astype(dtype)
         for mode in (0, 1, 2):
             _check(oracle, x, 0.5, mode, dim, dims)
+
+
+@pytest.mark.parametrize("dim,dims,n", [(1, (0, 0, 0), 98304), (1, (0, 0, 0), 9 << 20), (3, (64, 64, 36), 147456), (2, (4096, 4104, 1), 4096 * 4104)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_any_header_byte(device, oracle, dim, dims, n, mode):
+    """Streams that no compressor wrote: all 256 header bytes of outlier mode, all rates else, any payload."""
+    r = np.random.default_rng(n + mode)
+    nb = n // (32 if dim == 1 else 64)
+    unit = 4 if dim == 1 else 8
+    head = r.integers(0, 256 if mode == 2 else 32, nb, dtype=np.uint8)
+    head[r.random(nb) < 0.9] = 0   # most of a long stream stays short
+    if n < 1 << 20:
+        head = r.permutation(np.resize(np.arange(256 if mode == 2 else 32, dtype=np.uint8), nb))
+    R = (head & 31).astype(np.int64) if mode == 2 else head.astype(np.int64)
+    sel = (head >> 7).astype(np.int64) if mode == 2 else 0
+    size = np.where((R > 0) | (sel > 0), unit + unit * R, 0) + sel * (((head >> 5) & 3).astype(np.int64) + 1)
+    pad = -(-n // 32768) * 1024 - nb if dim == 1 else -nb % 4
+    cmp = head.tobytes() + bytes(pad) + r.integers(0, 256, int(size.sum()), dtype=np.uint8).tobytes()
+    y = gpu_decompress(cmp, n, np.float32, 0.5, mode, dim, dims)
+    ref = oracle.decompress(cmp, n, np.float32, 0.5, mode, dim, dims)
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
