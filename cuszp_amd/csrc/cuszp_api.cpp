@@ -147,24 +147,32 @@ int finish_blocking(Slot& s, hipStream_t st, size_t* total) {
 
 }  // namespace
 
-TilePlan plan_tiles(int dim, int type, bool compress, const Geom& g) {
+TilePlan plan_tiles(int dim, int type, const Geom& g) {
     static const int forced = [] {
         const char* e = std::getenv("CUSZP_WAVES");
         const int w = e ? std::atoi(e) : 0;
         return (w == 4 || w == 8) ? w : 0;
     }();
     const uint64_t groups = (dim == CUSZP_DIM_1D) ? g.H / 2 : g.nblocks;   // 64-element units
-    int waves = forced;
-    if (!waves) {
-        // 8-wave tiles halve the lookbacks per byte (measured faster from 16 Mi
-        // values up); arrays of fewer than 128 such tiles (16 MiB) keep 4-wave
-        // tiles, which spread over twice as many workgroups
-        const uint64_t per8 = tile_groups(type == CUSZP_TYPE_DOUBLE, 8);
-        waves = (groups + per8 - 1) / per8 >= 128 ? 8 : 4;
-    }
-    (void)compress;   // both directions use the same tile shape
-    const uint64_t per_tile = tile_groups(type == CUSZP_TYPE_DOUBLE, waves);
-    return TilePlan{waves, (groups + per_tile - 1) / per_tile};
+    const bool f64 = type == CUSZP_TYPE_DOUBLE;
+    const int full = f64 ? kChunksOf<double> : kChunksOf<float>;
+    int waves = forced, kc = full;
+    // The smallest tile of (4 waves, 1 chunk each), (4, 2), (8, 2), (8, 4), (8, 8)
+    // that makes no more tiles than one for each of the 256 CUs (8 waves: one and
+    // a half); longer arrays take the largest. A short array's time is that of one
+    // workgroup; more tiles than that lengthen the lookback and the sums over the
+    // header instead. 1D f32 compress / decompress with (4, 8) or (8, 8) before,
+    // and now: 64 Ki values 9.2 / 9.5 -> 5.8 / 4.2 us, 1 Mi 11.1 / 10.4 -> 8.1 / 5.4,
+    // 4 Mi 13.8 / 13.2 -> 11.3 / 8.7; 16 Mi 22.3 / 21.5 with (8, 8), 30.3 with
+    // (8, 4). Powers of two only: whole tiles fill a 1D header.
+    if (!waves)
+        for (waves = 4, kc = 1; waves != 8 || kc < full;) {
+            if (groups <= tile_groups(f64, waves, kc) * (waves == 4 ? 256 : 384)) break;
+            if (waves == 4 && kc == 2) waves = 8;
+            else kc *= 2;
+        }
+    const uint64_t per_tile = tile_groups(f64, waves, kc);
+    return TilePlan{waves, kc, (groups + per_tile - 1) / per_tile};
 }
 
 namespace {
@@ -184,8 +192,9 @@ int compress_once(const void* in, unsigned char* out, size_t cap, size_t n, size
     if (!in || !out) return CUSZP_ERROR_INVALID_ARGUMENT;
     if (max_stream_bytes(dim, g) > kMaxStream) return CUSZP_ERROR_TOO_LARGE;
     if (cap < g.H) return CUSZP_ERROR_OUTPUT_TOO_SMALL;
-    const TilePlan plan = plan_tiles(dim, type, true, g);
+    const TilePlan plan = plan_tiles(dim, type, g);
     g.ntiles = plan.ntiles;
+    g.kc = plan.kc;
     int dev = 0;
     CUSZP_HIP(hipGetDevice(&dev));
     Slot& s = slot_for(dev, st);
@@ -213,26 +222,32 @@ int decompress_once(void* out, const unsigned char* cmp, size_t n, size_t cmp_si
     if (!out || !cmp) return CUSZP_ERROR_INVALID_ARGUMENT;
     if (max_stream_bytes(dim, g) > kMaxStream) return CUSZP_ERROR_TOO_LARGE;
     if (cmp_size < g.H) return CUSZP_ERROR_CORRUPT_STREAM;
-    const TilePlan plan = plan_tiles(dim, type, false, g);
+    const TilePlan plan = plan_tiles(dim, type, g);
     g.ntiles = plan.ntiles;
+    g.kc = plan.kc;
     const bool f64 = type == CUSZP_TYPE_DOUBLE;
     const uint64_t nunits = plan.ntiles * (uint64_t)plan.waves;   // decode waves
     int dev = 0;
     CUSZP_HIP(hipGetDevice(&dev));
     Slot& s = slot_for(dev, st);
     std::lock_guard<std::mutex> lk(s.mu);
-    // the offset pass scans its segments with the slot's status words
-    rc = prepare(s, unit_segments(dim, f64, nunits), st);
-    if (!rc) rc = prepare_offsets(s, nunits, st);
+    // the offset pass scans its segments with the slot's status words; short
+    // headers need none
+    const bool direct = g.H <= kDirectHeader;
+    rc = prepare(s, direct ? 1 : unit_segments(dim, f64, nunits), st);
+    if (!rc && !direct) rc = prepare_offsets(s, nunits, st);
     if (rc) return rc;
     const ScanCtx sc = scan_ctx(s);
     Item item = make_item(cmp, out, cmp_size, nullptr, (unsigned int*)(s.d_misc + 2), decompress_param(eb, type),
                           dim, type, mode, g);
-    hipError_t e = f64 ? launch_unit_offsets_f64(dim, mode, item, nunits, s.d_offs, sc, st)
-                       : launch_unit_offsets_f32(dim, mode, item, nunits, s.d_offs, sc, st);
+    hipError_t e = hipSuccess;
+    if (!direct)
+        e = f64 ? launch_unit_offsets_f64(dim, mode, item, nunits, s.d_offs, sc, st)
+                : launch_unit_offsets_f32(dim, mode, item, nunits, s.d_offs, sc, st);
     if (e != hipSuccess) return CUSZP_ERROR_HIP;
-    e = f64 ? launch_decompress_f64(dim, mode, plan.waves, item, sc, s.d_offs, st)
-            : launch_decompress_f32(dim, mode, plan.waves, item, sc, s.d_offs, st);
+    const unsigned long long* const offs = direct ? nullptr : s.d_offs;
+    e = f64 ? launch_decompress_f64(dim, mode, plan.waves, item, sc, offs, st)
+            : launch_decompress_f32(dim, mode, plan.waves, item, sc, offs, st);
     if (e != hipSuccess) return CUSZP_ERROR_HIP;
     if (!blocking) return CUSZP_SUCCESS;
     return finish_blocking(s, st, nullptr);

@@ -80,6 +80,15 @@ constexpr uint32_t kSpinLimit = 1u << 18;
 // reference clock) makes the waiting wave compute pending predecessors itself.
 constexpr uint64_t kStealTicks = 10000;
 
+// Tile shape. A wave works through up to kChunksOf<T> chunks of 512 elements
+// (16 KiB of values), or fewer where an array would not fill the chip
+// (Geom::kc); a tile is WAVES * kc chunks, for compress and decompress alike.
+constexpr int kChunkElems = 512;
+template <class T> constexpr int kChunksOf = sizeof(T) == 4 ? 8 : 4;
+__host__ __device__ constexpr uint64_t tile_groups(bool f64, int waves, int kc = 0) {   // groups of 64 elements
+    return (uint64_t)waves * (kc ? kc : (f64 ? kChunksOf<double> : kChunksOf<float>)) * (kChunkElems / 64);
+}
+
 struct Geom {
     uint64_t n;         // elements
     uint64_t nblocks;   // cuSZp blocks
@@ -88,6 +97,7 @@ struct Geom {
     uint64_t XY;        // X*Y
     uint32_t X, Y, Z;
     uint32_t Bx, By;    // blocks along x and y (2D/3D)
+    uint32_t kc;        // chunks per wave of a tile (at most kChunksOf)
     uint32_t runs;      // every chunk's blocks lie inside the array, 2D/3D consecutive along x (extents multiples
                         // of the block, Bx of a chunk's 8 blocks), and their places fit 32-bit offsets
 };
@@ -1129,8 +1139,9 @@ __device__ __forceinline__ uint32_t or_half(uint32_t v) {
 // Payload bytes of local tile `lt` of a compress item, by one wave. Same block
 // sizes as pass 1 of compress_tile: a block's rate is the bit length of the OR of
 // its magnitudes (the highest non-zero plane), 1D ranks |-2^31| as 0.
-template <int DIM, int MODE, class T, int G, int WAVES>
+template <int DIM, int MODE, class T, int WAVES>
 __device__ uint64_t compress_tile_bytes(const T* __restrict__ in, const Geom& geo, T r, uint64_t lt, int lane) {
+    const int G = (int)geo.kc * (kChunkElems / 64);   // groups per wave
     constexpr int S = (DIM == 1) ? 4 : 8;
     LaneGeo<DIM> lg;
     lg.init(lane, geo);
@@ -1180,21 +1191,58 @@ __device__ uint64_t compress_tile_bytes(const T* __restrict__ in, const Geom& ge
     return sum;
 }
 
+// Payload bytes that header bytes describe, four at a time: sums over the bytes
+// of a word with v_sad_u8, counts of the non-zero ones with v_bcnt.
+template <int MODE, int S>
+struct HeaderSum {
+    uint32_t r = 0, n = 0, p = 0;   // rates, blocks with payload, prefix bytes
+    __device__ __forceinline__ void add(uint32_t x) {
+        const uint32_t rates = (MODE == kOutlier) ? x & 0x1f1f1f1fu : x;
+        r = __builtin_amdgcn_sad_u8(rates, 0u, r);
+        // bit 7 of a byte: it is not 0 (outlier: its rate is not 0, or it is a selected block's)
+        n += __builtin_popcount((((rates & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
+        if constexpr (MODE == kOutlier) {
+            const uint32_t sel = (x >> 7) & 0x01010101u;
+            p = __builtin_amdgcn_sad_u8((x >> 5) & (sel | (sel << 1)), 0u, p) + __builtin_popcount(sel);
+        }
+    }
+    __device__ __forceinline__ uint32_t bytes() const { return S * (r + n) + p; }
+};
+// This lane's share of the bytes that the header bytes [b0, b1) describe; both
+// are multiples of 16, lanes i of n take every n-th 16 bytes.
+template <int MODE, int S>
+__device__ __forceinline__ uint32_t header_share(const uint8_t* __restrict__ cmp, uint64_t b0, uint64_t b1, uint32_t i, uint32_t n) {
+    typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
+    constexpr int U = 4;   // loads in flight
+    HeaderSum<MODE, S> h;
+    for (uint64_t b = b0 + 16 * (uint64_t)i; b < b1; b += 16 * U * (uint64_t)n) {
+        v4uu w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t at = b + 16 * u * (uint64_t)n;
+            w[u] = *(const v4uu*)(cmp + (at < b1 ? at : b));
+            if (at >= b1) w[u] = 0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) h.add(w[u][k]);
+    }
+    return h.bytes();
+}
+
 // Payload bytes of local tile `lt` of a decompress item, from its header bytes.
-template <int DIM, int MODE, int G, int WAVES>
+template <int DIM, int MODE, int WAVES>
 __device__ uint64_t header_tile_bytes(const uint8_t* __restrict__ cmp, const Geom& geo, uint64_t lt, int lane) {
     constexpr int S = (DIM == 1) ? 4 : 8;
-    constexpr int BPT = WAVES * G * ((DIM == 1) ? 2 : 1);   // blocks per tile
+    const uint32_t bpt = WAVES * geo.kc * (kChunkElems / 64) * ((DIM == 1) ? 2 : 1);   // blocks per tile
     const uint64_t limit = (DIM == 1) ? geo.H : geo.nblocks;
     uint64_t sum = 0;
-#pragma unroll
-    for (int c = 0; c < (BPT + kWaveSize - 1) / kWaveSize; ++c) {
-        const uint64_t b = lt * BPT + (uint64_t)(c * kWaveSize + lane);
-        const bool in_tile = c * kWaveSize + lane < BPT;
-        const uint32_t byte = (in_tile && b < limit) ? (uint32_t)cmp[b] : 0u;
-        sum += wave_sum_u40(view_of<MODE, S>(byte).size);
+    for (uint32_t j = (uint32_t)lane; j < bpt; j += kWaveSize) {
+        const uint64_t b = lt * bpt + j;
+        sum += view_of<MODE, S>(b < limit ? (uint32_t)cmp[b] : 0u).size;
     }
-    return sum;
+    return wave_sum_u40(sum);
 }
 
 // Lookback window of a tile: 64 * kLookbackWords predecessors per round trip.
@@ -1212,52 +1260,50 @@ constexpr uint64_t kStatusGuard = 64 * kLookbackWords;
 //
 // The pass is itself one single-pass decoupled-lookback scan, over segments of
 // kPrefixThreads x kPrefixBytes header bytes: thread t of segment s sums the
-// block sizes of header bytes [(s * kPrefixThreads + t) * kPrefixBytes, +kPrefixBytes),
-// which hold kPrefixBytes / UB whole units.
+// block sizes of header bytes [(s * kPrefixThreads + t) * kPrefixBytes, +kPrefixBytes).
+// Few bytes per thread and many segments: the pass is bound by its latency, not
+// by the read (128 bytes per thread, one by one, took 12.5 us for the 2 MiB
+// header of 512^3 values, this 6.5).
 // ---------------------------------------------------------------------------
+// Longest header whose sums every workgroup takes by itself (single arrays,
+// arrays of a batch). The sums cost the number of tiles times the length, the
+// offset pass and its launch 3-4 us: 1D f32 with 128 KiB of header 13.2 against
+// 15.8 us, 256 KiB 14.8 against 15.7, 512 KiB 25.6 against 21.5; 1D f64 with
+// 128 KiB 11.5 against 13.0, 256 KiB 20.0 either way, 512 KiB 46.6 against 32.3.
+constexpr uint64_t kDirectHeader = 256 << 10;
+constexpr uint64_t kBatchDirectHeader = 16 << 10;
 constexpr int kPrefixThreads = 256;
-constexpr int kPrefixBytes = 128;
+constexpr int kPrefixBytes = 32;
 constexpr uint64_t kPrefixSegBytes = (uint64_t)kPrefixThreads * kPrefixBytes;
 
-// Payload bytes of the header bytes [b0, b0 + kPrefixBytes) per unit of UB
-// blocks; bytes at or past `limit` (2D/3D: the block count, so header pad
-// bytes count nothing) are blocks without payload.
-template <int MODE, int S, int UB>
-__device__ __forceinline__ void unit_sums(const uint8_t* __restrict__ cmp, uint64_t b0, uint64_t limit,
-                                          uint32_t (&sums)[kPrefixBytes / UB]) {
-    static_assert(kPrefixBytes % UB == 0 && UB % 16 == 0, "whole units of 16-byte words");
-    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+// Payload bytes of the header bytes [b0, b0 + kPrefixBytes); bytes at or past
+// `limit` (2D/3D: the block count, so header pad bytes count nothing) are
+// blocks without payload.
+template <int MODE, int S>
+__device__ __forceinline__ uint32_t thread_bytes(const uint8_t* __restrict__ cmp, uint64_t b0, uint64_t limit) {
     typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
     constexpr int V = kPrefixBytes / 16;
-    v4u w[V];
+    HeaderSum<MODE, S> h;
     if (b0 + kPrefixBytes <= limit) {
+        v4uu w[V];
 #pragma unroll
-        for (int i = 0; i < V; ++i) w[i] = __builtin_nontemporal_load((const v4uu*)(cmp + b0) + i);
+        for (int i = 0; i < V; ++i) w[i] = *((const v4uu*)(cmp + b0) + i);
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) h.add(w[i][k]);
     } else {
-        uint32_t* wb = (uint32_t*)w;
-#pragma unroll
-        for (int i = 0; i < 4 * V; ++i) {
+        for (int i = 0; i < kPrefixBytes / 4; ++i) {
             uint32_t v = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const uint64_t b = b0 + 4 * i + k;
                 v |= (b < limit ? (uint32_t)cmp[b] : 0u) << (8 * k);
             }
-            wb[i] = v;
+            h.add(v);
         }
     }
-    const uint32_t* wb = (const uint32_t*)w;
-#pragma unroll
-    for (int u = 0; u < kPrefixBytes / UB; ++u) {
-        uint32_t s = 0;
-#pragma unroll
-        for (int i = 0; i < UB / 4; ++i) {
-            const uint32_t x = wb[u * (UB / 4) + i];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) s += view_of<MODE, S>((x >> (8 * k)) & 0xffu).size;
-        }
-        sums[u] = s;
-    }
+    return h.bytes();
 }
 
 // Payload bytes of segment `seg`, by one wave (a waiting wave's recomputation
@@ -1280,7 +1326,7 @@ __global__ void __launch_bounds__(kPrefixThreads)
 unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const uint64_t H, const uint64_t nunits,
                     unsigned long long* __restrict__ offs, unsigned long long* __restrict__ total,
                     const ScanCtx sc, const uint64_t nseg, const uint64_t base) {
-    constexpr int UPT = kPrefixBytes / UB;   // units per thread
+    static_assert(UB % kPrefixBytes == 0 && kPrefixSegBytes % UB == 0, "units of whole threads in segments of whole units");
     constexpr int NW = kPrefixThreads / kWaveSize;
     __shared__ uint32_t wsum[NW];
     __shared__ uint64_t excl;
@@ -1288,12 +1334,8 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
     const int t = (int)threadIdx.x, lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint64_t th = seg * kPrefixThreads + (uint64_t)t;
-    uint32_t sums[UPT];
-    unit_sums<MODE, S, UB>(cmp, th * kPrefixBytes, limit, sums);
-    uint32_t tot = 0;
-#pragma unroll
-    for (int k = 0; k < UPT; ++k) tot += sums[k];
-    const uint32_t incl = scan_wave(tot);   // < 2^32: a segment holds at most 2^15 blocks of <= 2 KiB
+    const uint32_t tot = thread_bytes<MODE, S>(cmp, th * kPrefixBytes, limit);
+    const uint32_t incl = scan_wave(tot);   // < 2^32: a segment holds 2^13 blocks of <= 2 KiB
     if (lane == kWaveSize - 1) wsum[wave] = incl;
     // wave 0's first lookback read overlaps the other waves' sums
     LookbackWindow<kLookbackWords> pre = {};
@@ -1316,27 +1358,15 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
         }
     }
     __syncthreads();
-    uint64_t o = H + excl + wex + (incl - tot);
-#pragma unroll
-    for (int k = 0; k < UPT; ++k) {
-        const uint64_t u = th * UPT + (uint64_t)k;
-        if (u < nunits) offs[u] = o;
-        o += sums[k];
+    if (t % (UB / kPrefixBytes) == 0) {   // the unit's first thread
+        const uint64_t u = th / (UB / kPrefixBytes);
+        if (u < nunits) offs[u] = H + excl + wex + (incl - tot);
     }
 }
 
 // ---------------------------------------------------------------------------
 // one tile per workgroup pass
 // ---------------------------------------------------------------------------
-
-// Tile shape. A wave works through KC chunks of 512 elements (kChunksOf<T> of
-// them: 16 KiB of values); a tile is WAVES * KC chunks, for compress and
-// decompress alike.
-constexpr int kChunkElems = 512;
-template <class T> constexpr int kChunksOf = sizeof(T) == 4 ? 8 : 4;
-__host__ __device__ constexpr uint64_t tile_groups(bool f64, int waves) {   // groups of 64 elements
-    return (uint64_t)waves * (f64 ? 4 : 8) * (kChunkElems / 64);
-}
 
 // Compressed bytes a compress wave stages in LDS. A wave's chunks past that
 // (compression ratio below about 2.7 on its share of the tile) run twice.
@@ -1405,18 +1435,18 @@ template <int WAVES>
 struct SmemD {
     uint64_t wtot[WAVES];             // per-wave byte counts
     uint64_t excl;                    // the tile's exclusive prefix (wave 0's lookback)
+    uint32_t before[WAVES];           // per-wave shares of the payload before the tile
     DMeta meta[WAVES][kMetaPerWave];  // per-block metadata of the wave's blocks
     uint4 payload[WAVES][kWaveBuf / 16];  // stream words, loaded densely and read per lane: the wave's or one chunk's
     uint32_t zero[WAVES][2];          // two zero words per wave (read by lanes without a word)
 };
 
-// Chunks of a wave at group wgrp0 that end within `end` groups (round: the
+// Chunks (of kc) of a wave at group wgrp0 that end within `end` groups (round: the
 // groups by which the last one may go past it).
-template <int KC>
-__device__ __forceinline__ int chunks_of(uint64_t wgrp0, uint64_t end, uint64_t round) {
+__device__ __forceinline__ int chunks_of(int kc, uint64_t wgrp0, uint64_t end, uint64_t round) {
     if (wgrp0 >= end) return 0;
     const uint64_t n = (end - wgrp0 + round) / (kChunkElems / 64);
-    return n < KC ? (int)n : KC;
+    return n < (uint64_t)kc ? (int)n : kc;
 }
 
 // Compresses tile `tile` of array `cur` (every wave of the workgroup calls it).
@@ -1440,7 +1470,7 @@ __device__ __forceinline__ int chunks_of(uint64_t wgrp0, uint64_t end, uint64_t 
 // RUNS: 1D, or 2D/3D with every chunk a run of whole blocks along x
 // (Geom::runs), whose place is wave-uniform. Otherwise every quad is located
 // by itself.
-template <int DIM, int MODE, class T, int WAVES, bool RUNS, int KC = kChunksOf<T>>
+template <int DIM, int MODE, class T, int WAVES, bool RUNS>
 __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t tile, const ScanCtx& sc,
                                               SmemC<WAVES>& sm, const int window) {
     typedef QuadLane<DIM> QL;
@@ -1453,11 +1483,12 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     const int lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const Geom& geo = cur.geo;
+    const int KC = (int)geo.kc;
     const T r = (T)cur.param;
     const uint64_t lt = tile - cur.tile0;
     uint8_t* __restrict__ const dst = (uint8_t*)cur.dst;
     const T* __restrict__ const in = (const T*)cur.src;
-    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (KC * G);   // this wave's first group
+    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (uint64_t)(KC * G);   // this wave's first group
 
     QL ql;
     ql.init(lane);
@@ -1688,10 +1719,10 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     // past the array's groups is all zero: rate bytes 0 in every mode and no
     // payload.
     const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;   // groups holding elements
-    const int nch = chunks_of<KC>(wgrp0, gvalid, G - 1);                    // chunks with elements
+    const int nch = chunks_of(KC, wgrp0, gvalid, G - 1);                    // chunks with elements
     auto run = [&](int c0, auto&& before) {
         if constexpr (RUNS) {
-            const int nfull = (DIM == 1) ? chunks_of<KC>(wgrp0, geo.n / 64, 0) : nch;   // whole chunks
+            const int nfull = (DIM == 1) ? chunks_of(KC, wgrp0, geo.n / 64, 0) : nch;   // whole chunks
             if (c0 < nfull) {
                 Walker wkn;   // 2D/3D: the chunk whose loads are issued next
                 if constexpr (DIM != 1) wkn.init(wgrp0 + (uint64_t)c0 * G, geo);
@@ -1760,8 +1791,8 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     // offset); 2D/3D pad bytes [nblocks, H) are 0. Both H and the wave's first
     // block are multiples of 4 -------------------------------------------------
     {
-        constexpr int NW = KC * NB / 4;
-        static_assert(KC * NB % 4 == 0 && NW <= 32, "header words of a wave");
+        const int NW = KC * NB / 4;
+        static_assert(NB % 4 == 0 && kChunksOf<T> * NB / 4 <= 32, "header words of a wave");
         __builtin_amdgcn_wave_barrier();
         const uint64_t b = ((DIM == 1) ? 2 * wgrp0 : wgrp0) + 4 * (uint64_t)lane;
         if (lane < NW && b < geo.H) store_u32u(dst + b, sm.hdr[wave][lane]);
@@ -1781,7 +1812,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     }
     if (wave == 0) {
         const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
-            return compress_tile_bytes<DIM, MODE, T, KC * G, WAVES>((const T*)cur.src, geo, r, p - cur.tile0, lane);
+            return compress_tile_bytes<DIM, MODE, T, WAVES>((const T*)cur.src, geo, r, p - cur.tile0, lane);
         });
         if (lane == 0) {
             sm.excl = e;
@@ -1859,10 +1890,15 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
 //      the quad, one scan of DPP adds across the block's lanes) and stores
 //      (T)q * eb * 2.
 //
-// OFFS (single-array launches): the wave's payload offset comes from the
-// offset table `offs` written by unit_offsets_kernel: no lookback and no
-// workgroup barrier, every wave runs on its own.
-template <int DIM, int MODE, class T, int WAVES, bool RUNS, bool OFFS = false, int KC = kChunksOf<T>>
+// The wave's payload offset is the sum of the block sizes before it:
+//   * SINGLE (single-array launches) with an offset table `offs`
+//     (unit_offsets_kernel): read from there; no lookback and no workgroup
+//     barrier, every wave runs on its own;
+//   * SINGLE without, and arrays of a batch with short headers: the workgroup
+//     sums the header bytes in front of its tile itself (a read that hits in
+//     cache, and no pass and no waiting for other tiles);
+//   * else: the tile lookback.
+template <int DIM, int MODE, class T, int WAVES, bool RUNS, bool SINGLE>
 __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t tile, const ScanCtx& sc,
                                                 SmemD<WAVES>& sm, const int window,
                                                 const unsigned long long* __restrict__ offs = nullptr) {
@@ -1870,16 +1906,17 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     constexpr int G = kChunkElems / 64;
     constexpr int S = (DIM == 1) ? 4 : 8;
     constexpr int SB = QL::SB, NB = QL::NB;             // blocks per set, per chunk
-    constexpr int NBW = KC * NB;                        // blocks per wave
-    constexpr int BPL = (NBW + kWaveSize - 1) / kWaveSize;   // blocks per bookkeeping lane
-    static_assert(NBW <= 2 * kWaveSize && NBW <= kMetaPerWave, "a wave's blocks: at most two per lane");
+    constexpr int NBX = kChunksOf<T> * NB;              // blocks per wave, at most
+    constexpr int BPL = (NBX + kWaveSize - 1) / kWaveSize;   // blocks per bookkeeping lane
+    static_assert(NBX <= 2 * kWaveSize && NBX <= kMetaPerWave, "a wave's blocks: at most two per lane");
 
     const int lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const Geom& geo = cur.geo;
+    const int KC = (int)geo.kc, NBW = KC * NB;          // blocks per wave
     const uint8_t* __restrict__ cmp = (const uint8_t*)cur.src;
     const uint64_t lt = tile - cur.tile0;
-    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (KC * G);   // this wave's first group
+    const uint64_t wgrp0 = (lt * WAVES + (uint64_t)wave) * (uint64_t)(KC * G);   // this wave's first group
     const uint64_t wb0 = (DIM == 1) ? 2 * wgrp0 : wgrp0;               // and first block
 
     // ---- bookkeeping: lane j holds blocks BPL*j .. BPL*j + BPL-1 of the wave ------
@@ -1917,12 +1954,17 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     const uint64_t over31 = (MODE == kOutlier) ? 0ull : ballot(rmax > 31);
 
     uint64_t wave_base;
-    if constexpr (OFFS) {
-        (void)sc;
-        (void)window;
+    if (SINGLE && offs) {
         wave_base = uniform64(offs[lt * WAVES + (uint64_t)wave]);
         __builtin_amdgcn_wave_barrier();   // the metadata in LDS is this wave's own
     } else {
+        const bool direct = SINGLE || geo.H <= kBatchDirectHeader;
+        if (direct) {   // the header bytes in front of the tile: a multiple of 16
+            const uint64_t before = lt * WAVES * (uint64_t)NBW;
+            const uint32_t share = header_share<MODE, S>(cmp, 0, before, threadIdx.x, WAVES * kWaveSize);
+            const uint32_t sum = rdlane(scan_wave(share), kWaveSize - 1);   // < 2^32: at most kDirectHeader blocks
+            if (lane == 0) sm.before[wave] = sum;
+        }
         if (lane == 0) sm.wtot[wave] = wtot;
         __syncthreads();
         uint64_t wexcl = 0, ttot = 0;
@@ -1931,18 +1973,24 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
             const uint64_t t = sm.wtot[w];
             wexcl += (w < wave) ? t : 0;
             ttot += t;
+            if (direct) wexcl += sm.before[w];
         }
         // wave-uniform: kept in scalar registers across the lookback
         wexcl = uniform64(wexcl);
         ttot = uniform64(ttot);
-        if (wave == 0) {
-            const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
-                return header_tile_bytes<DIM, MODE, KC * G, WAVES>(cmp, geo, p - cur.tile0, lane);
-            });
-            if (lane == 0) sm.excl = e;
+        if constexpr (!SINGLE) {
+            if (!direct) {
+                if (wave == 0) {
+                    const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
+                        return header_tile_bytes<DIM, MODE, WAVES>(cmp, geo, p - cur.tile0, lane);
+                    });
+                    if (lane == 0) sm.excl = e;
+                }
+                __syncthreads();
+                wexcl += sm.excl;
+            }
         }
-        __syncthreads();
-        wave_base = geo.H + sm.excl + wexcl;
+        wave_base = geo.H + wexcl;
     }
     const uint8_t* const wbase = cmp + uniform64(wave_base);
     const bool intact = wave_base + wtot <= cur.limit;
@@ -1964,8 +2012,8 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     const T eb = (T)cur.param;
     const uint64_t gvalid = (DIM == 1) ? (geo.n + 63) / 64 : geo.nblocks;   // groups holding elements
     // chunks with elements of the array, and (1D) whole ones
-    const int nch = chunks_of<KC>(wgrp0, gvalid, G - 1);
-    const int nfull = (DIM == 1) ? chunks_of<KC>(wgrp0, geo.n / 64, 0) : nch;
+    const int nch = chunks_of(KC, wgrp0, gvalid, G - 1);
+    const int nfull = (DIM == 1) ? chunks_of(KC, wgrp0, geo.n / 64, 0) : nch;
     Walker wkc;   // 2D/3D: the chunk being stored
     if constexpr (DIM != 1) wkc.init(wgrp0, geo);
 
@@ -2131,23 +2179,20 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     // read a zero word). Loads with some lanes past the buffer range cost far
     // more memory-pipeline time than dense ones. Otherwise each lane loads its
     // own words from global memory.
-    uint32_t cs[KC + 1];   // chunk starts within the wave's payload (wave-uniform)
-#pragma unroll
-    for (int c = 0; c < KC; ++c) cs[c] = rdlane(excl0, c * LPC);
-    cs[KC] = wtot;
+    auto chunk_start = [&](int c) -> uint32_t { return c < KC ? rdlane(excl0, (uint32_t)(c * LPC)) : wtot; };   // in the wave's payload
     // Buffer loads check their range per dword, so the dwords holding the
     // payload's last bytes must lie inside it: an outlier stream whose length
     // is not a multiple of 4 ends inside a dword, and its last wave keeps the
     // per-lane loads (a truncated stream has an empty range: the same).
     const bool whole = ((wtot + 3u) & ~3u) <= (uint32_t)nrec;   // every payload dword inside the range
-    bool dense = whole;
-#pragma unroll
-    for (int c = 0; c < KC; ++c) dense &= cs[c + 1] - (cs[c] & ~3u) <= (uint32_t)kDenseBytes;
     // The wave's whole payload in one burst of loads before its first chunk,
     // where it fits the wave's buffer. A compute-free kernel with the 1D
     // decode's traffic (2^30 f32 written, 0.94 GB read) ran 2.5-4 % faster with
     // each wave's reads in one burst than with a read per chunk.
     const bool burst = whole && wtot <= (uint32_t)kWaveBuf;
+    bool dense = whole;
+    if (!burst)
+        for (int c = 0; c < KC; ++c) dense &= chunk_start(c + 1) - (chunk_start(c) & ~3u) <= (uint32_t)kDenseBytes;
     auto fetch_lds = [&](uint32_t origin) {
         return [=](uint32_t o) -> uint32_t {
             const lds_u8* const p = (int32_t)o < 0 ? zw : buf + (o - origin);
@@ -2182,8 +2227,7 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
         auto load_chunk = [&](int c, v4u (&P)[2]) {
             // from the chunk's aligned start; the second KiB only when needed
             // (else an offset past every range: no memory access)
-            const uint32_t a0 = rdlane(excl0, (uint32_t)(c * LPC)) & ~3u;
-            const uint32_t a1 = c + 1 < KC ? rdlane(excl0, (uint32_t)((c + 1) * LPC)) : wtot;
+            const uint32_t a0 = chunk_start(c) & ~3u, a1 = chunk_start(c + 1);
             P[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c < nch ? a0 + 16u * (uint32_t)lane : kAbsent, 0, 0);
             P[1] = __builtin_amdgcn_raw_buffer_load_b128(
                 rsrc, c < nch && a1 - a0 > 1024u ? a0 + 1024u + 16u * (uint32_t)lane : kAbsent, 0, 0);
@@ -2200,7 +2244,7 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
             ((lds_v4u*)buf)[64 + lane] = P[1];
             __builtin_amdgcn_wave_barrier();
             load_chunk(c + 1, P);
-            decode_chunk(c, fetch_lds(rdlane(excl0, (uint32_t)(c * LPC)) & ~3u), q);
+            decode_chunk(c, fetch_lds(chunk_start(c) & ~3u), q);
         }
     } else {
 #pragma unroll 1
@@ -2222,18 +2266,20 @@ __global__ void __launch_bounds__(WAVES * kWaveSize, kCompressWavesPerSimd)
 compress_kernel(const Item item, const ScanCtx sc, const uint64_t base) {
     __shared__ SmemC<WAVES> sm;
     // a compress tile's predecessors have mostly published by the time its
-    // payload is staged: the 128-tile window (2 words per lane) is enough
-    compress_tile<DIM, MODE, T, WAVES, RUNS>(item, base + blockIdx.x, sc, sm, 2);
+    // payload is staged: the 128-tile window (2 words per lane) is enough, or
+    // one window for all tiles of a short array
+    compress_tile<DIM, MODE, T, WAVES, RUNS>(item, base + blockIdx.x, sc, sm, item.geo.ntiles <= 64 * kLookbackWords ? kLookbackWords : 2);
 }
 
 // Waves take their payload offsets from `offs` (unit_offsets_kernel, launched
-// before on the same stream); sc is unused.
+// before on the same stream), or sum them up where it is null (arrays of at most
+// kDirectHeader header bytes); sc is unused.
 template <int DIM, int MODE, class T, int WAVES, bool RUNS>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kDecompressWavesPerSimd)
 decompress_kernel(const Item item, const ScanCtx sc, const unsigned long long* __restrict__ offs,
                   const uint64_t base) {
     __shared__ SmemD<WAVES> sm;
-    decompress_tile<DIM, MODE, T, WAVES, RUNS, true>(item, base + blockIdx.x, sc, sm, kLookbackWords, offs);
+    decompress_tile<DIM, MODE, T, WAVES, RUNS, true>(item, base + blockIdx.x, sc, sm, 0, offs);
 }
 
 // ---------------------------------------------------------------------------
@@ -2290,8 +2336,8 @@ decompress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx
     const uint64_t tile = base + blockIdx.x;
     const Item cur = src.get(src.locate(tile, 0));
 #define CUSZP_RUN_D(D, M, T)                                                            \
-    if (D == 1 || cur.geo.runs) decompress_tile<D, M, T, WAVES, true>(cur, tile, sc, sm, window); \
-    else decompress_tile<D, M, T, WAVES, D == 1>(cur, tile, sc, sm, window)
+    if (D == 1 || cur.geo.runs) decompress_tile<D, M, T, WAVES, true, false>(cur, tile, sc, sm, window); \
+    else decompress_tile<D, M, T, WAVES, D == 1, false>(cur, tile, sc, sm, window)
     switch (cur.variant) { CUSZP_BATCH_CASES(CUSZP_RUN_D) }
 #undef CUSZP_RUN_D
 }

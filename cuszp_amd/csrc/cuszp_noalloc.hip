@@ -90,11 +90,11 @@ extern "C" int cuSZp_compress_noalloc(const void* d_oriData, unsigned char* d_cm
     Geom g;
     int rc = make_geom(dim, nbEle, dims, g);
     if (rc) return rc;
-    TilePlan plan{4, 0};
+    TilePlan plan{4, 1, 0};
     if (nbEle) {
         if (!d_oriData || !d_cmpBytes) return CUSZP_ERROR_INVALID_ARGUMENT;
         if (max_stream_bytes(dim, g) > kMaxStream) return CUSZP_ERROR_TOO_LARGE;
-        plan = plan_tiles(dim, type, true, g);
+        plan = plan_tiles(dim, type, g);
         if (plan.ntiles > kNoAllocTiles) {
             std::fprintf(stderr,
                          "cuSZp_compress_noalloc: %zu values need %llu tiles; the fixed scratch holds %llu "
@@ -104,6 +104,7 @@ extern "C" int cuSZp_compress_noalloc(const void* d_oriData, unsigned char* d_cm
         }
         if (cmpCapacity < g.H) return CUSZP_ERROR_OUTPUT_TOO_SMALL;
         g.ntiles = plan.ntiles;
+        g.kc = plan.kc;
     }
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return CUSZP_ERROR_HIP;

@@ -9,20 +9,22 @@
 
 namespace cuszp {
 
-// Tile plan: waves per workgroup (4 or 8) and the number of tiles (tile
-// shape: tile_groups).
+// Tile plan: waves per workgroup (4 or 8), chunks per wave and the number of
+// tiles (tile shape: tile_groups).
 // CUSZP_WAVES in the environment overrides the choice (tuning experiments).
 struct TilePlan {
     int waves;
+    int kc;
     uint64_t ntiles;
 };
-TilePlan plan_tiles(int dim, int type, bool compress, const Geom& g);
+TilePlan plan_tiles(int dim, int type, const Geom& g);
 
 // Single-array launches; item.param is 0.5/eb (compress) or eb (decompress).
 hipError_t launch_compress_f32(int dim, int mode, int waves, const Item& item, const ScanCtx& sc, hipStream_t st);
 hipError_t launch_compress_f64(int dim, int mode, int waves, const Item& item, const ScanCtx& sc, hipStream_t st);
 // Single-array decompression reads each wave's payload offset from `offs`,
-// which launch_unit_offsets_* fills first on the same stream.
+// which launch_unit_offsets_* fills first on the same stream; a null `offs`
+// (headers of at most kDirectHeader bytes) has every workgroup sum them up.
 hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item, const ScanCtx& sc,
                                  const unsigned long long* offs, hipStream_t st);
 hipError_t launch_decompress_f64(int dim, int mode, int waves, const Item& item, const ScanCtx& sc,

@@ -59,6 +59,48 @@ def test_staging_area_overflows(device, oracle, dim, dtype):
             _check(oracle, x, 0.5, mode, dim, dims)
 
 
+def _batch(P, torch, direction, rows):
+    """rows: (in, out, values, capacity, bound, dim, dims, type, mode); the batch kernels' tiles are full ones."""
+    with P.BatchPlan([P.batch_item(*r) for r in rows], direction) as plan:
+        plan.execute()
+        sizes, _ = plan.results()
+    torch.cuda.synchronize()
+    return sizes
+
+
+# Values on both sides of each step of the tile shapes, of the longest header that a batch and a single call sum
+# without a pass over it (16 and 256 KiB), and a few in between.
+LINES = [(1, n + k) for n in (1, 2048, 65536, 524288, 1048576, 3145728, 6291456, 8388608) for k in (0, 1)]
+LINES += [(3, (128, 64, z)) for z in (64, 65, 128, 129, 384, 385)] + [(3, (256, 128, 197)), (3, (256, 256, 256)), (3, (256, 256, 257))]
+LINES += [(2, (1000, 1048, 1)), (2, (2048, 512, 1)), (2, (2044, 1537, 2)), (2, (4096, 4096, 1)), (2, (4096, 4097, 1))]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("line", LINES, ids=lambda s: f"{s[0]}D-{s[1]}")
+def test_tile_shapes(device, oracle, line, dtype):
+    import torch
+    from cuszp_amd import pycuSZp as P
+
+    dim, dims = line if line[0] > 1 else (1, (0, 0, 0))
+    n = line[1] if dim == 1 else dims[0] * dims[1] * dims[2]
+    r = np.random.default_rng(n)
+    x = np.cumsum(r.integers(-5, 6, n)).astype(dtype)
+    x[r.integers(0, n, n // 300 + 1)] += 5000
+    t, typ = torch.from_numpy(x).cuda(), int(dtype == np.float64)
+    for mode in (0, 1, 2):
+        cap = P.max_compressed_size(n, dim, dims, typ, mode)
+        one, two = torch.zeros(cap, dtype=torch.uint8, device="cuda"), torch.zeros(cap, dtype=torch.uint8, device="cuda")
+        size = P.compress_ex(t, one, cap, n, 0.5, dim, dims, typ, mode)
+        assert _batch(P, torch, P.BATCH_COMPRESS, [(t, two, n, cap, 0.5, dim, dims, typ, mode)]) == [size]
+        assert torch.equal(one, two)
+        if n <= 1 << 20:
+            assert one[:size].cpu().numpy().tobytes() == oracle.compress(x, 0.5, mode, dim, dims)
+        y, z = torch.full_like(t, float("nan")), torch.full_like(t, float("nan"))
+        P.decompress_ex(y, one, n, size, 0.5, dim, dims, typ, mode)
+        _batch(P, torch, P.BATCH_DECOMPRESS, [(one, z, n, size, 0.5, dim, dims, typ, mode)])
+        assert torch.equal(y, t) and torch.equal(z, t)   # the codes are the values
+
+
 @pytest.mark.parametrize("dim,dims,n", [(1, (0, 0, 0), 98304), (1, (0, 0, 0), 9 << 20), (3, (64, 64, 36), 147456), (2, (4096, 4104, 1), 4096 * 4104)])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_any_header_byte(device, oracle, dim, dims, n, mode):
