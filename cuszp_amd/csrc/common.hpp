@@ -61,14 +61,15 @@ inline hipError_t scan_state_alloc(unsigned long long** p, size_t bytes) {
 
 // Scan context of a launch over `status` (kStatusGuard guard words in front
 // are the caller's), with the launch's error word and the diagnostic words
-// diag[0..7].
+// diag[0..7]; `mark`: a pinned host word (Item::mark).
 inline ScanCtx make_scan_ctx(unsigned long long* status, unsigned int* err, unsigned long long* diag,
-                             unsigned long long tag) {
+                             unsigned long long tag, unsigned long long* mark = nullptr) {
     const ScanSettings& k = scan_settings();
     ScanCtx c;
     c.status = status;
     c.err = err;
     c.diag = diag;
+    c.mark = mark;
     c.tag = tag;
     c.steal_ticks = k.steal_ticks.load(std::memory_order_relaxed);
     c.hold_every = k.hold_every.load(std::memory_order_relaxed);
@@ -79,8 +80,7 @@ inline ScanCtx make_scan_ctx(unsigned long long* status, unsigned int* err, unsi
 }
 
 // Device words of a launch's scan state besides the status array:
-// [0] epoch (batched launches), [1] stream length (blocking entries),
-// [2] sticky bits, [4..7] watchdog diagnostics, [8..11] lookback counters.
+// [0] epoch (batched launches), [2] sticky bits, [4..7] watchdog diagnostics, [8..11] lookback counters.
 constexpr int kMiscWords = 16;
 constexpr int kMiscErr = 2, kMiscDiag = 4, kMiscCounters = 8;
 

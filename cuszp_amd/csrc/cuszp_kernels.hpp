@@ -109,6 +109,7 @@ struct ScanCtx {
     unsigned long long* diag;       // [0] first stalled tile + 1, [1] its missing predecessor, [2] word seen;
                                     // with `stats`: [4] polls that found a window unresolved, [5] lookbacks
                                     // that polled, [6] predecessors claimed, [7] clock ticks spent waiting
+    unsigned long long* mark;       // as Item::mark
     unsigned long long tag;         // epoch << kEpochShift
     uint32_t steal_ticks;           // wait (s_memrealtime ticks) before a pending predecessor is claimed
     uint32_t hold_every;            // scan stress: tile t with t % hold_every == hold_every - 1 waits
@@ -123,13 +124,23 @@ struct Item {
     void* dst;                      // compress: stream; decompress: values
     uint64_t limit;                 // compress: stream capacity; decompress: stream length
     unsigned long long* total;      // out: stream length, written by the last tile (may be null)
+    unsigned long long* host_total; // the same once more, in pinned host memory (may be null)
     unsigned int* err;              // sticky error bits of this array (kErrOverflow, kErrTruncated)
+    unsigned long long* mark;       // pinned host word set to 1 with every bit of an err word (may be null)
     double param;                   // compress: 0.5/eb, decompress: eb (exact in the array's type)
     uint64_t tile0;                 // first tile of the array in the launch (its scan segment start)
     uint32_t variant;               // type * 9 + (dim - 1) * 3 + mode
     uint32_t flags;                 // kItemStreamNt
     Geom geo;                       // geo.ntiles: tiles of this array
 };
+
+// Sets a bit of a sticky error word. The words stay in device memory, where all
+// workgroups meet; the mark tells the host, which would otherwise copy them back
+// after every call, that there is anything to read.
+__device__ __forceinline__ void raise_bit(unsigned int* err, uint32_t bit, unsigned long long* mark) {
+    atomicOr(err, bit);
+    if (mark) __hip_atomic_store(mark, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // ---------------------------------------------------------------------------
 // wave64 primitives
@@ -605,7 +616,7 @@ __device__ __forceinline__ uint64_t wave_lookback(const ScanCtx& sc, uint64_t ti
             const uint64_t a = agg_of((uint64_t)claimed);
             if (lane == 0) {
                 cas_status(sc.status + claimed, tag | kFlagClaim, tag | kFlagAgg | a);
-                atomicOr(sc.err, kInfoStolen);
+                raise_bit(sc.err, kInfoStolen, sc.mark);
                 if (sc.stats) atomicAdd(sc.diag + 6, 1ull);
             }
             claimed = -1;
@@ -658,7 +669,7 @@ __device__ __forceinline__ uint64_t wave_lookback(const ScanCtx& sc, uint64_t ti
                 // (the output is reported invalid; publishing below unblocks successors)
                 stalled = true;
                 if (lane == 0) {
-                    atomicOr(sc.err, kErrStall);
+                    raise_bit(sc.err, kErrStall, sc.mark);
                     if (atomicCAS(sc.diag, 0ull, tile + 1) == 0ull) {
                         sc.diag[1] = (uint64_t)pidx;
                         sc.diag[2] = pend;
@@ -1801,7 +1812,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     // ---- the tile's offset (wave 0) ---------------------------------------------
     if (lane == 0) {
         sm.wtot[wave] = wave_tot;
-        if (lossy) atomicOr(cur.err, kWarnLossy);
+        if (lossy) raise_bit(cur.err, kWarnLossy, cur.mark);
     }
     __syncthreads();
 #pragma unroll
@@ -1816,13 +1827,17 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
         });
         if (lane == 0) {
             sm.excl = e;
-            if (lt == geo.ntiles - 1 && cur.total) *cur.total = geo.H + e + ttot;
+            if (lt == geo.ntiles - 1) {
+                const unsigned long long bytes = geo.H + e + ttot;
+                if (cur.total) *cur.total = bytes;
+                if (cur.host_total) __hip_atomic_store(cur.host_total, bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
     }
     __syncthreads();
     excl = sm.excl;
     if (geo.H + excl + ttot > cur.limit) {   // never write past the caller's buffer
-        if (wave == 0 && lane == 0) atomicOr(cur.err, kErrOverflow);
+        if (wave == 0 && lane == 0) raise_bit(cur.err, kErrOverflow, cur.mark);
         return;
     }
     // ---- copy the staged payload: 16 bytes per lane, then the tail bytes ---------
@@ -1994,7 +2009,7 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     }
     const uint8_t* const wbase = cmp + uniform64(wave_base);
     const bool intact = wave_base + wtot <= cur.limit;
-    if (!intact && lane == 0) atomicOr(cur.err, kErrTruncated);
+    if (!intact && lane == 0) raise_bit(cur.err, kErrTruncated, cur.mark);
     // The wave's stream words go through a buffer resource over its payload:
     // 32-bit offsets, and an offset past the range (bit 31 set) reads 0, so
     // lanes without a word need no address select and no masking; a truncated
