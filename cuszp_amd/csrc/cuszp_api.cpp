@@ -261,8 +261,8 @@ int decompress_once(void* out, const unsigned char* cmp, size_t n, size_t cmp_si
                 : launch_unit_offsets_f32(dim, mode, item, nunits, s.d_offs, sc, st);
     if (e != hipSuccess) return CUSZP_ERROR_HIP;
     const unsigned long long* const offs = direct ? nullptr : s.d_offs;
-    e = f64 ? launch_decompress_f64(dim, mode, plan.waves, item, sc, offs, st)
-            : launch_decompress_f32(dim, mode, plan.waves, item, sc, offs, st);
+    e = f64 ? launch_decompress_f64(dim, mode, plan.waves, item, offs, st)
+            : launch_decompress_f32(dim, mode, plan.waves, item, offs, st);
     if (e != hipSuccess) return CUSZP_ERROR_HIP;
     if (!blocking) return CUSZP_SUCCESS;
     return finish_blocking(s, st, nullptr);

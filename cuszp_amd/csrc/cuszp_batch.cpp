@@ -5,9 +5,9 @@
 // A plan validates every array once (the same checks as cuSZp_compress_ex /
 // cuSZp_decompress_ex), lays the arrays' tiles end to end, uploads one Item
 // descriptor per non-empty array and owns the scan state: tile status words,
-// an epoch word bumped on the device before each launch (so replays of a
-// captured graph never see the previous run's status words as current), a
-// launch-wide error word and one error word and one stream length per array.
+// an epoch word bumped on the device for each launch (so replays of a captured
+// graph never see the previous run's status words as current), the offset table
+// of a decompression, a launch-wide error word and one error word and one stream length per array.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,15 +26,20 @@ struct cuszp_batch_plan_s {
     int dev = 0;
     int dir = CUSZP_BATCH_COMPRESS;
     int flags = 0;
-    int waves = 4;
-    int window = kLookbackWords;   // lookback words per lane (2 or 4)
+    // launch shape (choose_shape, or the tuner's): waves per workgroup, chunks per
+    // wave at most (a type's own limit holds), lookback words per lane (2 or 4)
+    int waves = 8, kc = kChunksOf<float>, window = kLookbackWords;
+    bool pass = false;             // decompress: some header is too long for the tiles to sum up
     std::vector<cuszp_batch_item_t> src;
     std::vector<Item> items;      // non-empty arrays, in caller order
     uint64_t ntiles = 0;
+    uint64_t nseg = 0;            // decompress: segments of the offset pass, 0 without it
     Item* d_items = nullptr;
     size_t cap_items = 0;
     unsigned long long* d_status = nullptr;
-    uint64_t cap_tiles = 0;
+    uint64_t cap_status = 0;
+    unsigned long long* d_offs = nullptr;   // decompress: payload offset of every decode wave
+    uint64_t cap_offs = 0;
     unsigned long long* d_misc = nullptr;   // kMiscWords: [0] epoch, [2] launch bits, [4..7] diagnostics, [8..11] counters
     unsigned int* d_err = nullptr;          // per array
     unsigned long long* d_sizes = nullptr;  // per array (compress)
@@ -65,19 +70,48 @@ int check_item(const cuszp_batch_item_t& it, int dir, Geom& g) {
     return CUSZP_SUCCESS;
 }
 
-// Lay out the tiles of every non-empty array for `waves` waves per workgroup
-// and upload the descriptors (grows device buffers as needed).
+int chunks(const cuszp_batch_item_t& s, int kc) {
+    return std::min(kc, s.type == CUSZP_TYPE_DOUBLE ? kChunksOf<double> : kChunksOf<float>);
+}
+uint64_t tiles(const cuszp_batch_item_t& s, const Geom& g, int waves, int kc) {
+    const uint64_t groups = (s.dim == CUSZP_DIM_1D) ? g.H / 2 : g.nblocks;
+    const uint64_t per_tile = tile_groups(s.type == CUSZP_TYPE_DOUBLE, waves, chunks(s, kc));
+    return (groups + per_tile - 1) / per_tile;
+}
+
+// The shape of a plan that is not tuned: as a single array's (plan_tiles), with
+// the tiles of all arrays together, and at least 4 chunks per wave under an
+// offset pass (a thread of the pass takes 32 header bytes). 256 arrays of 1 Ki to
+// 16 Mi values, 2.2 GB: 4 waves 522 / 429 us (compress / decompress), 8 waves
+// 471 / 417; 16 arrays of up to 256 Ki values, 30 / 27 us with full waves, 22 / 19
+// with the rule's (4, 2).
+void choose_shape(cuszp_batch_plan_s& p) {
+    typedef std::vector<std::pair<int, int>> Ladder;   // (waves, chunks)
+    for (const auto& shape : p.pass ? Ladder{{4, 4}, {8, 4}, {8, 8}} : Ladder{{4, 1}, {4, 2}, {8, 2}, {8, 4}, {8, 8}}) {
+        p.waves = shape.first;
+        p.kc = shape.second;
+        uint64_t n = 0;
+        for (const cuszp_batch_item_t& s : p.src) {
+            Geom g;
+            make_geom(s.dim, s.nbEle, s.dims, g);
+            if (s.nbEle) n += tiles(s, g, p.waves, p.kc);
+        }
+        if (n <= (p.waves == 4 ? 256u : 384u)) return;
+    }
+}
+
+// Lay out the tiles of every non-empty array for the plan's shape and upload the
+// descriptors (grows device buffers as needed).
 int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
     p.items.clear();
-    uint64_t tile0 = 0;
+    uint64_t tile0 = 0, seg0 = 0;
     for (size_t i = 0; i < p.src.size(); ++i) {
         const cuszp_batch_item_t& s = p.src[i];
         if (s.nbEle == 0) continue;
         Geom g;
         make_geom(s.dim, s.nbEle, s.dims, g);
-        const uint64_t groups = (s.dim == CUSZP_DIM_1D) ? g.H / 2 : g.nblocks;
-        const uint64_t per_tile = tile_groups(s.type == CUSZP_TYPE_DOUBLE, p.waves);
-        g.ntiles = (groups + per_tile - 1) / per_tile;
+        g.kc = chunks(s, p.kc);
+        g.ntiles = tiles(s, g, p.waves, p.kc);
         const bool c = p.dir == CUSZP_BATCH_COMPRESS;
         Item it = make_item(s.d_in, s.d_out, s.capacity, c ? p.d_sizes + i : nullptr, p.d_err + i,
                             c ? compress_param(s.errorBound, s.type) : decompress_param(s.errorBound, s.type),
@@ -86,9 +120,12 @@ int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
         if (c) it.host_total = p.h_res + 1 + i;
         it.tile0 = tile0;
         tile0 += g.ntiles;
+        it.seg0 = seg0;
+        seg0 += batch_segments(s.dim, s.type == CUSZP_TYPE_DOUBLE, (int)g.kc, g.ntiles * (uint64_t)p.waves);
         p.items.push_back(it);
     }
     p.ntiles = tile0;
+    p.nseg = p.pass ? seg0 : 0;
     // Growing a buffer: the old one is released before the new one is
     // allocated, and the capacity drops to 0 in between, so a failed
     // allocation leaves no buffer that a later call would take as large enough
@@ -101,19 +138,29 @@ int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
         BATCH_HIP(hipMalloc((void**)&p.d_items, p.items.size() * sizeof(Item)));
         p.cap_items = p.items.size();
     }
-    const uint64_t need = p.ntiles ? p.ntiles : 1;   // an empty table still gets a (cleared) status array
-    if (need > p.cap_tiles) {
+    const uint64_t words = p.dir == CUSZP_BATCH_COMPRESS ? p.ntiles : p.nseg;
+    const uint64_t need = words ? words : 1;   // an empty table still gets a (cleared) status array
+    if (need > p.cap_status) {
         if (p.d_status) BATCH_HIP(hipFree(p.d_status));
         p.d_status = nullptr;
-        p.cap_tiles = 0;
+        p.cap_status = 0;
         // kStatusGuard words in front (lookback windows of first tiles read there)
         BATCH_HIP(scan_state_alloc(&p.d_status, (kStatusGuard + need) * sizeof(unsigned long long)));
-        p.cap_tiles = need;
+        p.cap_status = need;
+    }
+    const uint64_t units = p.nseg ? p.ntiles * (uint64_t)p.waves : 0;
+    if (units > p.cap_offs) {
+        if (p.d_offs) BATCH_HIP(hipFree(p.d_offs));
+        p.d_offs = nullptr;
+        p.cap_offs = 0;
+        BATCH_HIP(scan_state_alloc(&p.d_offs, units * sizeof(unsigned long long)));
+        p.cap_offs = units;
     }
     // stale status words must not carry the current epoch: start from zero and
     // restart the epoch whenever the table changes
-    BATCH_HIP(hipMemsetAsync(p.d_status, 0, (kStatusGuard + p.cap_tiles) * sizeof(unsigned long long), st));
+    BATCH_HIP(hipMemsetAsync(p.d_status, 0, (kStatusGuard + p.cap_status) * sizeof(unsigned long long), st));
     BATCH_HIP(hipMemsetAsync(p.d_misc, 0, sizeof(unsigned long long), st));
+    if (p.nseg) BATCH_HIP(launch_bump_epoch(p.d_misc, st));   // the next pass's; then the decompress kernel advances it
     if (!p.items.empty())
         BATCH_HIP(hipMemcpyAsync(p.d_items, p.items.data(), p.items.size() * sizeof(Item), hipMemcpyHostToDevice, st));
     BATCH_HIP(hipStreamSynchronize(st));   // the host table may be rebuilt right after
@@ -125,12 +172,15 @@ int enqueue(const cuszp_batch_plan_s& p, hipStream_t st) {
     // the kernels read the epoch word for the tag
     const ScanCtx sc = make_scan_ctx(p.d_status + kStatusGuard, (unsigned int*)(p.d_misc + kMiscErr),
                                      p.d_misc + kMiscDiag, 0, p.h_res);
-    BATCH_HIP(launch_bump_epoch(p.d_misc, st));
     const uint32_t n = (uint32_t)p.items.size();
-    if (p.dir == CUSZP_BATCH_COMPRESS)
+    if (p.dir == CUSZP_BATCH_COMPRESS) {
+        BATCH_HIP(launch_bump_epoch(p.d_misc, st));
         BATCH_HIP(launch_compress_batch(p.waves, p.window, p.d_items, n, p.ntiles, sc, p.d_misc, st));
-    else
-        BATCH_HIP(launch_decompress_batch(p.waves, p.window, p.d_items, n, p.ntiles, sc, p.d_misc, st));
+        return CUSZP_SUCCESS;
+    }
+    if (p.nseg) BATCH_HIP(launch_offsets_batch(p.waves, p.d_items, n, p.nseg, p.d_offs, sc, p.d_misc, st));
+    BATCH_HIP(launch_decompress_batch(p.waves, p.d_items, n, p.ntiles, p.nseg ? p.d_offs : nullptr,
+                                      p.nseg ? p.d_misc : nullptr, st));
     return CUSZP_SUCCESS;
 }
 
@@ -162,7 +212,7 @@ int capture(cuszp_batch_plan_s& p) {
 // (log2 of its tile count and of its array count); later plans of the same
 // class start from the recorded shape.
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int>, std::pair<int, int>> g_tuned;   // -> (waves per workgroup, lookback window)
+std::map<std::tuple<int, int, int>, std::tuple<int, int, int>> g_tuned;   // -> (waves per workgroup, chunks per wave, lookback window)
 
 std::tuple<int, int, int> size_class(const cuszp_batch_plan_s& p) {
     uint64_t bytes = 0;
@@ -198,12 +248,18 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
     p->src.assign(items, items + count);
     int rc = CUSZP_SUCCESS;
     if (hipGetDevice(&p->dev) != hipSuccess) rc = CUSZP_ERROR_HIP;
+    for (const cuszp_batch_item_t& it : p->src) {
+        Geom g;
+        make_geom(it.dim, it.nbEle, it.dims, g);
+        p->pass |= direction == CUSZP_BATCH_DECOMPRESS && g.H > kBatchDirectHeader;
+    }
+    choose_shape(*p);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto f = g_tuned.find(size_class(*p));
         if (f != g_tuned.end()) {
-            p->waves = f->second.first;
-            p->window = f->second.second;
+            std::tie(p->waves, p->kc, p->window) = f->second;
+            if (p->pass) p->kc = std::max(p->kc, 4);
         }
     }
     if (!rc && hipMalloc((void**)&p->d_misc, kMiscWords * sizeof(unsigned long long)) != hipSuccess) rc = CUSZP_ERROR_HIP;
@@ -304,16 +360,21 @@ int cuSZp_batch_plan_scan_report(cuszp_batch_plan_t p, hipStream_t stream, cuszp
 int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_out, unsigned* grid_out) {
     if (!p) return CUSZP_ERROR_INVALID_ARGUMENT;
     if (p->items.empty()) return CUSZP_SUCCESS;
-    const int kShapes[4][2] = {{4, 4}, {8, 4}, {4, 2}, {8, 2}};   // (waves, lookback window)
+    // (waves, chunks, window): the rule's shape, then full waves; decompress tiles do not look back
+    std::vector<std::tuple<int, int, int>> shapes;
+    choose_shape(*p);
+    shapes.emplace_back(p->waves, p->kc, kLookbackWords);
+    for (int window : {kLookbackWords, 2})
+        for (int waves : {4, 8})
+            if (window == kLookbackWords || p->dir == CUSZP_BATCH_COMPRESS) shapes.emplace_back(waves, kChunksOf<float>, window);
     hipEvent_t e0, e1;
     BATCH_HIP(hipEventCreate(&e0));
     BATCH_HIP(hipEventCreate(&e1));
     float best = 1e30f;
-    int best_w = p->waves, best_k = p->window;
+    std::tuple<int, int, int> best_shape = shapes[0];
     int rc = CUSZP_SUCCESS;
-    for (const auto& shape : kShapes) {
-        p->waves = shape[0];
-        p->window = shape[1];
+    for (const auto& shape : shapes) {
+        std::tie(p->waves, p->kc, p->window) = shape;
         rc = build_table(*p, stream);
         if (rc) break;
         rc = enqueue(*p, stream);   // warm-up
@@ -329,20 +390,18 @@ int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_o
         hipEventElapsedTime(&ms, e0, e1);
         if (ms < best) {
             best = ms;
-            best_w = shape[0];
-            best_k = shape[1];
+            best_shape = shape;
         }
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     if (rc) return rc;
-    p->waves = best_w;
-    p->window = best_k;
+    std::tie(p->waves, p->kc, p->window) = best_shape;
     rc = build_table(*p, stream);
     if (rc) return rc;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tuned[size_class(*p)] = {best_w, best_k};
+        g_tuned[size_class(*p)] = best_shape;
     }
     if (p->exec || (p->flags & CUSZP_BATCH_GRAPH)) rc = capture(*p);
     // tuning runs leave per-array state from the candidate launches: clear it
@@ -351,7 +410,7 @@ int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_o
     if (!rc && hipMemsetAsync(p->d_misc + kMiscErr, 0, (kMiscWords - kMiscErr) * sizeof(unsigned long long),
                               stream) != hipSuccess)
         rc = CUSZP_ERROR_HIP;
-    if (waves_out) *waves_out = best_w;
+    if (waves_out) *waves_out = p->waves;
     if (grid_out) *grid_out = (unsigned)(p->ntiles < kMaxGrid ? p->ntiles : kMaxGrid);
     return rc;
 }
@@ -366,6 +425,7 @@ void cuSZp_batch_plan_destroy(cuszp_batch_plan_t p) {
     hipDeviceSynchronize();   // no launch of this plan may still use its buffers
     if (p->d_items) hipFree(p->d_items);
     if (p->d_status) hipFree(p->d_status);
+    if (p->d_offs) hipFree(p->d_offs);
     if (p->d_misc) hipFree(p->d_misc);
     if (p->d_err) hipFree(p->d_err);
     if (p->d_sizes) hipFree(p->d_sizes);

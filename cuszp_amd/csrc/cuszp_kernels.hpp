@@ -10,8 +10,8 @@
 //     blocks in 1D, one 8x8 (2D) or 4x4x4 (3D) block otherwise. A "chunk" is 8
 //     groups, 512 elements: a wave holds one, a lane two quads of four
 //     consecutive elements (QuadLane);
-//   * a workgroup is WAVES waves and handles one tile: each wave owns KC
-//     chunks. The grid has one workgroup per tile (tile = launch base +
+//   * a workgroup is WAVES waves and handles one tile: each wave owns
+//     Geom::kc chunks. The grid has one workgroup per tile (tile = launch base +
 //     blockIdx.x). No ticket atomics: one hot device-scope atomic serialises at
 //     about 12 ns per operation on MI355X;
 //   * sign and magnitude bits travel as byte slices of a quad, as many as the
@@ -21,7 +21,8 @@
 //   * a block's rate is the bit length of its largest residual; every lane
 //     keeps its own block's books in compression, and in decompression one lane
 //     per block, once per wave;
-//   * the inter-tile exclusive scan of compressed bytes is a single-pass
+//   * the inter-tile exclusive scan of compressed bytes (compress tiles, and the
+//     pass over a long header that precedes decompression) is a single-pass
 //     decoupled lookback: one 64-bit status word per tile packs
 //     {epoch, flag, value}, is read 128 or 256 predecessors at a time by one
 //     wave, and
@@ -129,6 +130,7 @@ struct Item {
     unsigned long long* mark;       // pinned host word set to 1 with every bit of an err word (may be null)
     double param;                   // compress: 0.5/eb, decompress: eb (exact in the array's type)
     uint64_t tile0;                 // first tile of the array in the launch (its scan segment start)
+    uint64_t seg0;                  // batched decompress: its first segment in the launch's offset pass
     uint32_t variant;               // type * 9 + (dim - 1) * 3 + mode
     uint32_t flags;                 // kItemStreamNt
     Geom geo;                       // geo.ntiles: tiles of this array
@@ -1120,12 +1122,13 @@ struct ChunkQuads {
 struct ItemTable {
     const Item* items;
     uint32_t count;
-    // last item whose tile0 <= tile, searching from `from` (tiles only move forward)
-    __device__ __forceinline__ uint32_t locate(uint64_t tile, uint32_t from) const {
-        uint32_t lo = from, hi = count;   // answer in [lo, hi)
+    // last item whose first tile (or segment: FIRST) is not past `tile`
+    template <uint64_t Item::*FIRST = &Item::tile0>
+    __device__ __forceinline__ uint32_t locate(uint64_t tile) const {
+        uint32_t lo = 0, hi = count;   // answer in [lo, hi)
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
-            if (items[mid].tile0 <= tile) lo = mid;
+            if (items[mid].*FIRST <= tile) lo = mid;
             else hi = mid;
         }
         return lo;
@@ -1219,14 +1222,14 @@ struct HeaderSum {
     }
     __device__ __forceinline__ uint32_t bytes() const { return S * (r + n) + p; }
 };
-// This lane's share of the bytes that the header bytes [b0, b1) describe; both
-// are multiples of 16, lanes i of n take every n-th 16 bytes.
+// This lane's share of the bytes that the first b1 header bytes (a multiple of
+// 16) describe; lanes i of n take every n-th 16 bytes.
 template <int MODE, int S>
-__device__ __forceinline__ uint32_t header_share(const uint8_t* __restrict__ cmp, uint64_t b0, uint64_t b1, uint32_t i, uint32_t n) {
+__device__ __forceinline__ uint32_t header_share(const uint8_t* __restrict__ cmp, uint64_t b1, uint32_t i, uint32_t n) {
     typedef uint32_t v4uu __attribute__((ext_vector_type(4), aligned(1)));
     constexpr int U = 4;   // loads in flight
     HeaderSum<MODE, S> h;
-    for (uint64_t b = b0 + 16 * (uint64_t)i; b < b1; b += 16 * U * (uint64_t)n) {
+    for (uint64_t b = 16 * (uint64_t)i; b < b1; b += 16 * U * (uint64_t)n) {
         v4uu w[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -1240,20 +1243,6 @@ __device__ __forceinline__ uint32_t header_share(const uint8_t* __restrict__ cmp
             for (int k = 0; k < 4; ++k) h.add(w[u][k]);
     }
     return h.bytes();
-}
-
-// Payload bytes of local tile `lt` of a decompress item, from its header bytes.
-template <int DIM, int MODE, int WAVES>
-__device__ uint64_t header_tile_bytes(const uint8_t* __restrict__ cmp, const Geom& geo, uint64_t lt, int lane) {
-    constexpr int S = (DIM == 1) ? 4 : 8;
-    const uint32_t bpt = WAVES * geo.kc * (kChunkElems / 64) * ((DIM == 1) ? 2 : 1);   // blocks per tile
-    const uint64_t limit = (DIM == 1) ? geo.H : geo.nblocks;
-    uint64_t sum = 0;
-    for (uint32_t j = (uint32_t)lane; j < bpt; j += kWaveSize) {
-        const uint64_t b = lt * bpt + j;
-        sum += view_of<MODE, S>(b < limit ? (uint32_t)cmp[b] : 0u).size;
-    }
-    return wave_sum_u40(sum);
 }
 
 // Lookback window of a tile: 64 * kLookbackWords predecessors per round trip.
@@ -1375,6 +1364,40 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
     }
 }
 
+// The pass for a batch: one wave per segment of kBatchSegBytes header bytes, each
+// array's segments a scan of their own; offs[w] for wave w of the launch's tiles.
+// Without it the decode tiles looked back themselves, between their header and
+// payload reads, and those waits set the pace: 256 arrays of 1 Ki to 16 Mi values,
+// 2.2 GB, 694 us a call with tiles looking back, 488 with this pass (20 us of it).
+constexpr uint64_t kBatchSegBytes = kWaveSize * kPrefixBytes;
+template <int WAVES>
+__global__ void __launch_bounds__(kWaveSize)
+unit_offsets_batch_kernel(const Item* __restrict__ items, uint32_t nitems,
+                          unsigned long long* __restrict__ offs, ScanCtx sc,
+                          const unsigned long long* __restrict__ epoch, const uint64_t base) {
+    sc.tag = (epoch[0] & kEpochMask) << kEpochShift;
+    const ItemTable src{items, nitems};
+    const uint64_t seg = base + blockIdx.x;
+    const Item cur = src.get(src.locate<&Item::seg0>(seg));
+    const int lane = (int)__lane_id();
+    const uint8_t* const cmp = (const uint8_t*)cur.src;
+    const bool one_d = cur.variant % 9 < 3, outlier = cur.variant % 3 == kOutlier;
+    const uint64_t limit = one_d ? cur.geo.H : cur.geo.nblocks;
+    auto bytes = [&](uint64_t s) -> uint32_t {   // of this lane's header bytes of segment s
+        const uint64_t b0 = (s - cur.seg0) * kBatchSegBytes + (uint64_t)lane * kPrefixBytes;
+        if (one_d) return outlier ? thread_bytes<kOutlier, 4>(cmp, b0, limit) : thread_bytes<kPlain, 4>(cmp, b0, limit);
+        return outlier ? thread_bytes<kOutlier, 8>(cmp, b0, limit) : thread_bytes<kPlain, 8>(cmp, b0, limit);
+    };
+    const uint32_t tot = bytes(seg);
+    const uint32_t incl = scan_wave(tot);   // < 2^32: a segment holds 2^11 blocks of <= 2 KiB
+    const uint64_t e = wave_lookback<kLookbackWords>(sc, seg, cur.seg0, rdlane(incl, kWaveSize - 1), lane,
+                                                     [&](uint64_t p) { return wave_sum_u40(bytes(p)); });
+    const uint32_t per = cur.geo.kc * (kChunkElems / (one_d ? 32 : 64)) / kPrefixBytes;   // lanes per unit
+    const uint64_t th = (seg - cur.seg0) * kWaveSize + (uint64_t)lane;
+    if (th % per == 0 && th / per < cur.geo.ntiles * WAVES)
+        offs[cur.tile0 * WAVES + th / per] = cur.geo.H + e + (incl - tot);
+}
+
 // ---------------------------------------------------------------------------
 // one tile per workgroup pass
 // ---------------------------------------------------------------------------
@@ -1445,7 +1468,6 @@ constexpr int kMetaPerWave = 128;
 template <int WAVES>
 struct SmemD {
     uint64_t wtot[WAVES];             // per-wave byte counts
-    uint64_t excl;                    // the tile's exclusive prefix (wave 0's lookback)
     uint32_t before[WAVES];           // per-wave shares of the payload before the tile
     DMeta meta[WAVES][kMetaPerWave];  // per-block metadata of the wave's blocks
     uint4 payload[WAVES][kWaveBuf / 16];  // stream words, loaded densely and read per lane: the wave's or one chunk's
@@ -1896,8 +1918,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
 //   1. each wave reads the header bytes of its blocks (one or two per lane),
 //      scans their sizes once and writes every block's metadata (offset within
 //      the wave's payload, planes) to LDS;
-//   2. the wave's payload offset: from the offset table (OFFS), else the wave
-//      totals combine in LDS and wave 0 runs the lookback;
+//   2. the wave's payload offset;
 //   3. each wave works through its chunks: every lane reads the plane words of
 //      its lane number from the payload (one per set and byte slice; as many
 //      slices as the chunk's largest rate needs), transposes them back to its
@@ -1905,18 +1926,14 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
 //      the quad, one scan of DPP adds across the block's lanes) and stores
 //      (T)q * eb * 2.
 //
-// The wave's payload offset is the sum of the block sizes before it:
-//   * SINGLE (single-array launches) with an offset table `offs`
-//     (unit_offsets_kernel): read from there; no lookback and no workgroup
-//     barrier, every wave runs on its own;
-//   * SINGLE without, and arrays of a batch with short headers: the workgroup
-//     sums the header bytes in front of its tile itself (a read that hits in
-//     cache, and no pass and no waiting for other tiles);
-//   * else: the tile lookback.
-template <int DIM, int MODE, class T, int WAVES, bool RUNS, bool SINGLE>
-__device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t tile, const ScanCtx& sc,
-                                                SmemD<WAVES>& sm, const int window,
-                                                const unsigned long long* __restrict__ offs = nullptr) {
+// The wave's payload offset is the sum of the block sizes before it: with an
+// offset table `offs` (unit_offsets_kernel, unit_offsets_batch_kernel) the entry
+// of the launch's wave, and every wave runs on its own, without a barrier; else
+// (short headers) the workgroup sums the header bytes in front of its tile
+// itself: a read that hits in cache, and no pass.
+template <int DIM, int MODE, class T, int WAVES, bool RUNS>
+__device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t tile, SmemD<WAVES>& sm,
+                                                const unsigned long long* __restrict__ offs) {
     typedef QuadLane<DIM> QL;
     constexpr int G = kChunkElems / 64;
     constexpr int S = (DIM == 1) ? 4 : 8;
@@ -1969,43 +1986,22 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     const uint64_t over31 = (MODE == kOutlier) ? 0ull : ballot(rmax > 31);
 
     uint64_t wave_base;
-    if (SINGLE && offs) {
-        wave_base = uniform64(offs[lt * WAVES + (uint64_t)wave]);
+    if (offs) {
+        wave_base = uniform64(offs[tile * WAVES + (uint64_t)wave]);
         __builtin_amdgcn_wave_barrier();   // the metadata in LDS is this wave's own
     } else {
-        const bool direct = SINGLE || geo.H <= kBatchDirectHeader;
-        if (direct) {   // the header bytes in front of the tile: a multiple of 16
-            const uint64_t before = lt * WAVES * (uint64_t)NBW;
-            const uint32_t share = header_share<MODE, S>(cmp, 0, before, threadIdx.x, WAVES * kWaveSize);
-            const uint32_t sum = rdlane(scan_wave(share), kWaveSize - 1);   // < 2^32: at most kDirectHeader blocks
-            if (lane == 0) sm.before[wave] = sum;
+        const uint64_t before = lt * WAVES * (uint64_t)NBW;   // header bytes in front of the tile: a multiple of 16
+        const uint32_t share = header_share<MODE, S>(cmp, before, threadIdx.x, WAVES * kWaveSize);
+        const uint32_t sum = rdlane(scan_wave(share), kWaveSize - 1);   // < 2^32: at most kDirectHeader blocks
+        if (lane == 0) {
+            sm.wtot[wave] = wtot;
+            sm.before[wave] = sum;
         }
-        if (lane == 0) sm.wtot[wave] = wtot;
         __syncthreads();
-        uint64_t wexcl = 0, ttot = 0;
+        uint64_t wexcl = 0;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const uint64_t t = sm.wtot[w];
-            wexcl += (w < wave) ? t : 0;
-            ttot += t;
-            if (direct) wexcl += sm.before[w];
-        }
-        // wave-uniform: kept in scalar registers across the lookback
-        wexcl = uniform64(wexcl);
-        ttot = uniform64(ttot);
-        if constexpr (!SINGLE) {
-            if (!direct) {
-                if (wave == 0) {
-                    const uint64_t e = lookback(sc, tile, cur.tile0, ttot, lane, window, [&](uint64_t p) {
-                        return header_tile_bytes<DIM, MODE, WAVES>(cmp, geo, p - cur.tile0, lane);
-                    });
-                    if (lane == 0) sm.excl = e;
-                }
-                __syncthreads();
-                wexcl += sm.excl;
-            }
-        }
-        wave_base = geo.H + wexcl;
+        for (int w = 0; w < WAVES; ++w) wexcl += sm.before[w] + ((w < wave) ? (uint64_t)sm.wtot[w] : 0);
+        wave_base = geo.H + uniform64(wexcl);
     }
     const uint8_t* const wbase = cmp + uniform64(wave_base);
     const bool intact = wave_base + wtot <= cur.limit;
@@ -2288,21 +2284,20 @@ compress_kernel(const Item item, const ScanCtx sc, const uint64_t base) {
 
 // Waves take their payload offsets from `offs` (unit_offsets_kernel, launched
 // before on the same stream), or sum them up where it is null (arrays of at most
-// kDirectHeader header bytes); sc is unused.
+// kDirectHeader header bytes).
 template <int DIM, int MODE, class T, int WAVES, bool RUNS>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kDecompressWavesPerSimd)
-decompress_kernel(const Item item, const ScanCtx sc, const unsigned long long* __restrict__ offs,
-                  const uint64_t base) {
+decompress_kernel(const Item item, const unsigned long long* __restrict__ offs, const uint64_t base) {
     __shared__ SmemD<WAVES> sm;
-    decompress_tile<DIM, MODE, T, WAVES, RUNS, true>(item, base + blockIdx.x, sc, sm, 0, offs);
+    decompress_tile<DIM, MODE, T, WAVES, RUNS>(item, base + blockIdx.x, sm, offs);
 }
 
 // ---------------------------------------------------------------------------
 // batched kernels: the arrays of a table, of any variant, in one launch with
 // one workgroup per tile of the concatenated tile space. A tile's array is
-// found by binary search on tile0, and each array's tiles form their own
-// lookback segment, so every array's stream is exactly its single-array
-// stream.
+// found by binary search on tile0, and each array's tiles (compress) or header
+// segments (decompress) form a lookback segment of their own, so every array's
+// stream is exactly its single-array stream.
 // ---------------------------------------------------------------------------
 #define CUSZP_BATCH_CASES(RUN)                                                        \
     case 0: RUN(1, kFixed, float); break;                                             \
@@ -2333,7 +2328,7 @@ compress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx s
     sc.tag = (epoch[0] & kEpochMask) << kEpochShift;
     const ItemTable src{items, nitems};
     const uint64_t tile = base + blockIdx.x;
-    const Item cur = src.get(src.locate(tile, 0));
+    const Item cur = src.get(src.locate(tile));
 #define CUSZP_RUN_C(D, M, T)                                                          \
     if (D == 1 || cur.geo.runs) compress_tile<D, M, T, WAVES, true>(cur, tile, sc, sm, window); \
     else compress_tile<D, M, T, WAVES, D == 1>(cur, tile, sc, sm, window)
@@ -2343,16 +2338,17 @@ compress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx s
 
 template <int WAVES>
 __global__ void __launch_bounds__(WAVES * kWaveSize, kDecompressWavesPerSimd)
-decompress_batch_kernel(const Item* __restrict__ items, uint32_t nitems, ScanCtx sc,
-                        const unsigned long long* __restrict__ epoch, const int window, const uint64_t base) {
+decompress_batch_kernel(const Item* __restrict__ items, uint32_t nitems,
+                        const unsigned long long* __restrict__ offs, unsigned long long* bump, const uint64_t base) {
     __shared__ SmemD<WAVES> sm;
-    sc.tag = (epoch[0] & kEpochMask) << kEpochShift;
+    // the pass that read this epoch has finished: no kernel of its own for that (2 us and a gap)
+    if (bump && base + blockIdx.x == 0 && threadIdx.x == 0) *bump += 1;
     const ItemTable src{items, nitems};
     const uint64_t tile = base + blockIdx.x;
-    const Item cur = src.get(src.locate(tile, 0));
+    const Item cur = src.get(src.locate(tile));
 #define CUSZP_RUN_D(D, M, T)                                                            \
-    if (D == 1 || cur.geo.runs) decompress_tile<D, M, T, WAVES, true, false>(cur, tile, sc, sm, window); \
-    else decompress_tile<D, M, T, WAVES, D == 1, false>(cur, tile, sc, sm, window)
+    if (D == 1 || cur.geo.runs) decompress_tile<D, M, T, WAVES, true>(cur, tile, sm, offs); \
+    else decompress_tile<D, M, T, WAVES, D == 1>(cur, tile, sm, offs)
     switch (cur.variant) { CUSZP_BATCH_CASES(CUSZP_RUN_D) }
 #undef CUSZP_RUN_D
 }

@@ -53,7 +53,8 @@ struct Lane {
     Item* d_items = nullptr;
     Item* h_items = nullptr;   // pinned staging of the table
     unsigned long long* d_status = nullptr;
-    uint64_t cap_tiles = 0;
+    unsigned long long* d_offs = nullptr;   // decompress: payload offset of every decode wave
+    uint64_t cap_tiles = 0;                 // tiles that both arrays have room for
     uint64_t launches = 0;
     unsigned long long* d_misc = nullptr;   // kMiscWords: [0] epoch, [2] launch bits, [4..7] diagnostics
     unsigned int* d_err = nullptr;
@@ -151,6 +152,7 @@ int lane_init(Lane& L, size_t max_batch, uint64_t tiles) {
     SRV_HIP(hipHostMalloc((void**)&L.h_sizes, max_batch * sizeof(unsigned long long), hipHostMallocDefault));
     SRV_HIP(hipHostMalloc((void**)&L.h_misc, kMiscWords * sizeof(unsigned long long), hipHostMallocDefault));
     SRV_HIP(hipMalloc((void**)&L.d_status, (kStatusGuard + tiles) * sizeof(unsigned long long)));
+    SRV_HIP(hipMalloc((void**)&L.d_offs, tiles * kServeWaves * sizeof(unsigned long long)));
     L.cap_tiles = tiles;
     SRV_HIP(hipMemsetAsync(L.d_status, 0, (kStatusGuard + tiles) * sizeof(unsigned long long), L.st));
     SRV_HIP(hipMemsetAsync(L.d_misc, 0, kMiscWords * sizeof(unsigned long long), L.st));
@@ -163,6 +165,7 @@ void lane_free(Lane& L) {
     if (L.d_items) hipFree(L.d_items);
     if (L.h_items) hipHostFree(L.h_items);
     if (L.d_status) hipFree(L.d_status);
+    if (L.d_offs) hipFree(L.d_offs);
     if (L.d_misc) hipFree(L.d_misc);
     if (L.d_err) hipFree(L.d_err);
     if (L.d_sizes) hipFree(L.d_sizes);
@@ -183,7 +186,8 @@ uint64_t tiles_of(const Req& r) {
 // Enqueues lane L's batch (L.reqs, compress first) on its stream. The lane is idle.
 int lane_launch(cuszp_server_s& s, Lane& L) {
     const size_t n = L.reqs.size();
-    uint64_t tc = 0, td = 0;
+    uint64_t tc = 0, td = 0, seg = 0;
+    bool pass = false;   // a decompressed array's header is too long for its tiles to sum up
     for (size_t k = 0; k < n; ++k) {
         Req& r = L.reqs[k];
         const bool c = r.dir == CUSZP_BATCH_COMPRESS;
@@ -197,6 +201,11 @@ int lane_launch(cuszp_server_s& s, Lane& L) {
         uint64_t& t = c ? tc : td;
         item.tile0 = t;
         t += g.ntiles;
+        if (!c) {
+            item.seg0 = seg;   // at most a segment per tile
+            seg += batch_segments(it.dim, it.type == CUSZP_TYPE_DOUBLE, 0, g.ntiles * kServeWaves);
+            pass |= g.H > kBatchDirectHeader;
+        }
         L.h_items[k] = item;
     }
     const uint64_t need = tc > td ? tc : td;
@@ -205,7 +214,10 @@ int lane_launch(cuszp_server_s& s, Lane& L) {
         if (L.d_status) SRV_HIP(hipFree(L.d_status));
         L.d_status = nullptr;
         L.cap_tiles = 0;   // a failed allocation below leaves no array to launch on
+        if (L.d_offs) SRV_HIP(hipFree(L.d_offs));
+        L.d_offs = nullptr;
         SRV_HIP(scan_state_alloc(&L.d_status, (kStatusGuard + cap) * sizeof(unsigned long long)));
+        SRV_HIP(scan_state_alloc(&L.d_offs, cap * kServeWaves * sizeof(unsigned long long)));
         L.cap_tiles = cap;
         SRV_HIP(hipMemsetAsync(L.d_status, 0, (kStatusGuard + cap) * sizeof(unsigned long long), L.st));
         L.launches = 0;
@@ -227,9 +239,12 @@ int lane_launch(cuszp_server_s& s, Lane& L) {
         ++L.launches;
     }
     if (n > nc) {
-        SRV_HIP(launch_bump_epoch(L.d_misc, L.st));
-        SRV_HIP(launch_decompress_batch(kServeWaves, kLookbackWords, L.d_items + nc, (uint32_t)(n - nc), td, sc, L.d_misc, L.st));
-        ++L.launches;
+        if (pass) {
+            SRV_HIP(launch_bump_epoch(L.d_misc, L.st));
+            SRV_HIP(launch_offsets_batch(kServeWaves, L.d_items + nc, (uint32_t)(n - nc), seg, L.d_offs, sc, L.d_misc, L.st));
+            ++L.launches;
+        }
+        SRV_HIP(launch_decompress_batch(kServeWaves, L.d_items + nc, (uint32_t)(n - nc), td, pass ? L.d_offs : nullptr, nullptr, L.st));
     }
     SRV_HIP(hipMemcpyAsync(L.h_err, L.d_err, n * sizeof(unsigned int), hipMemcpyDeviceToHost, L.st));
     if (nc) SRV_HIP(hipMemcpyAsync(L.h_sizes, L.d_sizes, nc * sizeof(unsigned long long), hipMemcpyDeviceToHost, L.st));

@@ -10,10 +10,10 @@ static hipError_t launch_c(const Item& item, const ScanCtx& sc, hipStream_t st) 
     return launch_tiles(compress_kernel<D, M, float, W, D == 1>, W * kWaveSize, item.geo.ntiles, st, item, sc);
 }
 template <int D, int M, int W>
-static hipError_t launch_d(const Item& item, const ScanCtx& sc, const unsigned long long* offs, hipStream_t st) {
+static hipError_t launch_d(const Item& item, const unsigned long long* offs, hipStream_t st) {
     if (D == 1 || item.geo.runs)
-        return launch_tiles(decompress_kernel<D, M, float, W, true>, W * kWaveSize, item.geo.ntiles, st, item, sc, offs);
-    return launch_tiles(decompress_kernel<D, M, float, W, D == 1>, W * kWaveSize, item.geo.ntiles, st, item, sc, offs);
+        return launch_tiles(decompress_kernel<D, M, float, W, true>, W * kWaveSize, item.geo.ntiles, st, item, offs);
+    return launch_tiles(decompress_kernel<D, M, float, W, D == 1>, W * kWaveSize, item.geo.ntiles, st, item, offs);
 }
 
 // offset pass: S bytes per plane (1D 4, 2D/3D 8), UB blocks per decode wave
@@ -32,9 +32,9 @@ hipError_t launch_compress_f32(int dim, int mode, int waves, const Item& item, c
     CUSZP_DISPATCH(launch_c, item, sc, st)
 }
 
-hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item, const ScanCtx& sc,
-                                 const unsigned long long* offs, hipStream_t st) {
-    CUSZP_DISPATCH(launch_d, item, sc, offs, st)
+hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item, const unsigned long long* offs,
+                                 hipStream_t st) {
+    CUSZP_DISPATCH(launch_d, item, offs, st)
 }
 
 hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,

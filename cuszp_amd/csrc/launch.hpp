@@ -25,10 +25,10 @@ hipError_t launch_compress_f64(int dim, int mode, int waves, const Item& item, c
 // Single-array decompression reads each wave's payload offset from `offs`,
 // which launch_unit_offsets_* fills first on the same stream; a null `offs`
 // (headers of at most kDirectHeader bytes) has every workgroup sum them up.
-hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item, const ScanCtx& sc,
-                                 const unsigned long long* offs, hipStream_t st);
-hipError_t launch_decompress_f64(int dim, int mode, int waves, const Item& item, const ScanCtx& sc,
-                                 const unsigned long long* offs, hipStream_t st);
+hipError_t launch_decompress_f32(int dim, int mode, int waves, const Item& item, const unsigned long long* offs,
+                                 hipStream_t st);
+hipError_t launch_decompress_f64(int dim, int mode, int waves, const Item& item, const unsigned long long* offs,
+                                 hipStream_t st);
 // Offset table of a single-array decompression (unit_offsets_kernel): offs[u]
 // for the nunits decode waves of `item`'s plan, from the header bytes of the
 // stream at item.src; sc's status words serve the pass's own scan (one per
@@ -38,7 +38,7 @@ hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t
 hipError_t launch_unit_offsets_f64(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
                                    const ScanCtx& sc, hipStream_t st);
 // Blocks one decode wave handles.
-inline uint64_t unit_blocks(int dim, bool f64) { return tile_groups(f64, 1) * (dim == 1 ? 2 : 1); }
+inline uint64_t unit_blocks(int dim, bool f64, int kc = 0) { return tile_groups(f64, 1, kc) * (dim == 1 ? 2 : 1); }
 // Segments of the offset pass over `nunits` units.
 inline uint64_t unit_segments(int dim, bool f64, uint64_t nunits) {
     return (nunits * unit_blocks(dim, f64) + kPrefixSegBytes - 1) / kPrefixSegBytes;
@@ -50,12 +50,22 @@ inline uint64_t unit_segments(int dim, bool f64, uint64_t nunits) {
 // lane, 2 or 4 (128 or 256 predecessors per round trip).
 hipError_t launch_compress_batch(int waves, int window, const Item* items, uint32_t nitems, uint64_t ntiles,
                                  const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
-hipError_t launch_decompress_batch(int waves, int window, const Item* items, uint32_t nitems, uint64_t ntiles,
-                                   const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
 hipError_t launch_compress_batch8(int window, const Item* items, uint32_t nitems, uint64_t ntiles, const ScanCtx& sc,
                                   const unsigned long long* epoch, hipStream_t st);
-hipError_t launch_decompress_batch8(int window, const Item* items, uint32_t nitems, uint64_t ntiles, const ScanCtx& sc,
-                                    const unsigned long long* epoch, hipStream_t st);
+// Batched decompression: offs[ntiles * waves], filled by launch_offsets_batch on
+// the same stream, or null where no array's header is longer than kBatchDirectHeader;
+// bump (may be null): an epoch word to advance, for the next pass.
+hipError_t launch_decompress_batch(int waves, const Item* items, uint32_t nitems, uint64_t ntiles,
+                                   const unsigned long long* offs, unsigned long long* bump, hipStream_t st);
+hipError_t launch_decompress_batch8(const Item* items, uint32_t nitems, uint64_t ntiles,
+                                    const unsigned long long* offs, unsigned long long* bump, hipStream_t st);
+// The offset pass over nseg segments in all (items ordered by seg0, batch_segments
+// each), whose waves have whole threads' header bytes (unit_blocks % kPrefixBytes == 0).
+hipError_t launch_offsets_batch(int waves, const Item* items, uint32_t nitems, uint64_t nseg, unsigned long long* offs,
+                                const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
+inline uint64_t batch_segments(int dim, bool f64, int kc, uint64_t nunits) {
+    return (nunits * unit_blocks(dim, f64, kc) + kBatchSegBytes - 1) / kBatchSegBytes;
+}
 // Increments *epoch (one thread); runs before each batched launch.
 hipError_t launch_bump_epoch(unsigned long long* epoch, hipStream_t st);
 // Largest grid of a tile launch; arrays with more tiles take several launches.
