@@ -37,17 +37,17 @@ struct GridWords {
         }
         return false;
     }
-    // N words from word i on, their loads in flight together; the few that are not there yet are polled.
+    // N words from word i on, `stride` apart, their loads in flight together; the few that are not there yet are polled.
     template <int N>
-    __device__ __forceinline__ bool get_n(uint64_t i, uint32_t (&v)[N]) const {
+    __device__ __forceinline__ bool get_n(uint64_t i, uint32_t (&v)[N], uint64_t stride = 1) const {
         unsigned long long x[N];
 #pragma unroll
-        for (int k = 0; k < N; ++k) x[k] = __hip_atomic_load(w + i + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = 0; k < N; ++k) x[k] = __hip_atomic_load(w + i + k * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         bool ok = true;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
             v[k] = (uint32_t)x[k];
-            if ((uint32_t)(x[k] >> 32) != tag) ok &= get(i + k, v[k]);
+            if ((uint32_t)(x[k] >> 32) != tag) ok &= get(i + k * stride, v[k]);
         }
         return ok;
     }

@@ -107,7 +107,7 @@ __device__ __forceinline__ void block_figures(Figures& f, double* sm) {
 // each array at a time (their loads in flight together), centres them on their
 // own means and merges the result into its moments. Bound by the read: 21.8 M
 // pairs of f32 (175 MB) took 124 us as two passes (means first, then centred
-// sums) and 60 us this way.
+// sums) and 48 us this way, about 10 of them the reductions at the end.
 // gw: kFigures values of two words per workgroup; res: the figures.
 template <class T>
 __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__ ori, const T* __restrict__ dec,
@@ -172,11 +172,14 @@ __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__
     block_figures(f, sm);
     typedef cuszp::Words<double> W;
     if (blockIdx.x != gridDim.x - 1) {
+        // word k of every workgroup in a row: the last workgroup's lanes read
+        // neighbours (each workgroup's words in a row, 57,000 lines read one by one,
+        // cost 12 us of the 60)
         if (threadIdx.x == 0)
             f.each([&](int k, double& v) {
                 const W w = W::of(v);
-                gw.put(((uint64_t)blockIdx.x * kFigures + k) * 2, w.u[0]);
-                gw.put(((uint64_t)blockIdx.x * kFigures + k) * 2 + 1, w.u[1]);
+                gw.put((uint64_t)(2 * k) * gridDim.x + blockIdx.x, w.u[0]);
+                gw.put((uint64_t)(2 * k + 1) * gridDim.x + blockIdx.x, w.u[1]);
             });
         return;
     }
@@ -184,7 +187,7 @@ __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__
     bool ok = true;
     for (unsigned b = threadIdx.x; b + 1 < gridDim.x; b += kThreads) {
         uint32_t u[2 * kFigures];
-        ok &= gw.get_n((uint64_t)b * kFigures * 2, u);
+        ok &= gw.get_n((uint64_t)b, u, gridDim.x);
         Figures g;
         g.each([&](int k, double& v) {
             W w;
@@ -209,6 +212,17 @@ static_assert(kFigures < cuszp::kGridResults, "the figures and the flag");
 // with c1 = (0.01 R)^2, c2 = (0.03 R)^2, c3 = c2 / 2, R the window's original
 // range (1 when the range is 0).
 constexpr int kWin = 7, kWinStep = 2;
+
+// Smaller and larger of two or three values, one instruction each (fmin would
+// quieten its operands first; a window with a NaN has no SSIM whatever its range).
+__device__ __forceinline__ float min_of(float a, float b) { asm("v_min_f32 %0, %1, %2" : "=v"(a) : "v"(a), "v"(b)); return a; }
+__device__ __forceinline__ double min_of(double a, double b) { asm("v_min_f64 %0, %1, %2" : "=v"(a) : "v"(a), "v"(b)); return a; }
+__device__ __forceinline__ float most_of(float a, float b) { asm("v_max_f32 %0, %1, %2" : "=v"(a) : "v"(a), "v"(b)); return a; }
+__device__ __forceinline__ double most_of(double a, double b) { asm("v_max_f64 %0, %1, %2" : "=v"(a) : "v"(a), "v"(b)); return a; }
+__device__ __forceinline__ float min_of(float a, float b, float c) { asm("v_min3_f32 %0, %1, %2, %3" : "=v"(a) : "v"(a), "v"(b), "v"(c)); return a; }
+__device__ __forceinline__ float most_of(float a, float b, float c) { asm("v_max3_f32 %0, %1, %2, %3" : "=v"(a) : "v"(a), "v"(b), "v"(c)); return a; }
+__device__ __forceinline__ double min_of(double a, double b, double c) { return min_of(min_of(a, b), c); }
+__device__ __forceinline__ double most_of(double a, double b, double c) { return most_of(most_of(a, b), c); }
 
 // Sums, centred sums and range of a set of pairs: a row of a window, a slice, or all of it.
 template <class T>
@@ -238,8 +252,8 @@ struct Join {
         s.xx += a.xx;
         s.yy += a.yy;
         s.xy += a.xy;
-        s.lo = a.lo < s.lo ? a.lo : s.lo;
-        s.hi = a.hi > s.hi ? a.hi : s.hi;
+        s.lo = min_of(s.lo, a.lo);
+        s.hi = most_of(s.hi, a.hi);
     }
     __device__ __forceinline__ WinStats<T> done(double n) const {
         WinStats<T> r = s;
@@ -253,9 +267,46 @@ struct Join {
     }
 };
 
+// Two slices as one set.
+constexpr double kSlice = kWin * kWin;   // values of a window's slice
+template <class T>
+__device__ __forceinline__ WinStats<T> pair_of(const WinStats<T>& a, const WinStats<T>& b) {
+    const double u = b.x - a.x, v = b.y - a.y, fu = u * (1 / (2 * kSlice)), fv = v * (1 / (2 * kSlice));
+    return {a.x + b.x, a.y + b.y, fma(fu, u, a.xx + b.xx), fma(fv, v, a.yy + b.yy), fma(fu, v, a.xy + b.xy),
+            min_of(a.lo, b.lo), most_of(a.hi, b.hi)};
+}
+// A window's seven slices: three pairs and one more. Distances of sums are
+// taken from the first pair's, as in Join.
+template <class T>
+__device__ __forceinline__ WinStats<T> window_of(const WinStats<T> (&p)[3], const WinStats<T>& d) {
+    static_assert(kWin == 7, "three pairs and a slice");
+    const double u1 = p[1].x - p[0].x, v1 = p[1].y - p[0].y, u2 = p[2].x - p[0].x, v2 = p[2].y - p[0].y;
+    const double du = u1 + u2, dv = v1 + v2, eu = du * (1.0 / 3), ev = dv * (1.0 / 3);
+    // the last slice's distance from the pairs' mean, times 6 slices
+    const double wu = fma(6.0, fma(-0.5, p[0].x, d.x), -du), wv = fma(6.0, fma(-0.5, p[0].y, d.y), -dv);
+    constexpr double f = 1 / (2 * kSlice), g = 1 / (42 * kSlice);
+    WinStats<T> r;
+    r.x = fma(3.0, p[0].x, du) + d.x;
+    r.y = fma(3.0, p[0].y, dv) + d.y;
+    r.xx = fma(wu * g, wu, fma(fma(-eu, du, fma(u1, u1, u2 * u2)), f, p[0].xx + p[1].xx + p[2].xx + d.xx));
+    r.yy = fma(wv * g, wv, fma(fma(-ev, dv, fma(v1, v1, v2 * v2)), f, p[0].yy + p[1].yy + p[2].yy + d.yy));
+    r.xy = fma(wu * g, wv, fma(fma(-eu, dv, fma(u1, v1, u2 * v2)), f, p[0].xy + p[1].xy + p[2].xy + d.xy));
+    r.lo = min_of(min_of(p[0].lo, p[1].lo, p[2].lo), d.lo);
+    r.hi = most_of(most_of(p[0].hi, p[1].hi, p[2].hi), d.hi);
+    return r;
+}
+
 template <class T>
 __device__ __forceinline__ double ssim_of(const WinStats<T>& s) {
     constexpr double np = kWin * kWin * kWin;
+    if constexpr (sizeof(T) == 4) {
+        // sums of floats are far from the limits of double: numerators and
+        // denominators scaled by the count instead of divided by it, one division
+        const double rr = (double)(T)(s.hi - s.lo), q = rr == 0 ? 1.0 : rr * rr;
+        const double c1 = (0.01 * 0.01) * (np * np) * q, c2 = (0.03 * 0.03) * np * q, d = s.xx + s.yy + c2;
+        if (c2 > 0 && d < INFINITY)
+            return fma(2 * s.x, s.y, c1) * fma(2.0, s.xy, c2) / (fma(s.x, s.x, fma(s.y, s.y, c1)) * d);
+    }
     const double mx = s.x / np, my = s.y / np, vx = s.xx / np, vy = s.yy / np, vxy = s.xy / np;
     const double rr = (double)(T)(s.hi - s.lo);   // the range in the values' type
     const double c1 = rr == 0 ? 0.01 * 0.01 : 0.01 * 0.01 * rr * rr;
@@ -278,22 +329,37 @@ struct SsimPlan {
     uint64_t depth;              // layers of windows per tile
 };
 
+// Barrier that orders LDS accesses only: loads from global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Workgroups per CU that the kernel is built for (registers, and LDS of 44 or 61 KB).
+template <class T> constexpr int kSsimPerCu = sizeof(T) == 4 ? 3 : 2;
+
 // One workgroup per tile (then the tile gridDim.x further on). It walks down
-// the tile's slices; for each, threads first make the statistics of the rows of
-// seven values that windows start with (2 TY + 5 rows, TX per row), then each
-// thread, one window column, joins seven of them to its slice of 7 x 7 and keeps
-// the last seven slices in registers; every second slice completes a layer.
-// A value takes part in 3.5 rows, 3.5 x 3.5 slices... through these sums and is
-// read 3.5 times (from L1), where a window by itself reads 343 pairs twice.
-// Bound by the f64 arithmetic: about 100 operations per value. 2.5 M windows of
-// f32 took 784 us as one thread per window, 190 us this way.
+// the tile's slices. The values of a slice come to LDS by way of registers, read
+// while the slice before is worked on; from there threads first make the
+// statistics of the rows of seven values that windows start with (2 TY + 5 rows,
+// TX per row), then each thread, one window column, joins seven of them to its
+// slice of 7 x 7 and those to pairs; three pairs and a slice are a window.
+// A value is read once and takes part in 3.5 rows, 3.5 x 3.5 slices... through
+// these sums, where a window by itself reads 343 pairs twice. Bound by the f64
+// arithmetic, about 80 operations per value, and the waits between its steps.
+// 2.5 M windows of f32: 784 us as one thread per window, 190 us with rows read
+// from memory as they are needed and 6 layers per tile, 156 us with LDS and deep
+// tiles, 131 us with the rows of two windows made together.
 template <class T, int TX>
-__global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2) ssim_kernel(const T* __restrict__ x, const T* __restrict__ y,
+__global__ void __launch_bounds__(kThreads, kSsimPerCu<T>) ssim_kernel(const T* __restrict__ x, const T* __restrict__ y,
                                                         const SsimPlan p, const cuszp::GridWords gw, double* res) {
-    constexpr int TY = kThreads / TX, ROWS = kWinStep * TY + kWin - kWinStep;
-    typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
-    __shared__ double rs[5][ROWS][TX];
-    __shared__ T rlo[ROWS][TX], rhi[ROWS][TX];
+    constexpr int TY = kThreads / TX, ROWS = kWinStep * TY + kWin - kWinStep, COLS = kWinStep * TX + kWin - kWinStep;
+    constexpr int STRIDE = (COLS + 1) / 2 * 2, NV = (ROWS * COLS + kThreads - 1) / kThreads;   // values per thread
+    typedef T V2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double rs[5][ROWS][TX];
+    __shared__ __align__(16) T rlo[ROWS][TX], rhi[ROWS][TX];
+    __shared__ V2 raw[2][ROWS][STRIDE / 2];
     __shared__ double sm[kThreads / 64];
     __shared__ bool lost;
     const int tid = (int)threadIdx.x, tx = tid % TX, ty = tid / TX;
@@ -304,57 +370,92 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2) ssim_kernel(
         const uint64_t wy0 = r % p.t1 * TY, wz0 = r / p.t1 * p.depth;
         const uint64_t layers = p.nw2 - wz0 < p.depth ? p.nw2 - wz0 : p.depth;
         const bool mine = wx0 + tx < p.nw0 && wy0 + ty < p.nw1;
-        // threads past the last window read the last one's values and count nothing
-        const uint64_t cx = kWinStep * (wx0 + tx < p.nw0 ? wx0 + tx : p.nw0 - 1);
-        WinStats<T> ring[kWin];
-        auto slice = [&](uint64_t z) -> WinStats<T> {   // this thread's 7 x 7 of slice z
-            __syncthreads();                            // the previous slice's rows have been read
-#pragma unroll 1
-            for (int r0 = 0; r0 < ROWS; r0 += TY) {
-                const int row = r0 + ty;
-                if (row < ROWS) {
-                    uint64_t yy = kWinStep * wy0 + row;
-                    yy = yy < p.s1 ? yy : p.s1 - 1;
-                    const uint64_t at = (z * p.s1 + yy) * p.s0 + cx;
-                    T a[kWin], c[kWin];
+        // this thread's values of a slice; past the extents the last ones again (in windows that count nothing)
+        uint64_t at[NV];
 #pragma unroll
-                    for (int i = 0; i < kWin / 2; ++i) {
-                        const V2 va = *(const V2*)(x + at + 2 * i), vc = *(const V2*)(y + at + 2 * i);
-                        a[2 * i] = va[0];
-                        a[2 * i + 1] = va[1];
-                        c[2 * i] = vc[0];
-                        c[2 * i + 1] = vc[1];
-                    }
-                    a[kWin - 1] = x[at + kWin - 1];
-                    c[kWin - 1] = y[at + kWin - 1];
-                    double sx = 0, sy = 0;
-                    T lo = a[0], hi = a[0];
+        for (int k = 0; k < NV; ++k) {
+            const int i = tid + k * kThreads < ROWS * COLS ? tid + k * kThreads : ROWS * COLS - 1;
+            uint64_t yy = kWinStep * wy0 + i / COLS, xx = kWinStep * wx0 + i % COLS;
+            yy = yy < p.s1 ? yy : p.s1 - 1;
+            xx = xx < p.s0 ? xx : p.s0 - 1;
+            at[k] = (kWinStep * wz0 * p.s1 + yy) * p.s0 + xx;
+        }
+        T vx[NV], vy[NV];
+        auto load = [&]() {   // and on to the next slice
 #pragma unroll
-                    for (int i = 0; i < kWin; ++i) {
-                        sx += (double)a[i];
-                        sy += (double)c[i];
-                        lo = a[i] < lo ? a[i] : lo;
-                        hi = a[i] > hi ? a[i] : hi;
-                    }
-                    const double mx = sx * (1.0 / kWin), my = sy * (1.0 / kWin);
-                    double xx = 0, yy2 = 0, xy = 0;
+            for (int k = 0; k < NV; ++k) {
+                vx[k] = x[at[k]];
+                vy[k] = y[at[k]];
+                at[k] += p.s0 * p.s1;
+            }
+        };
+        auto slice = [&](bool more) -> WinStats<T> {   // this thread's 7 x 7 of the slice in vx, vy; loads the next
 #pragma unroll
-                    for (int i = 0; i < kWin; ++i) {
-                        const double u = (double)a[i] - mx, v = (double)c[i] - my;
-                        xx = fma(u, u, xx);
-                        yy2 = fma(v, v, yy2);
-                        xy = fma(u, v, xy);
-                    }
-                    rs[0][row][tx] = sx;
-                    rs[1][row][tx] = sy;
-                    rs[2][row][tx] = xx;
-                    rs[3][row][tx] = yy2;
-                    rs[4][row][tx] = xy;
-                    rlo[row][tx] = lo;
-                    rhi[row][tx] = hi;
+            for (int k = 0; k < NV; ++k) {
+                const int i = tid + k * kThreads;
+                if (i < ROWS * COLS) {
+                    ((T*)raw[0][i / COLS])[i % COLS] = vx[k];
+                    ((T*)raw[1][i / COLS])[i % COLS] = vy[k];
                 }
             }
-            __syncthreads();
+            if (more) load();
+            lds_barrier();   // also: the rows of the slice before have been read
+#pragma unroll 1
+            for (int i = tid; i < ROWS * TX / 2; i += kThreads) {   // the rows of two windows, values 0-6 and 2-8
+                const int row = i / (TX / 2), wx = i % (TX / 2) * 2;
+                T a[kWin + 2], c[kWin + 2];
+#pragma unroll
+                for (int j = 0; j < (kWin + 2) / 2; ++j) {
+                    const V2 va = raw[0][row][wx + j], vc = raw[1][row][wx + j];
+                    a[2 * j] = va[0];
+                    a[2 * j + 1] = va[1];
+                    c[2 * j] = vc[0];
+                    c[2 * j + 1] = vc[1];
+                }
+                a[kWin + 1] = raw[0][row][wx + (kWin + 1) / 2][0];
+                c[kWin + 1] = raw[1][row][wx + (kWin + 1) / 2][0];
+                // distances from value 4, a member of both rows: the correction to
+                // their own mean cancels at most the number of values
+                const double ra = (double)a[4], rc = (double)c[4];
+                double u[kWin + 2], v[kWin + 2], su = 0, sv = 0, uu = 0, vv = 0, uv = 0;
+#pragma unroll
+                for (int j = 0; j < kWin + 2; ++j) {
+                    u[j] = (double)a[j] - ra;
+                    v[j] = (double)c[j] - rc;
+                }
+                auto add = [&](int j, double& su, double& sv, double& uu, double& vv, double& uv) {
+                    su += u[j];
+                    sv += v[j];
+                    uu = fma(u[j], u[j], uu);
+                    vv = fma(v[j], v[j], vv);
+                    uv = fma(u[j], v[j], uv);
+                };
+                for (int j : {2, 3, 5, 6}) add(j, su, sv, uu, vv, uv);
+                const T lo = min_of(min_of(a[2], a[3], a[4]), a[5], a[6]), hi = most_of(most_of(a[2], a[3], a[4]), a[5], a[6]);
+                typedef double D2 __attribute__((ext_vector_type(2)));
+                D2 o[5];
+                V2 ol, oh;
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    double s1 = su, s2 = sv, q1 = uu, q2 = vv, q3 = uv;
+                    const int e = w ? kWin : 0;   // the two values that are this row's alone
+                    add(e, s1, s2, q1, q2, q3);
+                    add(e + 1, s1, s2, q1, q2, q3);
+                    const double e1 = s1 * (1.0 / kWin), e2 = s2 * (1.0 / kWin);
+                    o[0][w] = fma((double)kWin, ra, s1);
+                    o[1][w] = fma((double)kWin, rc, s2);
+                    o[2][w] = fma(-e1, s1, q1);
+                    o[3][w] = fma(-e2, s2, q2);
+                    o[4][w] = fma(-e1, s2, q3);
+                    ol[w] = min_of(lo, a[e], a[e + 1]);
+                    oh[w] = most_of(hi, a[e], a[e + 1]);
+                }
+#pragma unroll
+                for (int k = 0; k < 5; ++k) *(D2*)&rs[k][row][wx] = o[k];
+                *(V2*)&rlo[row][wx] = ol;
+                *(V2*)&rhi[row][wx] = oh;
+            }
+            lds_barrier();
             auto at_row = [&](int row) -> WinStats<T> {
                 return WinStats<T>{rs[0][row][tx], rs[1][row][tx], rs[2][row][tx], rs[3][row][tx], rs[4][row][tx],
                                    rlo[row][tx], rhi[row][tx]};
@@ -365,23 +466,19 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2) ssim_kernel(
             for (int j = 1; j < kWin; ++j) q.next(at_row(kWinStep * ty + j));
             return q.done((double)kWin);
         };
-        // 2 * layers + 5 slices: one, then pairs; from the third pair on each completes a layer
-        const uint64_t z0 = kWinStep * wz0;
-        for (int k = 0; k < kWin; ++k) ring[k] = WinStats<T>{0, 0, 0, 0, 0, T(0), T(0)};
-        ring[kWin - 3] = slice(z0);
+        // 2 * layers + 5 slices in pairs; from the fourth pair on the first slice of each completes a layer
+        load();
+        WinStats<T> ring[3];
+        for (int k = 0; k < 3; ++k) ring[k] = WinStats<T>{0, 0, 0, 0, 0, T(0), T(0)};
 #pragma unroll 1
-        for (uint64_t l = 0; l < layers + 2; ++l) {
-#pragma unroll
-            for (int k = kWin - 2; k < kWin; ++k) ring[k] = slice(z0 + 2 * l + (uint64_t)(k - (kWin - 3)));
-            if (l >= 2 && mine) {
-                Join<T> q;
-                q.first(ring[0]);
-#pragma unroll
-                for (int k = 1; k < kWin; ++k) q.next(ring[k]);
-                total += ssim_of(q.done((double)(kWin * kWin)));
-            }
-#pragma unroll
-            for (int k = 0; k < kWin - 2; ++k) ring[k] = ring[k + 2];
+        for (uint64_t l = 0; l < layers + 3; ++l) {
+            const bool last = l == layers + 2;
+            const WinStats<T> d = slice(!last);
+            if (l >= 3 && mine) total += ssim_of(window_of(ring, d));
+            if (last) break;
+            ring[0] = ring[1];
+            ring[1] = ring[2];
+            ring[2] = pair_of(d, slice(true));
         }
     }
     auto block_sum = [&](double v) -> double {   // in thread 0
@@ -493,13 +590,21 @@ int run_ssim(const T* x, const T* y, cuszp_dims_t d, double* out, hipStream_t st
     const uint64_t tx = narrow ? 8 : 32, ty = kThreads / tx;
     p.t0 = (p.nw0 + tx - 1) / tx;
     p.t1 = (p.nw1 + ty - 1) / ty;
-    // Layers per tile: a tile reads 5 slices before its first layer, so few and
-    // deep tiles do less work, but the chip holds kMaxSsimBlocks workgroups and
-    // needs about that many; at least 4 layers.
-    uint64_t chunks = (kMaxSsimBlocks + p.t0 * p.t1 - 1) / (p.t0 * p.t1);
-    if (chunks > (p.nw2 + 3) / 4) chunks = (p.nw2 + 3) / 4;
-    p.depth = (p.nw2 + chunks - 1) / chunks;
-    p.tiles = p.t0 * p.t1 * ((p.nw2 + p.depth - 1) / p.depth);
+    // Layers per tile: a tile goes through 2 * depth + 5 slices, so deep tiles do
+    // less work, but the chip works on kResident tiles at a time and the last
+    // round should be full: the depth with the fewest slices in a row.
+    constexpr uint64_t kResident = 256 * kSsimPerCu<T>;
+    uint64_t best = ~0ull;
+    for (uint64_t chunks = 1; chunks <= p.nw2 && chunks <= 4 * kResident; ++chunks) {
+        const uint64_t depth = (p.nw2 + chunks - 1) / chunks, tiles = p.t0 * p.t1 * ((p.nw2 + depth - 1) / depth);
+        const uint64_t cost = (tiles + kResident - 1) / kResident * (kWinStep * depth + kWin - kWinStep);
+        if (cost < best) {
+            best = cost;
+            p.depth = depth;
+            p.tiles = tiles;
+        }
+        if (tiles > 4 * kResident) break;   // only more work from here on
+    }
     const unsigned blocks = p.tiles < kMaxSsimBlocks ? (unsigned)p.tiles : kMaxSsimBlocks;
     if (narrow)
         hipLaunchKernelGGL((ssim_kernel<T, 8>), dim3(blocks), dim3(kThreads), 0, st, x, y, p, gw, s.g.h_res);

@@ -64,3 +64,18 @@ def test_range_edges(device, oracle, dtype, n):
             t[off + at] = -1e6
             assert P.value_range(t[off:off + n]) == (float(h.min()), float(h.max()))
             t[off + at] = float(x[off + at])
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-20, 1e20, 1e37])
+def test_ssim_scales(device, oracle, scale):
+    """Floats near both ends of their range: the window formula's products stay within double's."""
+    import torch
+    from cuszp_amd import pycuSZp as P
+
+    dims = (40, 19, 13)
+    r = np.random.default_rng(3)
+    n = dims[0] * dims[1] * dims[2]
+    x = (r.normal(1, 0.5, n) * scale).astype(np.float32)
+    y = (x * (1 + 0.05 * r.normal(0, 1, n))).astype(np.float32)
+    got = P.ssim(torch.from_numpy(x).to(device), torch.from_numpy(y).to(device), dims)
+    assert got == pytest.approx(oracle.ssim(x, y, dims), rel=1e-9)
