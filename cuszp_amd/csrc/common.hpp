@@ -112,6 +112,9 @@ inline int make_geom(int dim, size_t n, cuszp_dims_t d, Geom& g) {
                                              : (d.x % 32 == 0 && d.y % 4 == 0 && d.z % 4 == 0);
     const uint64_t reach = (dim == CUSZP_DIM_2D) ? 8ull * d.x : 4ull * g.XY;
     g.runs = whole && reach < (1ull << 28);
+    // f64, up to one block row on, or (narrow arrays) eight
+    const uint64_t rows = (dim == CUSZP_DIM_2D) ? (uint64_t)(d.y < 8 ? d.y : 8) * d.x : (d.z < 4 ? d.z : 4) * g.XY;
+    g.near = rows < (1ull << (g.Bx >= 8 ? 27 : 24));
     if (g.nblocks >= (1ull << 40)) return CUSZP_ERROR_TOO_LARGE;
     g.H = (g.nblocks + 3) / 4 * 4;                  // src/cuSZp_kernels_2D_f32.cu:46
     return CUSZP_SUCCESS;

@@ -101,6 +101,7 @@ struct Geom {
     uint32_t kc;        // chunks per wave of a tile (at most kChunksOf)
     uint32_t runs;      // every chunk's blocks lie inside the array, 2D/3D consecutive along x (extents multiples
                         // of the block, Bx of a chunk's 8 blocks), and their places fit 32-bit offsets
+    uint32_t near;      // 2D/3D: the places of a chunk's blocks fit 32-bit offsets from the first one's
 };
 
 // Launch-wide scan state.
@@ -1062,9 +1063,121 @@ __device__ __forceinline__ void trade_codes(uint32_t (&q)[2][4]) {
     }
 }
 
-// Where the quads of a 2D/3D chunk lie. The chunk's 8 blocks follow each other
-// along x; past the end of the row they go on in the next one. With Bx >= 8
-// that happens at most once, and both rows' origins are wave-uniform.
+// The quads of the chunks of an array whose extents are not multiples (Geom::near):
+// a chunk's 8 blocks follow each other along x, past the end of the row they go
+// on in the next one. Most chunks lie inside one row of whole blocks, and every
+// lane's place is then the same number of bytes from the chunk's origin. Quads outside the array get an offset past
+// every buffer range: loads give zeros, stores do nothing. (Two 64-bit offsets
+// per lane and chunk and predicated accesses before: compress kernels of
+// 3000 x 1999 x 16 f32 outlier 152 -> 146 us, 600 x 450 x 152 f32 plain 71 -> 69,
+// 300 x 450 x 152 f64 outlier 70 -> 64; what is left is arithmetic, and lines that
+// two chunks share: 137 us with rows of 3008.)
+template <int DIM, class T>
+struct RaggedQuads {
+    static constexpr uint32_t BW = QuadLane<DIM>::BW, SB = QuadLane<DIM>::SB, kSet = SB * BW * (uint32_t)sizeof(T);
+    Walker wk;
+    uint64_t end;        // first block that is not the wave's (or the array's): its chunks are not loaded ahead
+    uint64_t org;        // the next chunk's origin
+    uint32_t lane_off;   // bytes
+    __device__ __forceinline__ void init(const Geom& g, const QuadLane<DIM>& ql, uint64_t b0, uint64_t b1) {
+        end = b1 < g.nblocks ? b1 : g.nblocks;
+        wk.init(b0, g);
+        org = block_origin<DIM>(g, wk);
+        lane_off = ((DIM == 3 ? ql.z * (uint32_t)g.XY : 0u) + ql.y * g.X + ql.x + ql.blk * BW) * (uint32_t)sizeof(T);
+        opaque(lane_off);
+    }
+    // The next chunk: its origin (elements), its quads' offsets from there (bytes);
+    // true if all of them lie inside the array.
+    __device__ __forceinline__ bool next(const Geom& g, uint64_t& base, uint32_t (&vo)[2]) {
+        base = org;
+        vo[0] = lane_off;
+        vo[1] = lane_off + kSet;
+        auto lane_place = [] {   // made anew where it is needed: nothing of it in registers across the chunk's work
+            uint32_t l = __lane_id();
+            opaque_here(l);
+            QuadLane<DIM> q;
+            q.init((int)l);
+            return q;
+        };
+        bool whole = false;
+        if (g.Bx < 8) {   // block by block
+            const QuadLane<DIM> q = lane_place();
+            const uint32_t blk = q.blk, x = q.x, y = q.y, z = q.z;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                uint32_t o = kAbsent;
+#pragma unroll 1
+                for (uint32_t i = 0; i < SB; ++i) {
+                    bool v = (wk.b < end) & (wk.by * BW + y < g.Y) & (blk == i);
+                    if constexpr (DIM == 2) v &= wk.bx * BW + x < g.X;
+                    else v &= wk.bz * 4 + z < g.Z;
+                    o = v ? (uint32_t)(block_origin<DIM>(g, wk) - base) * (uint32_t)sizeof(T) + lane_off - blk * (BW * (uint32_t)sizeof(T)) : o;
+                    wk.next(g);
+                }
+                vo[s] = o;
+            }
+            org = block_origin<DIM>(g, wk);
+        } else {   // blocks of two rows at most; selects, no branches: the wave's registers stay scalar
+            whole = ((wk.bx + 8) * BW <= g.X) & ((wk.by + 1) * BW <= g.Y) & (DIM == 2 || (wk.bz + 1) * 4 <= g.Z) &
+                    (wk.b + 8 <= end);
+            const uint32_t left = g.Bx - wk.bx;   // blocks of the chunk in its first row
+            const bool last_row = wk.by + 1 == g.By;
+            Walker w1 = wk;                       // the row after it
+            w1.bx = 0;
+            w1.by = last_row ? 0u : wk.by + 1;
+            w1.bz = wk.bz + (last_row ? 1u : 0u);
+            const uint64_t o1 = block_origin<DIM>(g, w1);
+            if (!whole) {
+                const QuadLane<DIM> q = lane_place();
+                const uint32_t blk = q.blk, x = q.x, y = q.y, z = q.z;
+                const uint32_t jump = (uint32_t)(o1 - org - (uint64_t)left * BW) * (uint32_t)sizeof(T);
+                const uint32_t y0 = g.Y - wk.by * BW, y1 = g.Y - w1.by * BW;
+                const uint32_t z0 = g.Z - wk.bz * 4, z1 = g.Z - w1.bz * 4;   // 3D
+                const uint64_t nb = wk.b < end ? end - wk.b : 0;
+                const uint32_t blocks = nb < 8 ? (uint32_t)nb : 8u;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const uint32_t i = blk + s * SB;
+                    const bool in0 = i < left;
+                    bool v = (i < blocks) & (y < (in0 ? y0 : y1));
+                    if constexpr (DIM == 2) v &= (in0 ? wk.bx + i : i - left) * BW + x < g.X;
+                    else v &= z < (in0 ? z0 : z1);
+                    vo[s] = v ? vo[s] + (in0 ? 0u : jump) : kAbsent;
+                }
+            }
+            const bool on = left > 8;   // the next chunk starts in the same row
+            org = on ? org + 8 * BW : o1 + (uint64_t)(8 - left) * BW;
+            wk.b += 8;
+            wk.bx = on ? wk.bx + 8 : 8 - left;
+            wk.by = on ? wk.by : w1.by;
+            wk.bz = on ? wk.bz : w1.bz;
+        }
+        return whole;
+    }
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const T* p) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)uniform64((uint64_t)p), 0, 0x7fffffff, kBufferWord3);
+    }
+    static __device__ __forceinline__ void load(const T* p, uint32_t vo, T (&x)[4]) {
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int j = 0; j < (int)sizeof(T) / 4; ++j) {
+            const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rsrc(p), vo, 16 * j, 0);
+            __builtin_memcpy((char*)&x[0] + 16 * j, &v, 16);
+        }
+    }
+    static __device__ __forceinline__ void store(T* p, uint32_t vo, const T (&x)[4]) {
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int j = 0; j < (int)sizeof(T) / 4; ++j) {
+            v4u v;
+            __builtin_memcpy(&v, (const char*)&x[0] + 16 * j, 16);
+            __builtin_amdgcn_raw_buffer_store_b128(v, rsrc(p), vo, 16 * j, 0);
+        }
+    }
+};
+
+// Where the quads of a 2D/3D chunk lie, for any extents: 64-bit offsets, blocks
+// one by one.
 template <int DIM>
 struct ChunkQuads {
     uint64_t off[2];   // element offset of set s's quad (0 where outside)
@@ -1074,41 +1187,19 @@ struct ChunkQuads {
         constexpr uint32_t BW = QuadLane<DIM>::BW, SB = QuadLane<DIM>::SB;
         uint32_t blk = ql.blk, x = ql.x, y = ql.y, z = ql.z;
         opaque_here(blk);   // nothing of this in registers across the chunk's work
-        if (g.Bx >= 8) {
-            const uint32_t left = g.Bx - wk.bx;   // blocks of the chunk in its first row
-            Walker w1 = wk;
-            w1.step(g, left);
-            const uint64_t o0 = block_origin<DIM>(g, wk), o1 = block_origin<DIM>(g, w1) - (uint64_t)left * BW;
-            const uint32_t y0 = g.Y - wk.by * BW, y1 = g.Y - w1.by * BW;
-            const uint32_t z0 = g.Z - wk.bz * 4, z1 = g.Z - w1.bz * 4;   // 3D
-            const uint64_t nb = wk.b < g.nblocks ? g.nblocks - wk.b : 0;
-            const uint32_t blocks = nb < 8 ? (uint32_t)nb : 8u;
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const uint32_t i = blk + s * SB;
-                const bool in0 = i < left;
-                bool v = (i < blocks) & (y < (in0 ? y0 : y1));
-                if constexpr (DIM == 2) v &= (in0 ? wk.bx + i : i - left) * BW + x < g.X;
-                else v &= z < (in0 ? z0 : z1);
-                ok[s] = v;
-                off[s] = (in0 ? o0 : o1) + (uint64_t)i * BW;
-            }
-            wk.step(g, 8);
-        } else {   // block by block
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                ok[s] = false;
-                off[s] = 0;
+        for (int s = 0; s < 2; ++s) {
+            ok[s] = false;
+            off[s] = 0;
 #pragma unroll 1
-                for (uint32_t i = 0; i < SB; ++i) {
-                    bool v = (wk.b < g.nblocks) & (wk.by * BW + y < g.Y);
-                    if constexpr (DIM == 2) v &= wk.bx * BW + x < g.X;
-                    else v &= wk.bz * 4 + z < g.Z;
-                    const uint64_t o = block_origin<DIM>(g, wk);
-                    ok[s] = blk == i ? v : ok[s];
-                    off[s] = blk == i ? o : off[s];
-                    wk.next(g);
-                }
+            for (uint32_t i = 0; i < SB; ++i) {
+                bool v = (wk.b < g.nblocks) & (wk.by * BW + y < g.Y);
+                if constexpr (DIM == 2) v &= wk.bx * BW + x < g.X;
+                else v &= wk.bz * 4 + z < g.Z;
+                const uint64_t o = block_origin<DIM>(g, wk);
+                ok[s] = blk == i ? v : ok[s];
+                off[s] = blk == i ? o : off[s];
+                wk.next(g);
             }
         }
         const uint64_t lane_off = (uint64_t)z * g.XY + (uint64_t)y * g.X + x;
@@ -1527,14 +1618,29 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
     ql.init(lane);
     PlaneConsts pc;
     pc.init(lane, false);
-    const uint32_t pl = plane_of_lane(ql.k);
     // LDS addresses of the wave's staging area and of the spare word past it,
     // where lanes without a word write
     lds_u8* const sbase = (lds_u8*)sm.stage[wave];
     const uint32_t s0 = (uint32_t)(size_t)sbase, spare = s0 + kStageBytes;
-    // this lane's plane word of slice 0 in a block, and its header byte
-    const uint32_t po = ql.plane_offset(pl);
-    lds_u8* const hbase = (lds_u8*)sm.hdr[wave] + (ql.blk + (ql.second ? SB : 0));
+    // This lane's plane of slice 0, its word's place in a block, and where its
+    // block's header byte goes. Ragged chunks leave no registers for them: they are
+    // made anew for each chunk (a spilled one's reload would wait for the next
+    // chunk's loads, which are issued before).
+    constexpr bool kKept = RUNS;
+    const uint32_t pl = kKept ? plane_of_lane(ql.k) : 0u, po = kKept ? ql.plane_offset(pl) : 0u;
+    lds_u8* const hbase = (lds_u8*)sm.hdr[wave] + (kKept ? ql.blk + (ql.second ? SB : 0) : 0);
+    auto fresh = [] {
+        uint32_t l = __lane_id();
+        opaque_here(l);
+        QL q;
+        q.init((int)l);
+        return q;
+    };
+    auto plane_word = [&](uint32_t& p, uint32_t& o) {
+        const QL q = fresh();
+        p = plane_of_lane(q.k);
+        o = q.plane_offset(p);
+    };
 
     uint64_t excl = 0, wexcl = 0, ttot = 0;
     uint32_t wave_tot = 0;   // the wave's payload so far, of which `copied` bytes have left the staging area
@@ -1544,9 +1650,9 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
 
     // Processes chunk c from xv; roll(s) runs right after set s's values are
     // consumed (the next chunk's loads into xv[s] go there). PIECES: xv holds
-    // pieces (see Pieces), all inside the array; else quads, with vm's bits
-    // 4s + i for the elements inside.
-    auto process = [&](auto piecesc, int c, T (&xv)[2][4], const uint32_t vm, auto&& roll) {
+    // pieces (see Pieces), all inside the array; else quads, all inside the array
+    // or (!whole, wave-uniform) those elements whose bits 4s + i of vm are set.
+    auto process = [&](auto piecesc, int c, T (&xv)[2][4], const bool whole, const uint32_t vm, auto&& roll) {
         constexpr bool PIECES = decltype(piecesc)::value;
         uint32_t q[2][4], d[2][4];
 #pragma unroll
@@ -1566,7 +1672,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
 #pragma unroll
                 for (int i = 1; i < 4; ++i) d[s][i] = q[s][i] - q[s][i - 1];
             }
-            if constexpr (!PIECES) {   // codes and residuals of padding are 0
+            if (!PIECES && !whole) {   // codes and residuals of padding are 0
 #pragma unroll
                 for (int i = 0; i < 4; ++i) d[s][i] = ((vm >> (4 * s + i)) & 1) ? d[s][i] : 0u;
             }
@@ -1639,7 +1745,12 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
         // header bytes go to the stream after the wave's chunks: no global
         // store inside the chunk loop, whose waits for the rolling loads would
         // otherwise also wait for those stores
-        hbase[c * NB] = (uint8_t)hb;   // the same from all lanes that keep the block's books
+        if constexpr (kKept) {
+            hbase[c * NB] = (uint8_t)hb;
+        } else {
+            const QL f = fresh();
+            hbase[c * NB + f.blk + (f.second ? SB : 0)] = (uint8_t)hb;
+        }   // the same from all lanes that keep the block's books
         const uint64_t over7 = ballot(b > 8), over15 = ballot(b > 16);
         const uint32_t info = sz | (b << 16) | (nb << 24);
         const uint32_t inf0 = QL::of_set(info, 0), inf1 = QL::of_set(info, 1);
@@ -1694,10 +1805,12 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
                 for (int i = 0; i < NS; ++i) w[j * NS + i] = t[i];
             }
             to_planes<N * NS>(w, pc);
+            uint32_t pk = 0, pp = 0;
+            if constexpr (!kKept) plane_word(pk, pp);
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
                 // plane p is there if p + 1 < b, the sign word if 0 < b
-                uint32_t k = pl, p = po;
+                uint32_t k = kKept ? pl : pk, p = kKept ? po : pp;
                 opaque_here(k);
                 opaque_here(p);
                 const bool sign = i == NS - 1 && k == 7;
@@ -1720,6 +1833,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
         } else {
             // blocks of 32 planes: all 32 bits are planes and the sign words go separately
             uint32_t k = ql.k, p = pl, o = po;
+            if constexpr (!kKept) plane_word(p, o);
             opaque_here(k);
             opaque_here(p);
             opaque_here(o);
@@ -1776,7 +1890,7 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
                 for (int c = c0; c < nfull; ++c) {
                     // a set's next loads follow as soon as its values are coded
                     before(c);
-                    process(std::true_type{}, c, xv, 0u, [&](int s) { load(c + 1, s, xv[s]); });
+                    process(std::true_type{}, c, xv, true, 0u, [&](int s) { load(c + 1, s, xv[s]); });
                 }
             }
             if (DIM == 1 && nfull < nch) {   // the array's last elements
@@ -1793,26 +1907,48 @@ __device__ __forceinline__ void compress_tile(const Item& cur, const uint64_t ti
                         xv[s][i] = v ? in[at] : T(0);
                         vm |= (uint32_t)v << (4 * s + i);
                     }
-                process(std::false_type{}, nfull, xv, vm, [](int) {});
+                process(std::false_type{}, nfull, xv, false, vm, [](int) {});
             }
         } else if (c0 < nch) {
-            Walker wk;
-            wk.init(wgrp0 + (uint64_t)c0 * G, geo);
-            ChunkQuads<DIM> cq;
-            cq.locate(geo, ql, wk);
+            const bool near = geo.near != 0;
+            RaggedQuads<DIM, T> rq;
+            rq.init(geo, ql, wgrp0 + (uint64_t)c0 * G, wgrp0 + (uint64_t)KC * G);
+            const T* p = in;          // the chunk's origin
+            uint32_t vo[2] = {kAbsent, kAbsent};
+            auto locate = [&]() -> bool {
+                uint64_t base;
+                const bool whole = rq.next(geo, base, vo);
+                p = in + base;
+                return whole;
+            };
+            auto inside = [&]() -> uint32_t { return ((int32_t)vo[0] >= 0 ? 0xfu : 0u) | ((int32_t)vo[1] >= 0 ? 0xf0u : 0u); };
             T xv[2][4];
+            bool whole = false;
+            if (near) whole = locate();
 #pragma unroll
-            for (int s = 0; s < 2; ++s) load_quad<NT>(in + cq.off[s], xv[s]);
+            for (int s = 0; s < 2; ++s) RaggedQuads<DIM, T>::load(p, vo[s], xv[s]);
+            uint32_t vm = inside();
+            bool next_whole = false;
+            if (near) next_whole = locate();
 #pragma unroll 1
             for (int c = c0; c < nch; ++c) {
                 before(c);
-                const uint32_t vm = (cq.ok[0] ? 0xfu : 0u) | (cq.ok[1] ? 0xf0u : 0u);
+                if (!near) {   // rows (2D) or slices (3D) of tens of millions of values: no loads ahead
+                    ChunkQuads<DIM> cq;
+                    cq.locate(geo, ql, rq.wk);
+                    vm = (cq.ok[0] ? 0xfu : 0u) | (cq.ok[1] ? 0xf0u : 0u);
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                    for (int s = 0; s < 2; ++s) {
+                        load_quad<false>(in + cq.off[s], xv[s]);   // quads outside the array read its first one
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) xv[s][i] = cq.ok[s] ? xv[s][i] : T(0);
-                cq.locate(geo, ql, wk);   // quads outside the array read its first one
-                process(std::false_type{}, c, xv, vm, [&](int s) { load_quad<NT>(in + cq.off[s], xv[s]); });
+                        for (int i = 0; i < 4; ++i) xv[s][i] = cq.ok[s] ? xv[s][i] : T(0);
+                    }
+                }
+                process(std::false_type{}, c, xv, whole, vm, [&](int s) { RaggedQuads<DIM, T>::load(p, vo[s], xv[s]); });
+                // the chunk after the next, while the next one's loads are under way
+                whole = next_whole;
+                vm = inside();
+                if (near) next_whole = locate();
             }
         }
     };
@@ -2026,7 +2162,11 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
     const int nch = chunks_of(KC, wgrp0, gvalid, G - 1);
     const int nfull = (DIM == 1) ? chunks_of(KC, wgrp0, geo.n / 64, 0) : nch;
     Walker wkc;   // 2D/3D: the chunk being stored
-    if constexpr (DIM != 1) wkc.init(wgrp0, geo);
+    RaggedQuads<DIM, T> rq;
+    if constexpr (DIM != 1) {
+        if (!RUNS && geo.near) rq.init(geo, ql, wgrp0, wgrp0 + (uint64_t)KC * G);
+        else wkc.init(wgrp0, geo);
+    }
 
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) v4u lds_v4u;
@@ -2070,6 +2210,19 @@ __device__ __forceinline__ void decompress_tile(const Item& cur, const uint64_t 
                     if (e + 256 * s + i < geo.n) out[e + 256 * s + i] = value_of(q[s][i]);
         } else {
             // every quad by its own place; plain stores, which meet in L2
+            if (geo.near) {
+                uint64_t base;
+                uint32_t vo[2];
+                rq.next(geo, base, vo);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    T x[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = value_of(q[s][i]);
+                    RaggedQuads<DIM, T>::store(out + base, vo[s], x);
+                }
+                return;
+            }
             ChunkQuads<DIM> cq;
             cq.locate(geo, ql, wkc);
 #pragma unroll

@@ -120,3 +120,19 @@ def test_any_header_byte(device, oracle, dim, dims, n, mode):
     y = gpu_decompress(cmp, n, np.float32, 0.5, mode, dim, dims)
     ref = oracle.decompress(cmp, n, np.float32, 0.5, mode, dim, dims)
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+
+
+# Offsets past 32 bits from a chunk's origin (general path, wide and narrow), the last extents inside them, narrow
+# arrays of every width, rows whose last block is half outside with a single row below.
+@pytest.mark.parametrize("dim,dims", [(2, (44739244, 3, 1)), (2, (16777212, 9, 1)), (2, (16777220, 9, 1)), (3, (4, 1048576, 5)), (3, (4, 1048572, 5)),
+                                      (3, (8196, 4095, 5))] +
+                         [(d, (x, 17, 5)) for d in (2, 3) for x in range(4, 76, 8)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+def test_ragged_offsets(device, oracle, dim, dims, dtype):
+    n = dims[0] * dims[1] * dims[2]
+    r = np.random.default_rng(dims[0])
+    x = (np.arange(n) * 7 % 1001 + r.integers(-9, 10, n)).astype(dtype)
+    for mode in (0, 2) if n < 1 << 20 else (2,):
+        want = oracle.compress(x, 0.5, mode, dim, dims, nthreads=oracle.max_threads())
+        assert gpu_compress(x, 0.5, mode, dim, dims) == want
+        assert np.array_equal(gpu_decompress(want, n, dtype, 0.5, mode, dim, dims), x)
