@@ -1350,11 +1350,13 @@ constexpr uint64_t kStatusGuard = 64 * kLookbackWords;
 // of the values' bytes, so the pass reads little.
 //
 // The pass is itself one single-pass decoupled-lookback scan, over segments of
-// kPrefixThreads x kPrefixBytes header bytes: thread t of segment s sums the
-// block sizes of header bytes [(s * kPrefixThreads + t) * kPrefixBytes, +kPrefixBytes).
-// Few bytes per thread and many segments: the pass is bound by its latency, not
-// by the read (128 bytes per thread, one by one, took 12.5 us for the 2 MiB
-// header of 512^3 values, this 6.5).
+// one workgroup's threads x kPrefixBytes header bytes: thread t of segment s sums
+// the block sizes of header bytes [(s * threads + t) * kPrefixBytes, +kPrefixBytes).
+// Few bytes per thread: the pass is bound by its latency, not by the read (128
+// bytes per thread, one by one, took 12.5 us for the 2 MiB header of 512^3
+// values, this 6.5). Small workgroups start and publish sooner, large ones make
+// fewer segments to look back over: a header of 32 MiB
+// (4 GiB of f32) took 36 us with 256 threads per workgroup, 23 with 1024.
 // ---------------------------------------------------------------------------
 // Longest header whose sums every workgroup takes by itself (single arrays,
 // arrays of a batch). The sums cost the number of tiles times the length, the
@@ -1363,9 +1365,9 @@ constexpr uint64_t kStatusGuard = 64 * kLookbackWords;
 // 128 KiB 11.5 against 13.0, 256 KiB 20.0 either way, 512 KiB 46.6 against 32.3.
 constexpr uint64_t kDirectHeader = 256 << 10;
 constexpr uint64_t kBatchDirectHeader = 16 << 10;
-constexpr int kPrefixThreads = 256;
+__host__ __device__ constexpr int prefix_threads(uint64_t header) { return header >= (4ull << 20) ? 1024 : 256; }
 constexpr int kPrefixBytes = 32;
-constexpr uint64_t kPrefixSegBytes = (uint64_t)kPrefixThreads * kPrefixBytes;
+__host__ __device__ constexpr uint64_t prefix_seg_bytes(int threads) { return (uint64_t)threads * kPrefixBytes; }
 
 // Payload bytes of the header bytes [b0, b0 + kPrefixBytes); bytes at or past
 // `limit` (2D/3D: the block count, so header pad bytes count nothing) are
@@ -1399,11 +1401,12 @@ __device__ __forceinline__ uint32_t thread_bytes(const uint8_t* __restrict__ cmp
 
 // Payload bytes of segment `seg`, by one wave (a waiting wave's recomputation
 // of a predecessor it claimed; see wave_lookback).
-template <int MODE, int S>
+template <int MODE, int S, int THREADS>
 __device__ uint64_t segment_bytes(const uint8_t* __restrict__ cmp, uint64_t limit, uint64_t seg, int lane) {
     uint64_t sum = 0;
-    for (uint32_t i = (uint32_t)lane; i < kPrefixSegBytes; i += kWaveSize) {
-        const uint64_t b = seg * kPrefixSegBytes + i;
+    constexpr uint32_t n = prefix_seg_bytes(THREADS);
+    for (uint32_t i = (uint32_t)lane; i < n; i += kWaveSize) {
+        const uint64_t b = seg * n + i;
         sum += view_of<MODE, S>(b < limit ? (uint32_t)cmp[b] : 0u).size;
     }
     return wave_sum_u40(sum);
@@ -1412,21 +1415,21 @@ __device__ uint64_t segment_bytes(const uint8_t* __restrict__ cmp, uint64_t limi
 // offs[u] = H + payload bytes of units 0 .. u-1, for u < nunits; segment =
 // base + blockIdx.x of nseg. With `total`, the last segment writes the stream
 // length the header describes, H + all payload bytes.
-template <int MODE, int S, int UB>
-__global__ void __launch_bounds__(kPrefixThreads)
+template <int MODE, int S, int UB, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const uint64_t H, const uint64_t nunits,
                     unsigned long long* __restrict__ offs, unsigned long long* __restrict__ total,
                     const ScanCtx sc, const uint64_t nseg, const uint64_t base) {
-    static_assert(UB % kPrefixBytes == 0 && kPrefixSegBytes % UB == 0, "units of whole threads in segments of whole units");
-    constexpr int NW = kPrefixThreads / kWaveSize;
+    static_assert(UB % kPrefixBytes == 0 && prefix_seg_bytes(THREADS) % UB == 0, "units of whole threads in segments of whole units");
+    constexpr int NW = THREADS / kWaveSize;
     __shared__ uint32_t wsum[NW];
     __shared__ uint64_t excl;
     const uint64_t seg = base + blockIdx.x;
     const int t = (int)threadIdx.x, lane = (int)__lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint64_t th = seg * kPrefixThreads + (uint64_t)t;
+    const uint64_t th = seg * THREADS + (uint64_t)t;
     const uint32_t tot = thread_bytes<MODE, S>(cmp, th * kPrefixBytes, limit);
-    const uint32_t incl = scan_wave(tot);   // < 2^32: a segment holds 2^13 blocks of <= 2 KiB
+    const uint32_t incl = scan_wave(tot);   // < 2^32: a segment holds at most 2^15 blocks of <= 2 KiB
     if (lane == kWaveSize - 1) wsum[wave] = incl;
     // wave 0's first lookback read overlaps the other waves' sums
     LookbackWindow<kLookbackWords> pre = {};
@@ -1441,7 +1444,7 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
     }
     if (wave == 0) {
         const uint64_t e = wave_lookback<kLookbackWords>(sc, seg, 0, stot, lane, [&](uint64_t p) {
-            return segment_bytes<MODE, S>(cmp, limit, p, lane);
+            return segment_bytes<MODE, S, THREADS>(cmp, limit, p, lane);
         }, pre, true);
         if (lane == 0) {
             excl = e;

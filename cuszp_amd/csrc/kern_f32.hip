@@ -21,9 +21,10 @@ template <int M, int S, int UB>
 static hipError_t launch_o(const Item& item, uint64_t nunits, unsigned long long* offs, const ScanCtx& sc,
                            hipStream_t st) {
     const uint64_t limit = S == 4 ? item.geo.H : item.geo.nblocks;   // 2D/3D header pad bytes hold no block
-    const uint64_t nseg = (nunits * UB + kPrefixSegBytes - 1) / kPrefixSegBytes;
-    return launch_tiles(unit_offsets_kernel<M, S, UB>, kPrefixThreads, nseg, st, (const uint8_t*)item.src, limit,
-                        item.geo.H, nunits, offs, (unsigned long long*)nullptr, sc, nseg);
+    const int threads = prefix_threads(nunits * UB);
+    const uint64_t seg = prefix_seg_bytes(threads), nseg = (nunits * UB + seg - 1) / seg;
+    return launch_tiles(threads == 256 ? unit_offsets_kernel<M, S, UB, 256> : unit_offsets_kernel<M, S, UB, 1024>, threads, nseg,
+                        st, (const uint8_t*)item.src, limit, item.geo.H, nunits, offs, (unsigned long long*)nullptr, sc, nseg);
 }
 
 #include "dispatch.inc"

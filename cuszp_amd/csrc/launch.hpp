@@ -32,7 +32,7 @@ hipError_t launch_decompress_f64(int dim, int mode, int waves, const Item& item,
 // Offset table of a single-array decompression (unit_offsets_kernel): offs[u]
 // for the nunits decode waves of `item`'s plan, from the header bytes of the
 // stream at item.src; sc's status words serve the pass's own scan (one per
-// segment of kPrefixSegBytes header bytes).
+// segment of prefix_seg_bytes header bytes).
 hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
                                    const ScanCtx& sc, hipStream_t st);
 hipError_t launch_unit_offsets_f64(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
@@ -41,7 +41,8 @@ hipError_t launch_unit_offsets_f64(int dim, int mode, const Item& item, uint64_t
 inline uint64_t unit_blocks(int dim, bool f64, int kc = 0) { return tile_groups(f64, 1, kc) * (dim == 1 ? 2 : 1); }
 // Segments of the offset pass over `nunits` units.
 inline uint64_t unit_segments(int dim, bool f64, uint64_t nunits) {
-    return (nunits * unit_blocks(dim, f64) + kPrefixSegBytes - 1) / kPrefixSegBytes;
+    const uint64_t header = nunits * unit_blocks(dim, f64), seg = prefix_seg_bytes(prefix_threads(header));
+    return (header + seg - 1) / seg;
 }
 
 // Batched launches over a device table of items (ordered by tile0), one
