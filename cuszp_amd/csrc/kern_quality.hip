@@ -46,9 +46,10 @@ __device__ __forceinline__ Moments merge(const Moments& a, const Moments& b) {
     const double eo = b.mo - a.mo, ed = b.md - a.md, w = a.n * f;
     r.mo = a.mo + eo * f;
     r.md = a.md + ed * f;
-    r.oo = a.oo + b.oo + eo * eo * w;
-    r.dd = a.dd + b.dd + ed * ed * w;
-    r.od = a.od + b.od + eo * ed * w;
+    // w first: it is 0 where either set is empty, and a distance (then a mean) may square to infinity
+    r.oo = a.oo + b.oo + eo * w * eo;
+    r.dd = a.dd + b.dd + ed * w * ed;
+    r.od = a.od + b.od + eo * w * ed;
     return r;
 }
 
