@@ -297,6 +297,43 @@ __device__ __forceinline__ WinStats<T> window_of(const WinStats<T> (&p)[3], cons
     return r;
 }
 
+// A window by itself, from its 343 pairs (at: the first one's index): the means, then centred sums.
+template <class T>
+__device__ __forceinline__ WinStats<T> window_at(const T* __restrict__ x, const T* __restrict__ y, uint64_t s0, uint64_t s1,
+                                                 uint64_t at) {
+    constexpr double np = kWin * kWin * kWin;
+    WinStats<T> r = {0, 0, 0, 0, 0, x[at], x[at]};
+    auto rows = [&](auto&& take) {
+#pragma unroll 1
+        for (int j = 0; j < kWin * kWin; ++j) {
+            const uint64_t b = at + s0 * ((uint64_t)(j % kWin) + s1 * (uint64_t)(j / kWin));
+#pragma unroll
+            for (int i = 0; i < kWin; ++i) take(x[b + i], y[b + i]);
+        }
+    };
+    rows([&](T a, T c) {
+        r.lo = min_of(r.lo, a);
+        r.hi = most_of(r.hi, a);
+        r.x += (double)a;
+        r.y += (double)c;
+    });
+    const double mx = r.x / np, my = r.y / np;
+    rows([&](T a, T c) {
+        const double u = (double)a - mx, v = (double)c - my;
+        r.xx = fma(u, u, r.xx);
+        r.yy = fma(v, v, r.yy);
+        r.xy = fma(u, v, r.xy);
+    });
+    return r;
+}
+// Whether a window's values are finite but its centred sums are not: the squares of
+// distances between sums of up to 98 values leave double's range before
+// those of the values do (f64 deviations of 1e152 and more).
+template <class T>
+__device__ __forceinline__ bool overflown(const WinStats<T>& s) {
+    return sizeof(T) == 8 && !(s.xx + s.yy + fabs(s.xy) < INFINITY) && fabs(s.x) < INFINITY && fabs(s.y) < INFINITY;
+}
+
 template <class T>
 __device__ __forceinline__ double ssim_of(const WinStats<T>& s) {
     constexpr double np = kWin * kWin * kWin;
@@ -475,7 +512,13 @@ __global__ void __launch_bounds__(kThreads, kSsimPerCu<T>) ssim_kernel(const T* 
         for (uint64_t l = 0; l < layers + 3; ++l) {
             const bool last = l == layers + 2;
             const WinStats<T> d = slice(!last);
-            if (l >= 3 && mine) total += ssim_of(window_of(ring, d));
+            if (l >= 3 && mine) {
+                WinStats<T> w = window_of(ring, d);
+                if (overflown(w))
+                    w = window_at(x, y, p.s0, p.s1,
+                                  (kWinStep * (wz0 + l - 3) * p.s1 + kWinStep * (wy0 + ty)) * p.s0 + kWinStep * (wx0 + tx));
+                total += ssim_of(w);
+            }
             if (last) break;
             ring[0] = ring[1];
             ring[1] = ring[2];

@@ -26,3 +26,23 @@ def test_figures_far_means(device, oracle, mean, n):
         assert got[k] == want[k], k
     for k in ("mse", "nrmse", "correlation"):
         assert np.isfinite(want[k]) and got[k] == pytest.approx(want[k], rel=1e-9), k
+
+
+@pytest.mark.parametrize("scale", [1e-150, 1e150, 3e151, 3e152, 6e152])
+@pytest.mark.parametrize("offset", [0.0, 1.0])
+@pytest.mark.parametrize("dims", [(7, 7, 7), (40, 19, 13), (9, 70, 11)])
+def test_ssim_far_deviations(device, oracle, scale, offset, dims):
+    """Deviations whose own squares sum to less than double's largest value, while
+    those of sums of many of them do not; the same tolerance as near 1."""
+    import torch
+    from cuszp_amd import pycuSZp as P
+
+    r = np.random.default_rng(11)
+    n = dims[0] * dims[1] * dims[2]
+    x = (r.uniform(-1.7, 1.7, n) + offset) * scale
+    y = x * (1 + 0.05 * r.uniform(-1.7, 1.7, n))
+    want = oracle.ssim(x, y, dims)
+    assert np.isfinite(want)
+    assert P.ssim(torch.from_numpy(x).to(device), torch.from_numpy(y).to(device), dims) == pytest.approx(want, rel=1e-9)
+    x[n // 2] = np.inf   # no window's values by themselves
+    assert np.isnan(P.ssim(torch.from_numpy(x).to(device), torch.from_numpy(y).to(device), dims)) == np.isnan(oracle.ssim(x, y, dims))
