@@ -297,35 +297,6 @@ __device__ __forceinline__ WinStats<T> window_of(const WinStats<T> (&p)[3], cons
     return r;
 }
 
-// A window by itself, from its 343 pairs (at: the first one's index): the means, then centred sums.
-template <class T>
-__device__ __forceinline__ WinStats<T> window_at(const T* __restrict__ x, const T* __restrict__ y, uint64_t s0, uint64_t s1,
-                                                 uint64_t at) {
-    constexpr double np = kWin * kWin * kWin;
-    WinStats<T> r = {0, 0, 0, 0, 0, x[at], x[at]};
-    auto rows = [&](auto&& take) {
-#pragma unroll 1
-        for (int j = 0; j < kWin * kWin; ++j) {
-            const uint64_t b = at + s0 * ((uint64_t)(j % kWin) + s1 * (uint64_t)(j / kWin));
-#pragma unroll
-            for (int i = 0; i < kWin; ++i) take(x[b + i], y[b + i]);
-        }
-    };
-    rows([&](T a, T c) {
-        r.lo = min_of(r.lo, a);
-        r.hi = most_of(r.hi, a);
-        r.x += (double)a;
-        r.y += (double)c;
-    });
-    const double mx = r.x / np, my = r.y / np;
-    rows([&](T a, T c) {
-        const double u = (double)a - mx, v = (double)c - my;
-        r.xx = fma(u, u, r.xx);
-        r.yy = fma(v, v, r.yy);
-        r.xy = fma(u, v, r.xy);
-    });
-    return r;
-}
 // Whether a window's values are finite but its centred sums are not: the squares of
 // distances between sums of up to 98 values leave double's range before
 // those of the values do (f64 deviations of 1e152 and more).
@@ -358,6 +329,50 @@ __device__ __forceinline__ double ssim_of(const WinStats<T>& s) {
     return lum * ((2 * sx * sy + c2) / (sx * sx + sy * sy + c2)) * ((vxy + c3) / (sx * sy + c3));
 }
 
+// The SSIM of the window at (o0, o1, o2) by itself, from its 343 pairs: the means, then centred sums.
+template <class T>
+__device__ double window_ssim(const T* __restrict__ x, const T* __restrict__ y, uint64_t s1, uint64_t s0,
+                              uint64_t o0, uint64_t o1, uint64_t o2) {
+    const uint64_t b = o0 + s0 * (o1 + s1 * o2);
+    T xmin = x[b], xmax = x[b];
+    double xs = 0, ys = 0;
+    // Rows one by one, a whole row of x before that of y: lanes' rows lie far apart in the volumes
+    // that come here, and what one row's loads bring to the L1 is used before the next one's
+    // (f64 7 x 9 x 60005 117 us with the two rows' loads mixed, 97 this way).
+    auto rows = [&](auto&& take) {
+#pragma unroll 1
+        for (int k = 0; k < kWin; ++k)
+#pragma unroll 1
+            for (int j = 0; j < kWin; ++j) {
+                const uint64_t r = b + s0 * ((uint64_t)j + s1 * (uint64_t)k);
+                T a[kWin], c[kWin];
+#pragma unroll
+                for (int i = 0; i < kWin; ++i) a[i] = x[r + i];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kWin; ++i) c[i] = y[r + i];
+#pragma unroll
+                for (int i = 0; i < kWin; ++i) take(a[i], c[i]);
+            }
+    };
+    rows([&](T a, T c) {
+        xmin = a < xmin ? a : xmin;
+        xmax = a > xmax ? a : xmax;
+        xs += (double)a;
+        ys += (double)c;
+    });
+    constexpr double np = kWin * kWin * kWin;
+    const double mx = xs / np, my = ys / np;
+    double vx = 0, vy = 0, vxy = 0;
+    rows([&](T o, T d) {
+        const double a = (double)o - mx, c = (double)d - my;
+        vx += a * a;
+        vy += c * c;
+        vxy += a * c;
+    });
+    return ssim_of(WinStats<T>{xs, ys, vx, vy, vxy, xmin, xmax});
+}
+
 // Windows of a volume, tiled: TX x TY windows of a tile along x and y, `depth`
 // layers of windows along z.
 struct SsimPlan {
@@ -372,6 +387,43 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The mean of all threads' totals over n, to res (sm: a double per wave; lost: set to false before).
+__device__ __forceinline__ void grid_mean(double total, double n, double* sm, bool& lost, const cuszp::GridWords& gw, double* res) {
+    const int tid = (int)threadIdx.x;
+    auto block_sum = [&](double v) -> double {   // in thread 0
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        __syncthreads();
+        if ((tid & 63) == 0) sm[tid >> 6] = v;
+        __syncthreads();
+        double t = 0;
+        for (int j = 0; j < kThreads / 64; ++j) t += sm[j];
+        return t;
+    };
+    typedef cuszp::Words<double> W;
+    total = block_sum(total);
+    if (blockIdx.x != gridDim.x - 1) {
+        if (tid == 0) {
+            const W w = W::of(total);
+            gw.put((uint64_t)blockIdx.x * 2, w.u[0]);
+            gw.put((uint64_t)blockIdx.x * 2 + 1, w.u[1]);
+        }
+        return;
+    }
+    if (tid != 0) total = 0;
+    bool ok = true;
+    for (unsigned b = threadIdx.x; b + 1 < gridDim.x; b += kThreads) {
+        W w;
+        ok &= gw.get_n((uint64_t)b * 2, w.u);
+        total += w.value();
+    }
+    if (!ok) lost = true;
+    total = block_sum(total);
+    if (tid == 0) {
+        cuszp::host_store(res, total / n);
+        cuszp::host_store(res + cuszp::kGridResults - 1, lost ? 1.0 : 0.0);
+    }
 }
 
 // Workgroups per CU that the kernel is built for (registers, and LDS of 44 or 61 KB).
@@ -513,11 +565,11 @@ __global__ void __launch_bounds__(kThreads, kSsimPerCu<T>) ssim_kernel(const T* 
             const bool last = l == layers + 2;
             const WinStats<T> d = slice(!last);
             if (l >= 3 && mine) {
-                WinStats<T> w = window_of(ring, d);
+                const WinStats<T> w = window_of(ring, d);
                 if (overflown(w))
-                    w = window_at(x, y, p.s0, p.s1,
-                                  (kWinStep * (wz0 + l - 3) * p.s1 + kWinStep * (wy0 + ty)) * p.s0 + kWinStep * (wx0 + tx));
-                total += ssim_of(w);
+                    total += window_ssim(x, y, p.s1, p.s0, kWinStep * (wx0 + tx), kWinStep * (wy0 + ty), kWinStep * (wz0 + l - 3));
+                else
+                    total += ssim_of(w);
             }
             if (last) break;
             ring[0] = ring[1];
@@ -525,38 +577,25 @@ __global__ void __launch_bounds__(kThreads, kSsimPerCu<T>) ssim_kernel(const T* 
             ring[2] = pair_of(d, slice(true));
         }
     }
-    auto block_sum = [&](double v) -> double {   // in thread 0
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        __syncthreads();
-        if ((tid & 63) == 0) sm[tid >> 6] = v;
-        __syncthreads();
-        double t = 0;
-        for (int j = 0; j < kThreads / 64; ++j) t += sm[j];
-        return t;
-    };
-    typedef cuszp::Words<double> W;
-    total = block_sum(total);
-    if (blockIdx.x != gridDim.x - 1) {
-        if (tid == 0) {
-            const W w = W::of(total);
-            gw.put((uint64_t)blockIdx.x * 2, w.u[0]);
-            gw.put((uint64_t)blockIdx.x * 2 + 1, w.u[1]);
-        }
-        return;
+    grid_mean(total, (double)(p.nw0 * p.nw1 * p.nw2), sm, lost, gw, res);
+}
+
+// One thread per window: every window reads its own pairs, twice. For volumes
+// of few windows along two axes, most of whose tiles' lanes would have no window
+// (window_by_window).
+template <class T>
+__global__ void __launch_bounds__(kThreads) windows_kernel(const T* __restrict__ x, const T* __restrict__ y, const SsimPlan p,
+                                                           const cuszp::GridWords gw, double* res) {
+    __shared__ double sm[kThreads / 64];
+    __shared__ bool lost;
+    if (threadIdx.x == 0) lost = false;
+    const uint64_t n = p.nw0 * p.nw1 * p.nw2;
+    double total = 0;
+    for (uint64_t w = (uint64_t)blockIdx.x * kThreads + threadIdx.x; w < n; w += (uint64_t)gridDim.x * kThreads) {
+        const uint64_t w0 = w % p.nw0, w1 = (w / p.nw0) % p.nw1, w2 = w / (p.nw0 * p.nw1);
+        total += window_ssim(x, y, p.s1, p.s0, w0 * kWinStep, w1 * kWinStep, w2 * kWinStep);
     }
-    if (tid != 0) total = 0;
-    bool ok = true;
-    for (unsigned b = threadIdx.x; b + 1 < gridDim.x; b += kThreads) {
-        W w;
-        ok &= gw.get_n((uint64_t)b * 2, w.u);
-        total += w.value();
-    }
-    if (!ok) lost = true;
-    total = block_sum(total);
-    if (tid == 0) {
-        cuszp::host_store(res, total / (double)(p.nw0 * p.nw1 * p.nw2));
-        cuszp::host_store(res + cuszp::kGridResults - 1, lost ? 1.0 : 0.0);
-    }
+    grid_mean(total, (double)n, sm, lost, gw, res);
 }
 
 struct State {
@@ -612,6 +651,19 @@ int run(const T* ori, const T* dec, size_t n, double* out, hipStream_t st) {
     return CUSZP_SUCCESS;
 }
 
+// Whether a volume of n windows, nw0 along x, is faster with a thread per window than with
+// tiles, whose workgroups go through `slices` slices in a row. A slice takes about 3 us once
+// every CU has its workgroups, whatever share of their lanes has windows; a thread per window
+// 30-50 us in all while the chip is not full, then 0.3 ns a window (f64 0.6), and more where
+// there is one window along x and lanes read rows far apart. us a call, tiles and thread per
+// window: f32 7 x 7 x 60005 298 and 62, 13 x 13 x 8755 78 and 50, 13 x 13 x 37505 190 and 111,
+// 600005 x 7 x 7 272 and 116; f64 13 x 13 x 37505 224 and 222, 7 x 21 x 75005 444 and 577.
+template <class T>
+bool window_by_window(uint64_t slices, uint64_t n, uint64_t nw0) {
+    constexpr uint64_t kPerSlice = sizeof(T) == 4 ? 9000 : 3900, kPerSliceFar = sizeof(T) == 4 ? 6000 : 1560;
+    return slices > 9 + (n <= 65536 ? 0 : n / (nw0 > 1 ? kPerSlice : kPerSliceFar));
+}
+
 template <class T>
 int run_ssim(const T* x, const T* y, cuszp_dims_t d, double* out, hipStream_t st) {
     if (d.x < (unsigned)kWin || d.y < (unsigned)kWin || d.z < (unsigned)kWin) return CUSZP_ERROR_INVALID_DIMS;
@@ -638,9 +690,10 @@ int run_ssim(const T* x, const T* y, cuszp_dims_t d, double* out, hipStream_t st
     // less work, but the chip works on kResident tiles at a time and the last
     // round should be full: the depth with the fewest slices in a row.
     constexpr uint64_t kResident = 256 * kSsimPerCu<T>;
-    uint64_t best = ~0ull;
-    for (uint64_t chunks = 1; chunks <= p.nw2 && chunks <= 4 * kResident; ++chunks) {
-        const uint64_t depth = (p.nw2 + chunks - 1) / chunks, tiles = p.t0 * p.t1 * ((p.nw2 + depth - 1) / depth);
+    uint64_t best = ~0ull, depth;
+    for (uint64_t chunks = 1; chunks <= p.nw2 && chunks <= 4 * kResident; chunks = depth > 1 ? (p.nw2 + depth - 2) / (depth - 1) : ~0ull) {
+        depth = (p.nw2 + chunks - 1) / chunks;   // and on to the fewest chunks that are less deep
+        const uint64_t tiles = p.t0 * p.t1 * ((p.nw2 + depth - 1) / depth);
         const uint64_t cost = (tiles + kResident - 1) / kResident * (kWinStep * depth + kWin - kWinStep);
         if (cost < best) {
             best = cost;
@@ -649,8 +702,16 @@ int run_ssim(const T* x, const T* y, cuszp_dims_t d, double* out, hipStream_t st
         }
         if (tiles > 4 * kResident) break;   // only more work from here on
     }
-    const unsigned blocks = p.tiles < kMaxSsimBlocks ? (unsigned)p.tiles : kMaxSsimBlocks;
-    if (narrow)
+    const uint64_t n = p.nw0 * p.nw1 * p.nw2;
+    const bool single = window_by_window<T>(best, n, p.nw0);
+    const uint64_t work = single ? (n + kThreads - 1) / kThreads : p.tiles;
+    // A thread per window: two or four workgroups per CU. Where lanes read rows far apart (f64, or one window
+    // along x) more of them only push each other's lines out of the L1: f32 7 x 9 x 2000005 3047 us with
+    // four, 2100 with two; 4000005 x 7 x 7 628 with four, 960 with two.
+    const unsigned cap = !single ? kMaxSsimBlocks : (sizeof(T) == 8 || p.nw0 == 1 ? 512 : 1024), blocks = work < cap ? (unsigned)work : cap;
+    if (single)
+        hipLaunchKernelGGL(windows_kernel<T>, dim3(blocks), dim3(kThreads), 0, st, x, y, p, gw, s.g.h_res);
+    else if (narrow)
         hipLaunchKernelGGL((ssim_kernel<T, 8>), dim3(blocks), dim3(kThreads), 0, st, x, y, p, gw, s.g.h_res);
     else
         hipLaunchKernelGGL((ssim_kernel<T, 32>), dim3(blocks), dim3(kThreads), 0, st, x, y, p, gw, s.g.h_res);
