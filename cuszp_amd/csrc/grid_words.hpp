@@ -27,29 +27,24 @@ struct GridWords {
     __device__ __forceinline__ void put(uint64_t i, uint32_t v) const {
         __hip_atomic_store(w + i, ((unsigned long long)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    // Word i's value; false if it did not arrive within the bound.
-    __device__ __forceinline__ bool get(uint64_t i, uint32_t& v) const {
-        for (uint32_t k = 0; k < kWordPolls; ++k) {
-            const unsigned long long x = __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            v = (uint32_t)x;
-            if ((uint32_t)(x >> 32) == tag) return true;
+    // N words from word i on, `stride` apart, their loads in flight together, until all of them
+    // carry the tag; false if they did not within the bound.
+    template <int N>
+    __device__ __forceinline__ bool get_n(uint64_t i, uint32_t (&v)[N], uint64_t stride = 1) const {
+        for (uint32_t p = 0; p < kWordPolls; ++p) {
+            unsigned long long x[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) x[k] = __hip_atomic_load(w + i + k * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bool ok = true;
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                v[k] = (uint32_t)x[k];
+                ok &= (uint32_t)(x[k] >> 32) == tag;
+            }
+            if (ok) return true;
             __builtin_amdgcn_s_sleep(1);
         }
         return false;
-    }
-    // N words from word i on, `stride` apart, their loads in flight together; the few that are not there yet are polled.
-    template <int N>
-    __device__ __forceinline__ bool get_n(uint64_t i, uint32_t (&v)[N], uint64_t stride = 1) const {
-        unsigned long long x[N];
-#pragma unroll
-        for (int k = 0; k < N; ++k) x[k] = __hip_atomic_load(w + i + k * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bool ok = true;
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            v[k] = (uint32_t)x[k];
-            if ((uint32_t)(x[k] >> 32) != tag) ok &= get(i + k * stride, v[k]);
-        }
-        return ok;
     }
 };
 
