@@ -179,7 +179,7 @@ TilePlan plan_tiles(int dim, int type, const Geom& g) {
     // (8, 4). Powers of two only: whole tiles fill a 1D header.
     if (!waves)
         for (waves = 4, kc = 1; waves != 8 || kc < full;) {
-            if (groups <= tile_groups(f64, waves, kc) * (waves == 4 ? 256 : 384)) break;
+            if (groups <= tile_groups(f64, waves, kc) * shape_tiles(waves)) break;
             if (waves == 4 && kc == 2) waves = 8;
             else kc *= 2;
         }

@@ -96,7 +96,7 @@ void choose_shape(cuszp_batch_plan_s& p) {
             make_geom(s.dim, s.nbEle, s.dims, g);
             if (s.nbEle) n += tiles(s, g, p.waves, p.kc);
         }
-        if (n <= (p.waves == 4 ? 256u : 384u)) return;
+        if (n <= shape_tiles(p.waves)) return;
     }
 }
 

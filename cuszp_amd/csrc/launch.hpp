@@ -18,6 +18,8 @@ struct TilePlan {
     uint64_t ntiles;
 };
 TilePlan plan_tiles(int dim, int type, const Geom& g);
+// Tiles up to which a shape short of the largest is taken, by its waves.
+constexpr uint64_t shape_tiles(int waves) { return waves == 4 ? 256 : 384; }
 
 // Single-array launches; item.param is 0.5/eb (compress) or eb (decompress).
 hipError_t launch_compress_f32(int dim, int mode, int waves, const Item& item, const ScanCtx& sc, hipStream_t st);
@@ -38,7 +40,14 @@ hipError_t launch_unit_offsets_f32(int dim, int mode, const Item& item, uint64_t
 hipError_t launch_unit_offsets_f64(int dim, int mode, const Item& item, uint64_t nunits, unsigned long long* offs,
                                    const ScanCtx& sc, hipStream_t st);
 // Blocks one decode wave handles.
-inline uint64_t unit_blocks(int dim, bool f64, int kc = 0) { return tile_groups(f64, 1, kc) * (dim == 1 ? 2 : 1); }
+constexpr uint64_t unit_blocks(int dim, bool f64, int kc = 0) { return tile_groups(f64, 1, kc) * (dim == 1 ? 2 : 1); }
+// The pass of a single array takes every wave for a full one (unit_blocks without kc,
+// the kernels' UB). It runs for headers above kDirectHeader only, and those make more
+// groups (1D two blocks each) than the longest array of a shorter shape has.
+constexpr bool pass_takes_full_tiles(bool f64) {
+    return kDirectHeader / 2 >= tile_groups(f64, 8, (f64 ? kChunksOf<double> : kChunksOf<float>) / 2) * shape_tiles(8);
+}
+static_assert(pass_takes_full_tiles(false) && pass_takes_full_tiles(true), "the offset pass needs full tiles");
 // Segments of the offset pass over `nunits` units.
 inline uint64_t unit_segments(int dim, bool f64, uint64_t nunits) {
     const uint64_t header = nunits * unit_blocks(dim, f64), seg = prefix_seg_bytes(prefix_threads(header));
@@ -64,6 +73,8 @@ hipError_t launch_decompress_batch8(const Item* items, uint32_t nitems, uint64_t
 // each), whose waves have whole threads' header bytes (unit_blocks % kPrefixBytes == 0).
 hipError_t launch_offsets_batch(int waves, const Item* items, uint32_t nitems, uint64_t nseg, unsigned long long* offs,
                                 const ScanCtx& sc, const unsigned long long* epoch, hipStream_t st);
+static_assert(unit_blocks(2, false, 4) % kPrefixBytes == 0 && unit_blocks(2, true, 4) % kPrefixBytes == 0,
+              "4 chunks per wave, the fewest under a pass, are whole threads' header bytes");
 inline uint64_t batch_segments(int dim, bool f64, int kc, uint64_t nunits) {
     return (nunits * unit_blocks(dim, f64, kc) + kBatchSegBytes - 1) / kBatchSegBytes;
 }
