@@ -34,6 +34,7 @@ struct cuszp_batch_plan_s {
     std::vector<Item> items;      // non-empty arrays, in caller order
     uint64_t ntiles = 0;
     uint64_t nseg = 0;            // decompress: segments of the offset pass, 0 without it
+    bool epoch_used = false;            // an offset pass took the epoch and the decode kernel that advances it was not launched
     Item* d_items = nullptr;
     size_t cap_items = 0;
     unsigned long long* d_status = nullptr;
@@ -161,13 +162,23 @@ int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
     BATCH_HIP(hipMemsetAsync(p.d_status, 0, (kStatusGuard + p.cap_status) * sizeof(unsigned long long), st));
     BATCH_HIP(hipMemsetAsync(p.d_misc, 0, sizeof(unsigned long long), st));
     if (p.nseg) BATCH_HIP(launch_bump_epoch(p.d_misc, st));   // the next pass's; then the decompress kernel advances it
+    p.epoch_used = false;
     if (!p.items.empty())
         BATCH_HIP(hipMemcpyAsync(p.d_items, p.items.data(), p.items.size() * sizeof(Item), hipMemcpyHostToDevice, st));
     BATCH_HIP(hipStreamSynchronize(st));   // the host table may be rebuilt right after
     return CUSZP_SUCCESS;
 }
 
-int enqueue(const cuszp_batch_plan_s& p, hipStream_t st) {
+// A new epoch where the last one was used up by a call that failed halfway: the
+// next pass would take that call's status words for its own.
+int renew_epoch(cuszp_batch_plan_s& p, hipStream_t st) {
+    if (!p.epoch_used) return CUSZP_SUCCESS;
+    BATCH_HIP(launch_bump_epoch(p.d_misc, st));
+    p.epoch_used = false;
+    return CUSZP_SUCCESS;
+}
+
+int enqueue(cuszp_batch_plan_s& p, hipStream_t st) {
     if (p.items.empty()) return CUSZP_SUCCESS;
     // the kernels read the epoch word for the tag
     const ScanCtx sc = make_scan_ctx(p.d_status + kStatusGuard, (unsigned int*)(p.d_misc + kMiscErr),
@@ -178,9 +189,15 @@ int enqueue(const cuszp_batch_plan_s& p, hipStream_t st) {
         BATCH_HIP(launch_compress_batch(p.waves, p.window, p.d_items, n, p.ntiles, sc, p.d_misc, st));
         return CUSZP_SUCCESS;
     }
-    if (p.nseg) BATCH_HIP(launch_offsets_batch(p.waves, p.d_items, n, p.nseg, p.d_offs, sc, p.d_misc, st));
+    if (p.nseg) {
+        const int rc = renew_epoch(p, st);
+        if (rc) return rc;
+        p.epoch_used = true;
+        BATCH_HIP(launch_offsets_batch(p.waves, p.d_items, n, p.nseg, p.d_offs, sc, p.d_misc, st));
+    }
     BATCH_HIP(launch_decompress_batch(p.waves, p.d_items, n, p.ntiles, p.nseg ? p.d_offs : nullptr,
                                       p.nseg ? p.d_misc : nullptr, st));
+    p.epoch_used = false;
     return CUSZP_SUCCESS;
 }
 
@@ -287,7 +304,11 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
 int cuSZp_batch_plan_execute(cuszp_batch_plan_t p, hipStream_t stream) {
     if (!p) return CUSZP_ERROR_INVALID_ARGUMENT;
     if (p->exec) {
+        const int rc = renew_epoch(*p, stream);
+        if (rc) return rc;
+        p->epoch_used = p->nseg != 0;   // until the launch has succeeded
         BATCH_HIP(hipGraphLaunch(p->exec, stream));
+        p->epoch_used = false;
         return CUSZP_SUCCESS;
     }
     return enqueue(*p, stream);

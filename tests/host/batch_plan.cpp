@@ -1,0 +1,117 @@
+// Host program for the batched plans: cuszp_batch.cpp over a HIP runtime and kernel
+// launches that are replaced here by host memory and a log. It shows what the
+// plan launches when a launch or an allocation fails, which needs no GPU.
+//   batch_plan epoch   a decode launch that fails after its offset pass
+//   batch_plan tune    allocations that fail while shapes are tried
+#include "../../cuszp_amd/csrc/cuszp_batch.cpp"
+
+#include <cstdlib>
+#include <string>
+
+namespace {
+std::vector<std::string> g_log;      // one entry per launch
+std::vector<unsigned long long> g_pass_epochs;
+int g_fail_decodes = 0;              // decode launches that fail
+bool g_null = false;                 // a launch was given no buffer
+int g_graphs = 0, g_captured = 0;
+
+#define CHECK(x)                                                    \
+    do {                                                            \
+        if (!(x)) {                                                 \
+            std::printf("line %d: %s\n", __LINE__, #x);             \
+            std::exit(1);                                           \
+        }                                                           \
+    } while (0)
+
+void seen(const char* what, const void* items, const void* status, const void* offs) {
+    g_log.push_back(what);
+    g_null |= !items || status == (const unsigned long long*)nullptr + kStatusGuard || !offs;
+}
+}  // namespace
+
+// ---- the runtime -----------------------------------------------------------
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) { return *p = std::calloc(n ? n : 1, 1), hipSuccess; }
+hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return std::memset(p, v, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)1, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return *g = (hipGraph_t)1, hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { return ++g_captured, *e = (hipGraphExec_t)1, hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return ++g_graphs, hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = (hipEvent_t)1, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { return *t = 1.0f, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+}
+
+// ---- the launches ----------------------------------------------------------
+namespace cuszp {
+hipError_t launch_bump_epoch(unsigned long long* epoch, hipStream_t) { return ++*epoch, hipSuccess; }
+hipError_t launch_compress_batch(int, int, const Item* items, uint32_t, uint64_t, const ScanCtx& sc, const unsigned long long*, hipStream_t) {
+    return seen("compress", items, sc.status, items), hipSuccess;
+}
+hipError_t launch_offsets_batch(int, const Item* items, uint32_t, uint64_t, unsigned long long* offs, const ScanCtx& sc,
+                                const unsigned long long* epoch, hipStream_t) {
+    g_pass_epochs.push_back(*epoch);
+    return seen("pass", items, sc.status, offs), hipSuccess;
+}
+hipError_t launch_decompress_batch(int, const Item* items, uint32_t, uint64_t, const unsigned long long* offs, unsigned long long* bump,
+                                   hipStream_t) {
+    if (g_fail_decodes && g_fail_decodes--) return hipErrorLaunchFailure;
+    if (bump) ++*bump;
+    return seen("decode", items, items, offs), hipSuccess;
+}
+}  // namespace cuszp
+
+namespace {
+char g_buf[8];   // arrays' addresses are not followed
+
+cuszp_batch_plan_t plan(int dir, int flags = 0) {
+    // 4 Mi values: a header of 128 KiB, long enough for the offset pass
+    cuszp_batch_item_t it{};
+    it.d_in = g_buf;
+    it.d_out = g_buf;
+    it.nbEle = 4u << 20;
+    it.capacity = 1ull << 30;
+    it.errorBound = 1e-3;
+    it.dim = CUSZP_DIM_1D;
+    it.type = CUSZP_TYPE_FLOAT;
+    it.mode = CUSZP_MODE_PLAIN;
+    cuszp_batch_plan_t p = nullptr;
+    CHECK(cuSZp_batch_plan_create(&p, &it, 1, dir, flags, nullptr, nullptr) == CUSZP_SUCCESS);
+    return p;
+}
+
+void epoch() {
+    cuszp_batch_plan_t p = plan(CUSZP_BATCH_DECOMPRESS);
+    CHECK(cuSZp_batch_plan_execute(p, nullptr) == CUSZP_SUCCESS);
+    for (int k = 0; k < 2; ++k) {
+        g_fail_decodes = 1;
+        CHECK(cuSZp_batch_plan_execute(p, nullptr) == CUSZP_ERROR_HIP);
+        CHECK(cuSZp_batch_plan_execute(p, nullptr) == CUSZP_SUCCESS);
+    }
+    CHECK(g_pass_epochs.size() == 5);
+    for (size_t i = 0; i < 5; ++i)
+        for (size_t j = 0; j < i; ++j) CHECK(g_pass_epochs[i] != g_pass_epochs[j]);   // no pass reads another's words as its own
+    cuSZp_batch_plan_destroy(p);
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "epoch") epoch();
+    else return 2;
+    std::puts("ok");
+    return 0;
+}
