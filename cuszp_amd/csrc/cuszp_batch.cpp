@@ -34,6 +34,7 @@ struct cuszp_batch_plan_s {
     std::vector<Item> items;      // non-empty arrays, in caller order
     uint64_t ntiles = 0;
     uint64_t nseg = 0;            // decompress: segments of the offset pass, 0 without it
+    bool built = false;           // the device table, scan state and offsets fit `items`
     bool epoch_used = false;            // an offset pass took the epoch and the decode kernel that advances it was not launched
     Item* d_items = nullptr;
     size_t cap_items = 0;
@@ -104,6 +105,7 @@ void choose_shape(cuszp_batch_plan_s& p) {
 // Lay out the tiles of every non-empty array for the plan's shape and upload the
 // descriptors (grows device buffers as needed).
 int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
+    p.built = false;   // until all of it is there: nothing may be launched on part of it
     p.items.clear();
     uint64_t tile0 = 0, seg0 = 0;
     for (size_t i = 0; i < p.src.size(); ++i) {
@@ -166,6 +168,7 @@ int build_table(cuszp_batch_plan_s& p, hipStream_t st) {
     if (!p.items.empty())
         BATCH_HIP(hipMemcpyAsync(p.d_items, p.items.data(), p.items.size() * sizeof(Item), hipMemcpyHostToDevice, st));
     BATCH_HIP(hipStreamSynchronize(st));   // the host table may be rebuilt right after
+    p.built = true;
     return CUSZP_SUCCESS;
 }
 
@@ -303,6 +306,7 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
 
 int cuSZp_batch_plan_execute(cuszp_batch_plan_t p, hipStream_t stream) {
     if (!p) return CUSZP_ERROR_INVALID_ARGUMENT;
+    if (!p->built) return CUSZP_ERROR_HIP;   // tuning ran out of memory, and so did going back
     if (p->exec) {
         const int rc = renew_epoch(*p, stream);
         if (rc) return rc;
@@ -378,9 +382,13 @@ int cuSZp_batch_plan_scan_report(cuszp_batch_plan_t p, hipStream_t stream, cuszp
     return CUSZP_SUCCESS;
 }
 
-int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_out, unsigned* grid_out) {
-    if (!p) return CUSZP_ERROR_INVALID_ARGUMENT;
-    if (p->items.empty()) return CUSZP_SUCCESS;
+}  // extern "C"
+
+namespace {
+
+// Times the plan in each shape and leaves it in the best one, on record for its size
+// class. A failure leaves it in the shape that failed, perhaps without a table.
+int try_shapes(cuszp_batch_plan_s* p, hipStream_t stream) {
     // (waves, chunks, window): the rule's shape, then full waves; decompress tiles do not look back
     std::vector<std::tuple<int, int, int>> shapes;
     choose_shape(*p);
@@ -424,7 +432,27 @@ int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_o
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tuned[size_class(*p)] = best_shape;
     }
-    if (p->exec || (p->flags & CUSZP_BATCH_GRAPH)) rc = capture(*p);
+    return CUSZP_SUCCESS;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cuSZp_batch_plan_tune(cuszp_batch_plan_t p, hipStream_t stream, int* waves_out, unsigned* grid_out) {
+    if (!p) return CUSZP_ERROR_INVALID_ARGUMENT;
+    if (p->built && p->items.empty()) return CUSZP_SUCCESS;
+    // a graph's kernels hold the present buffers, which a larger shape replaces
+    BATCH_HIP(hipStreamSynchronize(stream));
+    drop_graph(*p);
+    const auto before = std::make_tuple(p->waves, p->kc, p->window);
+    int rc = try_shapes(p, stream);
+    if (rc) {   // back to the shape that worked, with whatever memory there is
+        std::tie(p->waves, p->kc, p->window) = before;
+        if (!build_table(*p, stream) && (p->flags & CUSZP_BATCH_GRAPH)) (void)capture(*p);
+        return rc;
+    }
+    if (p->flags & CUSZP_BATCH_GRAPH) rc = capture(*p);
     // tuning runs leave per-array state from the candidate launches: clear it
     const size_t n = p->src.size() ? p->src.size() : 1;
     if (!rc && hipMemsetAsync(p->d_err, 0, n * sizeof(unsigned int), stream) != hipSuccess) rc = CUSZP_ERROR_HIP;

@@ -2,7 +2,8 @@
 // launches that are replaced here by host memory and a log. It shows what the
 // plan launches when a launch or an allocation fails, which needs no GPU.
 //   batch_plan epoch   a decode launch that fails after its offset pass
-//   batch_plan tune    allocations that fail while shapes are tried
+//   batch_plan tune [graph], tune-lost [graph]
+//                      an allocation that fails while shapes are tried, and again when the former one is restored
 #include "../../cuszp_amd/csrc/cuszp_batch.cpp"
 
 #include <cstdlib>
@@ -77,12 +78,13 @@ hipError_t launch_decompress_batch(int, const Item* items, uint32_t, uint64_t, c
 namespace {
 char g_buf[8];   // arrays' addresses are not followed
 
-cuszp_batch_plan_t plan(int dir, int flags = 0) {
-    // 4 Mi values: a header of 128 KiB, long enough for the offset pass
+// 4 Mi values: a header of 128 KiB, long enough for the offset pass. 16 Mi: 512
+// tiles, of which the shapes of four waves make 1024
+cuszp_batch_plan_t plan(int dir, size_t n = 4u << 20, int flags = 0) {
     cuszp_batch_item_t it{};
     it.d_in = g_buf;
     it.d_out = g_buf;
-    it.nbEle = 4u << 20;
+    it.nbEle = n;
     it.capacity = 1ull << 30;
     it.errorBound = 1e-3;
     it.dim = CUSZP_DIM_1D;
@@ -106,11 +108,38 @@ void epoch() {
         for (size_t j = 0; j < i; ++j) CHECK(g_pass_epochs[i] != g_pass_epochs[j]);   // no pass reads another's words as its own
     cuSZp_batch_plan_destroy(p);
 }
+
+// fails: status arrays that cannot be allocated while the shapes are tried
+void tune(int flags, unsigned fails) {
+    cuszp_batch_plan_t p = plan(CUSZP_BATCH_COMPRESS, 16u << 20, flags);
+    CHECK(cuSZp_batch_plan_execute(p, nullptr) == CUSZP_SUCCESS);
+    failing_allocs().store(fails);
+    CHECK(cuSZp_batch_plan_tune(p, nullptr, nullptr, nullptr) == CUSZP_ERROR_HIP);
+    failing_allocs().store(0);
+    const size_t launches = g_log.size();
+    const int graphs = g_graphs, rc = cuSZp_batch_plan_execute(p, nullptr);
+    CHECK(!g_null);
+    if (fails == 1) {   // the shape from before is there again, and so is its graph
+        CHECK(rc == CUSZP_SUCCESS);
+        CHECK(p->waves == 8 && p->ntiles == 512);
+        CHECK(flags ? g_graphs == graphs + 1 && p->exec : g_log.size() == launches + 1);
+        if (flags) CHECK(g_captured == 2);
+    } else {            // no table: nothing is launched
+        CHECK(rc == CUSZP_ERROR_HIP);
+        CHECK(g_log.size() == launches && g_graphs == graphs);
+    }
+    CHECK(cuSZp_batch_plan_tune(p, nullptr, nullptr, nullptr) == CUSZP_SUCCESS);
+    CHECK(cuSZp_batch_plan_execute(p, nullptr) == CUSZP_SUCCESS);
+    CHECK(!g_null);
+    cuSZp_batch_plan_destroy(p);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "epoch") epoch();
+    else if (what == "tune") tune(argc > 2 ? CUSZP_BATCH_GRAPH : 0, 1);
+    else if (what == "tune-lost") tune(argc > 2 ? CUSZP_BATCH_GRAPH : 0, 2);
     else return 2;
     std::puts("ok");
     return 0;

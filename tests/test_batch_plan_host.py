@@ -26,7 +26,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["epoch"])
+@pytest.mark.parametrize("case", ["epoch", "tune", "tune graph", "tune-lost", "tune-lost graph"])
 def test_plan(program, case):
-    r = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
+    r = subprocess.run([program, *case.split()], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
