@@ -159,7 +159,7 @@ __device__ __forceinline__ uint32_t dpp(uint32_t v) {
         return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, BANKS, false);
 }
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
-constexpr int kDppWaveShr1 = 0x138, kDppRowMirror = 0x140, kDppHalfMirror = 0x141;
+constexpr int kDppWaveShr1 = 0x138, kDppHalfMirror = 0x141;
 constexpr int kDppRowRor8 = 0x128;
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
 constexpr int kDppQuadSwap1 = 0xB1;   // quad_perm [1,0,3,2]
@@ -1413,13 +1413,11 @@ __device__ uint64_t segment_bytes(const uint8_t* __restrict__ cmp, uint64_t limi
 }
 
 // offs[u] = H + payload bytes of units 0 .. u-1, for u < nunits; segment =
-// base + blockIdx.x of nseg. With `total`, the last segment writes the stream
-// length the header describes, H + all payload bytes.
+// base + blockIdx.x.
 template <int MODE, int S, int UB, int THREADS>
 __global__ void __launch_bounds__(THREADS)
 unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const uint64_t H, const uint64_t nunits,
-                    unsigned long long* __restrict__ offs, unsigned long long* __restrict__ total,
-                    const ScanCtx sc, const uint64_t nseg, const uint64_t base) {
+                    unsigned long long* __restrict__ offs, const ScanCtx sc, const uint64_t base) {
     static_assert(UB % kPrefixBytes == 0 && prefix_seg_bytes(THREADS) % UB == 0, "units of whole threads in segments of whole units");
     constexpr int NW = THREADS / kWaveSize;
     __shared__ uint32_t wsum[NW];
@@ -1446,10 +1444,7 @@ unit_offsets_kernel(const uint8_t* __restrict__ cmp, const uint64_t limit, const
         const uint64_t e = wave_lookback<kLookbackWords>(sc, seg, 0, stot, lane, [&](uint64_t p) {
             return segment_bytes<MODE, S, THREADS>(cmp, limit, p, lane);
         }, pre, true);
-        if (lane == 0) {
-            excl = e;
-            if (seg == nseg - 1 && total) *total = H + e + stot;
-        }
+        if (lane == 0) excl = e;
     }
     __syncthreads();
     if (t % (UB / kPrefixBytes) == 0) {   // the unit's first thread

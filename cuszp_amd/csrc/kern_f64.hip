@@ -24,7 +24,7 @@ static hipError_t launch_o(const Item& item, uint64_t nunits, unsigned long long
     const int threads = prefix_threads(nunits * UB);
     const uint64_t seg = prefix_seg_bytes(threads), nseg = (nunits * UB + seg - 1) / seg;
     return launch_tiles(threads == 256 ? unit_offsets_kernel<M, S, UB, 256> : unit_offsets_kernel<M, S, UB, 1024>, threads, nseg,
-                        st, (const uint8_t*)item.src, limit, item.geo.H, nunits, offs, (unsigned long long*)nullptr, sc, nseg);
+                        st, (const uint8_t*)item.src, limit, item.geo.H, nunits, offs, sc);
 }
 
 #include "dispatch.inc"
