@@ -53,35 +53,31 @@ __device__ __forceinline__ Moments merge(const Moments& a, const Moments& b) {
     return r;
 }
 
-// A share's sums (ori, dec, dec^2, err^2), maxima (ori, -ori, err, rel err) and moments.
-constexpr int kFigures = 14;
+// A share's sums (dec^2, err^2), maxima (ori, -ori, err, rel err) and moments.
+constexpr int kFigures = 12;
 struct Figures {
-    double s[4], m[4];
+    double s[2], m[4];
     Moments c;
     __device__ __forceinline__ void init() {
-        for (int k = 0; k < 4; ++k) {
-            s[k] = 0;
-            m[k] = k < 2 ? -INFINITY : 0.0;
-        }
+        for (int k = 0; k < 2; ++k) s[k] = 0;
+        for (int k = 0; k < 4; ++k) m[k] = k < 2 ? -INFINITY : 0.0;
         c = Moments{0, 0, 0, 0, 0, 0};
     }
     __device__ __forceinline__ void add(const Figures& b) {
-        for (int k = 0; k < 4; ++k) {
-            s[k] += b.s[k];
-            m[k] = fmax(m[k], b.m[k]);
-        }
+        for (int k = 0; k < 2; ++k) s[k] += b.s[k];
+        for (int k = 0; k < 4; ++k) m[k] = fmax(m[k], b.m[k]);
         c = merge(c, b.c);
     }
     template <class F>
     __device__ __forceinline__ void each(F&& f) {
-        for (int k = 0; k < 4; ++k) f(k, s[k]);
-        for (int k = 0; k < 4; ++k) f(4 + k, m[k]);
-        f(8, c.n);
-        f(9, c.mo);
-        f(10, c.md);
-        f(11, c.oo);
-        f(12, c.dd);
-        f(13, c.od);
+        for (int k = 0; k < 2; ++k) f(k, s[k]);
+        for (int k = 0; k < 4; ++k) f(2 + k, m[k]);
+        f(6, c.n);
+        f(7, c.mo);
+        f(8, c.md);
+        f(9, c.oo);
+        f(10, c.dd);
+        f(11, c.od);
     }
 };
 
@@ -124,8 +120,8 @@ __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__
     T m[4] = {-INFINITY, -INFINITY, T(0), T(0)};
     auto take = [&](T o, T d) {
         const T err = abs_err(d, o);
-        f.s[2] += (double)(T)(d * d);
-        f.s[3] += (double)(T)(err * err);
+        f.s[0] += (double)(T)(d * d);
+        f.s[1] += (double)(T)(err * err);
         m[0] = max_of(m[0], o);
         m[1] = max_of(m[1], -o);
         m[2] = max_of(m[2], err);
@@ -148,8 +144,6 @@ __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__
                 so += (double)vo[u][j];
                 sd += (double)vd[u][j];
             }
-        f.s[0] += so;
-        f.s[1] += sd;
         Moments c = {(double)E, so * (1.0 / E), sd * (1.0 / E), 0, 0, 0};
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -165,8 +159,6 @@ __global__ void __launch_bounds__(kThreads) figures_kernel(const T* __restrict__
     if (blockIdx.x == gridDim.x - 1)   // fewer than one step's elements are left
         for (uint64_t i = steps * kThreads * E + threadIdx.x; i < n; i += kThreads) {
             take(ori[i], dec[i]);
-            f.s[0] += (double)ori[i];
-            f.s[1] += (double)dec[i];
             f.c = merge(f.c, Moments{1, (double)ori[i], (double)dec[i], 0, 0, 0});
         }
     for (int k = 0; k < 4; ++k) f.m[k] = (double)m[k];
@@ -638,16 +630,16 @@ int run(const T* ori, const T* dec, size_t n, double* out, hipStream_t st) {
     const double* r = s.g.h_res;
     if (r[cuszp::kGridResults - 1] != 0.0) return CUSZP_ERROR_INTERNAL;
     const double N = (double)n;
-    const double mse = r[3] / N, range = r[4] + r[5];            // r[5]: max of -ori
+    const double mse = r[1] / N, range = r[2] + r[3];            // r[3]: max of -ori
     out[0] = mse;                                                // src/cuSZp_utility.cu:937-946
     out[1] = range;
     out[2] = 20 * log10(range) - 10 * log10(mse);
-    out[3] = sqrt(r[3]);
-    out[4] = sqrt(r[3]) / sqrt(r[2]);
+    out[3] = sqrt(r[1]);
+    out[4] = sqrt(r[1]) / sqrt(r[0]);
     out[5] = sqrt(mse) / range;
-    out[6] = r[6];                                               // max |dec - ori|
-    out[7] = r[7];                                               // max |dec - ori| / |ori| over ori != 0
-    out[8] = (r[13] / N) / sqrt(r[11] / N) / sqrt(r[12] / N);    // correlation (acEff)
+    out[6] = r[4];                                               // max |dec - ori|
+    out[7] = r[5];                                               // max |dec - ori| / |ori| over ori != 0
+    out[8] = (r[11] / N) / sqrt(r[9] / N) / sqrt(r[10] / N);     // correlation (acEff)
     return CUSZP_SUCCESS;
 }
 
