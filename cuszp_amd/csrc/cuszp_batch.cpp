@@ -89,17 +89,23 @@ uint64_t tiles(const cuszp_batch_item_t& s, const Geom& g, int waves, int kc) {
 // with the rule's (4, 2).
 void choose_shape(cuszp_batch_plan_s& p) {
     typedef std::vector<std::pair<int, int>> Ladder;   // (waves, chunks)
-    for (const auto& shape : p.pass ? Ladder{{4, 4}, {8, 4}, {8, 8}} : Ladder{{4, 1}, {4, 2}, {8, 2}, {8, 4}, {8, 8}}) {
+    for (const auto& shape : p.pass ? Ladder{{4, 4}, {8, 4}} : Ladder{{4, 1}, {4, 2}, {8, 2}, {8, 4}}) {
         p.waves = shape.first;
         p.kc = shape.second;
+        // counted up to the limit only: some hundred arrays at most, however many there are (4,000 arrays,
+        // counted in full for each shape, took 40 us of a plan's creation)
+        const uint64_t limit = shape_tiles(p.waves);
         uint64_t n = 0;
-        for (const cuszp_batch_item_t& s : p.src) {
+        for (size_t i = 0; i < p.src.size() && n <= limit; ++i) {
+            const cuszp_batch_item_t& s = p.src[i];
             Geom g;
             make_geom(s.dim, s.nbEle, s.dims, g);
             if (s.nbEle) n += tiles(s, g, p.waves, p.kc);
         }
-        if (n <= shape_tiles(p.waves)) return;
+        if (n <= limit) return;
     }
+    p.waves = 8;
+    p.kc = kChunksOf<float>;
 }
 
 // Lay out the tiles of every non-empty array for the plan's shape and upload the
@@ -254,6 +260,7 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
     if ((direction != CUSZP_BATCH_COMPRESS && direction != CUSZP_BATCH_DECOMPRESS) || (count && !items) ||
         count > 0xffffffffull)
         return CUSZP_ERROR_INVALID_ARGUMENT;
+    bool pass = false;
     for (size_t i = 0; i < count; ++i) {
         Geom g;
         const int rc = check_item(items[i], direction, g);
@@ -261,6 +268,7 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
             if (bad_index) *bad_index = i;
             return rc;
         }
+        pass |= direction == CUSZP_BATCH_DECOMPRESS && g.H > kBatchDirectHeader;
     }
     cuszp_batch_plan_s* p = new cuszp_batch_plan_s();
     p->dir = direction;
@@ -268,11 +276,7 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
     p->src.assign(items, items + count);
     int rc = CUSZP_SUCCESS;
     if (hipGetDevice(&p->dev) != hipSuccess) rc = CUSZP_ERROR_HIP;
-    for (const cuszp_batch_item_t& it : p->src) {
-        Geom g;
-        make_geom(it.dim, it.nbEle, it.dims, g);
-        p->pass |= direction == CUSZP_BATCH_DECOMPRESS && g.H > kBatchDirectHeader;
-    }
+    p->pass = pass;
     choose_shape(*p);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
