@@ -60,6 +60,44 @@ namespace {
         if (e_ != hipSuccess) return CUSZP_ERROR_HIP;  \
     } while (0)
 
+// Pinned words that the kernels write. Allocating and freeing pinned memory takes about 33 us, as
+// much as the rest of a plan's creation and a third of a one-shot call on small arrays, so the
+// words of a destroyed plan wait for the next plan on that GPU: at most kKeptBuffers of kKeptWords
+// per GPU (256 KiB). More of them, and those of plans of more arrays, are freed at once. A
+// buffer comes back only when its GPU is idle, and is cleared for the next plan.
+constexpr size_t kKeptBuffers = 4, kKeptWords = 8192;
+std::mutex g_words_mu;
+auto& g_words = *new std::map<int, std::vector<unsigned long long*>>;   // per GPU, idle; never destroyed, plans may be at exit
+
+unsigned long long* take_words(int dev, size_t n) {
+    unsigned long long* w = nullptr;
+    if (n <= kKeptWords) {
+        std::lock_guard<std::mutex> lk(g_words_mu);
+        auto& kept = g_words[dev];
+        if (!kept.empty()) {
+            w = kept.back();
+            kept.pop_back();
+        }
+    }
+    if (!w && hipHostMalloc((void**)&w, std::max(n, kKeptWords) * sizeof(unsigned long long), hipHostMallocCoherent) != hipSuccess)
+        return nullptr;
+    std::memset(w, 0, n * sizeof(unsigned long long));
+    return w;
+}
+// idle: no kernel writes the words any more
+void return_words(int dev, unsigned long long* w, size_t n, bool idle) {
+    if (!w) return;
+    if (n <= kKeptWords && idle) {
+        std::lock_guard<std::mutex> lk(g_words_mu);
+        auto& kept = g_words[dev];
+        if (kept.size() < kKeptBuffers) {
+            kept.push_back(w);
+            return;
+        }
+    }
+    hipHostFree(w);
+}
+
 int check_item(const cuszp_batch_item_t& it, int dir, Geom& g) {
     const int dim = it.dim, type = it.type, mode = it.mode;
     if (bad_enums(dim, type, mode) || bad_eb(it.errorBound, type)) return CUSZP_ERROR_INVALID_ARGUMENT;
@@ -290,9 +328,7 @@ int cuSZp_batch_plan_create(cuszp_batch_plan_t* out, const cuszp_batch_item_t* i
     const size_t n = count ? count : 1;
     if (!rc && hipMalloc((void**)&p->d_err, n * sizeof(unsigned int)) != hipSuccess) rc = CUSZP_ERROR_HIP;
     if (!rc && hipMalloc((void**)&p->d_sizes, n * sizeof(unsigned long long)) != hipSuccess) rc = CUSZP_ERROR_HIP;
-    if (!rc && hipHostMalloc((void**)&p->h_res, (1 + n) * sizeof(unsigned long long), hipHostMallocCoherent) != hipSuccess)
-        rc = CUSZP_ERROR_HIP;
-    if (!rc) std::memset(p->h_res, 0, (1 + n) * sizeof(unsigned long long));
+    if (!rc && !(p->h_res = take_words(p->dev, 1 + n))) rc = CUSZP_ERROR_HIP;
     if (!rc && hipMemsetAsync(p->d_misc, 0, kMiscWords * sizeof(unsigned long long), stream) != hipSuccess)
         rc = CUSZP_ERROR_HIP;
     if (!rc && hipMemsetAsync(p->d_err, 0, n * sizeof(unsigned int), stream) != hipSuccess) rc = CUSZP_ERROR_HIP;
@@ -475,14 +511,18 @@ void cuSZp_batch_plan_destroy(cuszp_batch_plan_t p) {
         hipStreamSynchronize(p->cap_stream);
         hipStreamDestroy(p->cap_stream);
     }
-    hipDeviceSynchronize();   // no launch of this plan may still use its buffers
+    int dev = p->dev;
+    hipGetDevice(&dev);
+    if (dev != p->dev) hipSetDevice(p->dev);
+    const bool idle = hipDeviceSynchronize() == hipSuccess;   // no launch of this plan may still use its buffers
     if (p->d_items) hipFree(p->d_items);
     if (p->d_status) hipFree(p->d_status);
     if (p->d_offs) hipFree(p->d_offs);
     if (p->d_misc) hipFree(p->d_misc);
     if (p->d_err) hipFree(p->d_err);
     if (p->d_sizes) hipFree(p->d_sizes);
-    if (p->h_res) hipHostFree(p->h_res);
+    return_words(p->dev, p->h_res, 1 + (p->src.empty() ? 1 : p->src.size()), idle);
+    if (dev != p->dev) hipSetDevice(dev);
     delete p;
 }
 

@@ -2,6 +2,7 @@
 // launches that are replaced here by host memory and a log. It shows what the
 // plan launches when a launch or an allocation fails, which needs no GPU.
 //   batch_plan epoch   a decode launch that fails after its offset pass
+//   batch_plan words   pinned result words that outlive their plan
 //   batch_plan tune [graph], tune-lost [graph]
 //                      an allocation that fails while shapes are tried, and again when the former one is restored
 #include "../../cuszp_amd/csrc/cuszp_batch.cpp"
@@ -15,6 +16,9 @@ std::vector<unsigned long long> g_pass_epochs;
 int g_fail_decodes = 0;              // decode launches that fail
 bool g_null = false;                 // a launch was given no buffer
 int g_graphs = 0, g_captured = 0;
+int g_pinned = 0, g_pinned_allocs = 0;   // pinned buffers alive, and ever allocated
+int g_device = 0, g_synced = -1;     // the current device, and the last one that was synchronised
+bool g_idle = true;                  // whether the device can be synchronised
 
 #define CHECK(x)                                                    \
     do {                                                            \
@@ -34,12 +38,13 @@ void seen(const char* what, const void* items, const void* status, const void* o
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) { return *p = std::calloc(n ? n : 1, 1), hipSuccess; }
 hipError_t hipFree(void* p) { return std::free(p), hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return ++g_pinned, ++g_pinned_allocs, hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { return --g_pinned, hipFree(p); }
 hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return std::memset(p, v, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
-hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = g_device, hipSuccess; }
+hipError_t hipSetDevice(int d) { return g_device = d, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return g_synced = g_device, g_idle ? hipSuccess : hipErrorLaunchFailure; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)1, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
@@ -133,6 +138,54 @@ void tune(int flags, unsigned fails) {
     CHECK(!g_null);
     cuSZp_batch_plan_destroy(p);
 }
+
+// n arrays of one value
+cuszp_batch_plan_t plan_of(size_t n) {
+    cuszp_batch_item_t it{};
+    it.d_in = it.d_out = g_buf;
+    it.nbEle = 1;
+    it.capacity = 1 << 20;
+    it.errorBound = 1e-3;
+    it.dim = CUSZP_DIM_1D;
+    it.type = CUSZP_TYPE_FLOAT;
+    it.mode = CUSZP_MODE_PLAIN;
+    std::vector<cuszp_batch_item_t> items(n, it);
+    cuszp_batch_plan_t p = nullptr;
+    CHECK(cuSZp_batch_plan_create(&p, items.data(), n, CUSZP_BATCH_COMPRESS, 0, nullptr, nullptr) == CUSZP_SUCCESS);
+    for (size_t i = 0; i <= n; ++i) CHECK(p->h_res[i] == 0);   // nothing of a plan before
+    std::memset(p->h_res, 0xff, (n + 1) * sizeof(*p->h_res));   // as its kernels would
+    return p;
+}
+
+// Pinned words outlive their plan, a bounded number of them.
+void words() {
+    for (int k = 0; k < 20; ++k) cuSZp_batch_plan_destroy(plan_of(1 + 300 * k));
+    CHECK(g_pinned_allocs == 1);
+    std::vector<cuszp_batch_plan_t> many;
+    for (int k = 0; k < 10; ++k) many.push_back(plan_of(3));
+    for (size_t i = 0; i < many.size(); ++i)
+        for (size_t j = 0; j < i; ++j) CHECK(many[i]->h_res != many[j]->h_res);
+    for (auto p : many) cuSZp_batch_plan_destroy(p);
+    CHECK(g_pinned == (int)kKeptBuffers);
+    cuSZp_batch_plan_destroy(plan_of(kKeptWords - 1));   // the most that fits
+    CHECK(g_pinned == (int)kKeptBuffers && g_pinned_allocs == 10);
+    cuSZp_batch_plan_destroy(plan_of(kKeptWords));       // one more: its own buffer, freed with it
+    CHECK(g_pinned == (int)kKeptBuffers && g_pinned_allocs == 11);
+    cuSZp_batch_plan_destroy(plan_of(0));
+    // a plan is finished on its own device, and its words stay there
+    cuszp_batch_plan_t p = plan_of(3);
+    unsigned long long* const w = p->h_res;
+    g_device = 1;
+    cuSZp_batch_plan_destroy(p);
+    CHECK(g_synced == 0 && g_device == 1);
+    p = plan_of(3);
+    CHECK(p->h_res != w);
+    // kernels may still write: not kept
+    g_idle = false;
+    const int alive = g_pinned;
+    cuSZp_batch_plan_destroy(p);
+    CHECK(g_pinned == alive - 1);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -140,6 +193,7 @@ int main(int argc, char** argv) {
     if (what == "epoch") epoch();
     else if (what == "tune") tune(argc > 2 ? CUSZP_BATCH_GRAPH : 0, 1);
     else if (what == "tune-lost") tune(argc > 2 ? CUSZP_BATCH_GRAPH : 0, 2);
+    else if (what == "words") words();
     else return 2;
     std::puts("ok");
     return 0;

@@ -1,4 +1,4 @@
-"""Batched plans when a launch or an allocation fails, on the CPU: cuszp_batch.cpp
+"""Batched plans when a launch or an allocation fails, and what outlives them, on the CPU: cuszp_batch.cpp
 built with a HIP runtime and launches of host memory (tests/host/batch_plan.cpp)."""
 import os
 import shutil
@@ -26,7 +26,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["epoch", "tune", "tune graph", "tune-lost", "tune-lost graph"])
+@pytest.mark.parametrize("case", ["epoch", "words", "tune", "tune graph", "tune-lost", "tune-lost graph"])
 def test_plan(program, case):
     r = subprocess.run([program, *case.split()], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
