@@ -6,7 +6,8 @@
 namespace cuszp {
 
 // Advances the scan epoch of a batched plan; runs (one thread) before every
-// batched launch, also inside captured graphs.
+// compress launch, also inside captured graphs. (A decode kernel advances the
+// epoch of its offset pass itself; the server's epochs come with its items.)
 __global__ void bump_epoch_kernel(unsigned long long* epoch) {
     if (threadIdx.x == 0) epoch[0] = epoch[0] + 1;
 }

@@ -78,7 +78,7 @@ static_assert(unit_blocks(2, false, 4) % kPrefixBytes == 0 && unit_blocks(2, tru
 inline uint64_t batch_segments(int dim, bool f64, int kc, uint64_t nunits) {
     return (nunits * unit_blocks(dim, f64, kc) + kBatchSegBytes - 1) / kBatchSegBytes;
 }
-// Increments *epoch (one thread); runs before each batched launch.
+// Increments *epoch (one thread); runs before each compress launch of a plan.
 hipError_t launch_bump_epoch(unsigned long long* epoch, hipStream_t st);
 // Largest grid of a tile launch; arrays with more tiles take several launches.
 constexpr uint64_t kMaxGrid = 1ull << 22;

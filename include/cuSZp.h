@@ -245,7 +245,9 @@ const unsigned long long* cuSZp_batch_plan_device_sizes(cuszp_batch_plan_t plan)
  * workgroups of 4 or 8 waves of 64 lanes, and lookback windows of 128 or 256
  * predecessor tiles per round trip; keeps the fastest for this plan and for
  * later plans of the same size class. Returns its workgroup size (waves) in
- * *waves and the workgroups of its (first) launch, one per tile, in *grid. */
+ * *waves and the workgroups of its (first) launch, one per tile, in *grid. After
+ * an error the plan has the shape it had before; if even that could not be
+ * allocated again, executes return CUSZP_ERROR_HIP until a tuning run succeeds. */
 int cuSZp_batch_plan_tune(cuszp_batch_plan_t plan, hipStream_t stream, int* waves, unsigned* grid);
 void cuSZp_batch_plan_destroy(cuszp_batch_plan_t plan);
 /* cuSZp_scan_report for the plan's launches (synchronises `stream`). */
